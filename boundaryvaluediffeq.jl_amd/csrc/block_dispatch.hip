@@ -59,11 +59,18 @@ int block_blocks_per_cu(int M, int method, int precision) {
     return 1;
 }
 
-size_t block_record_values(int M) {
-    switch (M) {
-    case 8: return BRec<8>::SIZE;
-    case 16: return BRec<16>::SIZE;
-    case 32: return BRec<32>::SIZE;
-    }
-    return 0;
+template <int M> static size_t slot_bytes(int precision, int rec_cap) {
+    const size_t rec = precision == BVP_PREC_FP32_REFINE64 ? BRec<M, float>::SIZE * sizeof(float)
+                                                           : BRec<M, double>::SIZE * sizeof(double);
+    return ((BRoot<M>::BYTES + 255) & ~(size_t)255) + ((rec * (size_t)rec_cap + 255) & ~(size_t)255);
+}
+
+size_t block_slot_bytes(int M, int precision, int rec_cap) {
+    return M == 8 ? slot_bytes<8>(precision, rec_cap)
+         : M == 16 ? slot_bytes<16>(precision, rec_cap) : slot_bytes<32>(precision, rec_cap);
+}
+
+size_t block_aux_doubles(int M, int method, int cap) {
+    const size_t stage = (size_t)((method == 6 ? Tab<6>::s : Tab<4>::s) + 1) * M;
+    return (size_t)cap * (2 * M + stage + 1);
 }

@@ -253,26 +253,26 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
         scratch_doubles = D.scratch_per_slot * slots;
         D.rec_cap = cap;
     } else {
-        // factor records of one instance live in its wave's slot: rec_cap intervals.
-        const size_t esz = (o->precision == BVP_PREC_FP32_REFINE64) ? 4 : 8;
-        const size_t rv = block_record_values(M);
+        // factor records of one instance live in its workgroup's slot: rec_cap intervals.
         // budget: 80% of the device memory free at this point (the problem data is
         // already allocated)
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b == 0) free_b = (size_t)120 << 30;
         const size_t budget = free_b / 10 * 8;
+        D.aux_per_slot = block_aux_doubles(M, o->method, cap);
+        auto per_slot = [&](int rc) {
+            return block_slot_bytes(M, o->precision, rc) + D.aux_per_slot * sizeof(double);
+        };
         // room for every mesh the solve may reach (max_num_subintervals) when it fits,
         // else for meshes up to twice the largest initial one, else for that one
         int rec_cap = std::max(o->max_num_subintervals, maxN0);
-        if ((size_t)rec_cap * rv * esz * slots > budget) rec_cap = std::min(rec_cap, 2 * maxN0);
-        if ((size_t)rec_cap * rv * esz * slots > budget) rec_cap = maxN0;
-        const size_t per_slot = (size_t)rec_cap * rv;  // in factor-type elements
-        if (per_slot * esz * slots > budget) slots = std::max(1, (int)(budget / (per_slot * esz)));
+        if (per_slot(rec_cap) * slots > budget) rec_cap = std::min(rec_cap, 2 * maxN0);
+        if (per_slot(rec_cap) * slots > budget) rec_cap = maxN0;
+        if (per_slot(rec_cap) * slots > budget) slots = std::max(1, (int)(budget / per_slot(rec_cap)));
         D.rec_cap = rec_cap;
         D.tree_base = 0;
-        D.scratch_per_slot = per_slot;
-        D.aux_per_slot = (size_t)cap * (3 * M + 1);
-        scratch_doubles = (per_slot * esz * slots + 7) / 8;
+        D.scratch_per_slot = block_slot_bytes(M, o->precision, rec_cap);
+        scratch_doubles = D.scratch_per_slot / 8 * slots;
     }
     B->max_slots = slots;
     B->blocks = std::min(slots, std::max(1, std::min(n, ctx->num_cus * per_cu)));

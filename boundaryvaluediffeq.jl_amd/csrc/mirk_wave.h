@@ -54,7 +54,7 @@ struct BatchDev {
 
     // per-slot (persistent wave) scratch
     double *scratch;
-    size_t scratch_per_slot;  // doubles
+    size_t scratch_per_slot;  // doubles (block kernels: bytes)
     size_t tree_base;         // offset of the tree records inside a slot
     double *aux;              // [slot][cap*(3M+1)]: delta, trial state, transfer indices, J'F
                               //   (block kernels: their own layout)
@@ -154,4 +154,7 @@ bool block_supports(int M, int family);
 hipError_t block_launch_solve(const BatchDev &B, int method, int precision, int blocks, hipStream_t s);
 hipError_t block_launch_component(const BatchDev &B, int method, int precision, int op, int blocks, hipStream_t s);
 int block_blocks_per_cu(int M, int method, int precision);
-size_t block_record_values(int M);  // values (of the factor type) per interval record
+// bytes of a workgroup's slot: the end-node system and the records of rec_cap nodes
+size_t block_slot_bytes(int M, int precision, int rec_cap);
+// doubles of its work area: correction, refinement residual, stage records, transfer indices
+size_t block_aux_doubles(int M, int method, int cap);

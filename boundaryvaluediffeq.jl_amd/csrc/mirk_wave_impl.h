@@ -1773,7 +1773,10 @@ __device__ inline void half_mesh_into(const double *mesh, int N, double *out, in
 // the halving threshold (1 for DefectControl, 2 for the global-error controllers).
 // Writes the new mesh into new_mesh and returns the new N, or -1 on failure (cap
 // exceeded).
-template <typename SH>
+struct BlockSync {
+    __device__ void operator()() const { __syncthreads(); }
+};
+template <typename SH, class Sync = BlockSync>
 __device__ inline int mesh_select(const double *mesh, int N, double *shat, double r1, double r2, int max_sub,
                                   double *new_mesh, int lane, SH &sh, double rho = 1.0) {
     const int n = N;
@@ -1785,7 +1788,7 @@ __device__ inline int mesh_select(const double *mesh, int N, double *shat, doubl
         const long long Ns = 2LL * n;
         if (Ns > max_sub) return -1;
         half_mesh_into(mesh, N, new_mesh, lane);
-        __syncthreads();
+        Sync()();
         return (int)Ns;
     }
     const long long lb = (n + 1) / 2, ub = 4LL * n;
@@ -1802,7 +1805,7 @@ __device__ inline int mesh_select(const double *mesh, int N, double *shat, doubl
         acc += s * h;
     }
     const double zeta = wave_sum(acc) / (double)Ns;
-    __syncthreads();
+    Sync()();
     if (lane == 0) {
         // sequential equidistribution walk (MIRK/adaptivity.jl:254-273)
         new_mesh[0] = mesh[0];
@@ -1829,7 +1832,7 @@ __device__ inline int mesh_select(const double *mesh, int N, double *shat, doubl
         new_mesh[Ns] = mesh[n];
         sh.flag = ok;
     }
-    __syncthreads();
+    Sync()();
     return sh.flag ? (int)Ns : -1;
 }
 
