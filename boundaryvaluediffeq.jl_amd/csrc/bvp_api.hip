@@ -302,7 +302,7 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
         tab.order = ftab.order;
         FirkTab *dtab = nullptr;
         if ((rc = upload(ctx, A, dtab, std::vector<FirkTab>(1, tab))) ||
-            (rc = dalloc(ctx, A, D.stK, (size_t)n * cap * ftab.s * M))) {
+            (rc = dalloc(ctx, A, D.stK, (size_t)n * ((size_t)cap + 64) * ftab.s * M))) {
             delete B;
             return rc;
         }

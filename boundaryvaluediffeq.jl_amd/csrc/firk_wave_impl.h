@@ -24,16 +24,55 @@
 
 namespace bvpdev {
 
-// stage values of instance b: [cap][S][M] (interval, stage, component)
+// Per-interval data of a wave (stage values, their corrections, the condensation records)
+// is interleaved over the lanes that own the intervals: field q of interval k lies at
+// [step i][q][64 lanes] with k the i-th interval of its lane's chunk, so that the 64 lanes
+// walking their chunks read and write whole 512-byte lines.  (In [interval][field] order
+// every access of the wave touched 64 lines.)  An area holds kFirkPad<cap> intervals.
+__host__ __device__ inline size_t firk_pad(int cap) { return (size_t)cap + WAVE; }
+
+struct FirkAt {
+    int lane, i;
+};
+__device__ inline FirkAt firk_at(int N, int k) {
+    const int P = N < WAVE ? N : WAVE, q = N / P, r = N % P;
+    FirkAt a;
+    if (k < r * (q + 1)) { a.lane = k / (q + 1); a.i = k % (q + 1); }
+    else { a.lane = r + (k - r * (q + 1)) / q; a.i = (k - r * (q + 1)) % q; }
+    return a;
+}
+// offset of field 0 of step i in an area of NF fields (field q: + q * WAVE)
+template <int NF> __device__ __forceinline__ size_t firk_off(int lane, int i) { return (size_t)i * (NF * WAVE) + lane; }
+template <int NF> __device__ __forceinline__ size_t firk_off(int N, int k, bool) {
+    const FirkAt a = firk_at(N, k);
+    return firk_off<NF>(a.lane, a.i);
+}
+// calls fn(offset of the interval's stage values in lane-interleaved areas of NF fields)
+// for the intervals of this lane's chunk
+template <int NF, typename Fn> __device__ __forceinline__ void firk_each(int N, int lane, Fn &&fn) {
+    int P, start, len;
+    chunk_of(N, lane, P, start, len);
+    for (int i = 0; i < len; ++i) fn(firk_off<NF>(lane, i));
+}
+
+// stage values of instance b (lane-interleaved, S M fields per interval)
 template <int M, int S>
 __device__ inline double *firk_stages_of(const BatchDev &B, int b) {
-    return as_global(B.stK + (size_t)b * B.cap * S * M);
+    return as_global(B.stK + (size_t)b * firk_pad(B.cap) * S * M);
+}
+
+// the batch's tableau, in constant memory for the compiler (no kernel writes it): uniform
+// entries come by scalar loads
+__device__ inline const FirkTab &firk_tab_of(const BatchDev &B) {
+    return *(const FirkTab *)(const __attribute__((address_space(4))) FirkTab *)B.firk_tab;
 }
 
 // ------------------------------------------------------------------ dense solve
 // W X = R in place (R becomes X), Gaussian elimination with partial pivoting (first
 // maximum).  Small systems stay in registers (unrolled, row swaps by selects); larger
 // ones (S M > 8) run as loops over private arrays.  Returns false on a zero pivot.
+// (All unrolled loops have constant trip counts with a condition inside: triangular bounds
+// leave the arrays in private memory, with a store for every update.)
 template <int NN, int NR>
 __device__ inline bool lu_solve_small(double (&W)[NN][NN], double (&R)[NN][NR]) {
 #pragma unroll
@@ -41,16 +80,19 @@ __device__ inline bool lu_solve_small(double (&W)[NN][NN], double (&R)[NN][NR]) 
         int p = j;
         double best = fabs(W[j][j]);
 #pragma unroll
-        for (int i = j + 1; i < NN; ++i) {
+        for (int i = 0; i < NN; ++i) {
+            if (i <= j) continue;
             const double v = fabs(W[i][j]);
             if (v > best) { best = v; p = i; }
         }
         if (!(best > 0.0)) return false;
 #pragma unroll
-        for (int i = j + 1; i < NN; ++i) {
+        for (int i = 0; i < NN; ++i) {
+            if (i <= j) continue;
             const bool sw = (i == p);
 #pragma unroll
-            for (int c = j; c < NN; ++c) {
+            for (int c = 0; c < NN; ++c) {
+                if (c < j) continue;
                 const double t = W[j][c];
                 W[j][c] = sw ? W[i][c] : W[j][c];
                 W[i][c] = sw ? t : W[i][c];
@@ -64,22 +106,26 @@ __device__ inline bool lu_solve_small(double (&W)[NN][NN], double (&R)[NN][NR]) 
         }
         const double inv = 1.0 / W[j][j];
 #pragma unroll
-        for (int i = j + 1; i < NN; ++i) {
+        for (int i = 0; i < NN; ++i) {
+            if (i <= j) continue;
             const double m = W[i][j] * inv;
 #pragma unroll
-            for (int c = j + 1; c < NN; ++c) W[i][c] -= m * W[j][c];
+            for (int c = 0; c < NN; ++c)
+                if (c > j) W[i][c] -= m * W[j][c];
 #pragma unroll
             for (int c = 0; c < NR; ++c) R[i][c] -= m * R[j][c];
         }
     }
 #pragma unroll
-    for (int i = NN - 1; i >= 0; --i) {
+    for (int q = 0; q < NN; ++q) {
+        const int i = NN - 1 - q;
         const double inv = 1.0 / W[i][i];
 #pragma unroll
         for (int c = 0; c < NR; ++c) {
             double v = R[i][c];
 #pragma unroll
-            for (int k = i + 1; k < NN; ++k) v -= W[i][k] * R[k][c];
+            for (int k = 0; k < NN; ++k)
+                if (k > i) v -= W[i][k] * R[k][c];
             R[i][c] = v * inv;
         }
     }
@@ -146,47 +192,76 @@ __device__ inline bool lu_solve(double (&W)[NN][NN], double (&R)[NN][NR]) {
     else return lu_solve_loop<NN, NR>(W, R);
 }
 
+// The same solve where no step needs a row exchange: false when some pivot is not the first
+// maximum of its column (or is zero or NaN) in this lane, with W and R then undefined.
+template <int NN, int NR>
+__device__ __forceinline__ bool lu_solve_diag(double (&W)[NN][NN], double (&R)[NN][NR]) {
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < NN; ++j) {
+        const double best = fabs(W[j][j]);
+        ok &= best > 0.0;
+        const double inv = 1.0 / W[j][j];
+#pragma unroll
+        for (int i = 0; i < NN; ++i) {
+            if (i <= j) continue;
+            ok &= !(fabs(W[i][j]) > best);
+            const double m = W[i][j] * inv;
+#pragma unroll
+            for (int c = 0; c < NN; ++c)
+                if (c > j) W[i][c] -= m * W[j][c];
+#pragma unroll
+            for (int c = 0; c < NR; ++c) R[i][c] -= m * R[j][c];
+        }
+        W[j][j] = inv;
+    }
+#pragma unroll
+    for (int q = 0; q < NN; ++q) {
+        const int i = NN - 1 - q;
+#pragma unroll
+        for (int c = 0; c < NR; ++c) {
+            double v = R[i][c];
+#pragma unroll
+            for (int k = 0; k < NN; ++k)
+                if (k > i) v -= W[i][k] * R[k][c];
+            R[i][c] = v * W[i][i];
+        }
+    }
+    return ok;
+}
+
 // ------------------------------------------------------------------ one interval
 // Stage points Y_r = h (sum_j a_rj K_j) + y_i, stage residuals G_r = f(t_i + c_r h, Y_r)
 // - K_r and the continuity residual Phi = (y_{i+1} - y_i) - h (sum_j b_j K_j), in the
-// order of operations of Phi! (FIRK/collocation.jl:59-93); with JAC the stage
-// Jacobians J_r by forward-mode dual numbers.
+// order of operations of Phi! (FIRK/collocation.jl:59-93); with JAC the stage Jacobians
+// J_r.  Where the exchange area ([field][64 lanes], in the LDS that the tree uses between
+// the interval passes) holds f and J of all stages, the stages run as a loop (the families'
+// code once instead of S times) and pass them through the lane's column sl of it.  Without
+// it (LD false), and for systems of more than 12 unknowns, whose arrays lie in private
+// memory in any case, the pieces run out of line, so that a kernel holds their frames once.
+template <int M, int S> constexpr int kFirkSlot = S * (M + M * M);  // fields of the exchange area
+template <int M, int S> constexpr bool kFirkBig = S * M > 12;
+template <int M, int S> constexpr bool kFirkSlotLds = !kFirkBig<M, S> && kFirkSlot<M, S> * WAVE <= kStageNodes<M> * M;
+
 template <int M, int S, bool JAC>
-__device__ inline void firk_interval(const Inst<M> &I, const FirkTab &T, double ti, double h, const double *yi,
-                                     const double *yj, const double (&K)[S][M], double (&G)[S][M], double (&Phi)[M],
-                                     double (&J)[S][M][M]) {
+__device__ __forceinline__ void firk_stage(const Inst<M> &I, const FirkTab &T, int r, double ti, double h,
+                                           const double *yi, const double (&K)[S][M], double (&F)[M],
+                                           double (&Jr)[M][M]) {
+    double Y[M];
 #pragma unroll
-    for (int r = 0; r < S; ++r) {
-        double Y[M];
+    for (int c = 0; c < M; ++c) {
+        double a = 0.0;
 #pragma unroll
-        for (int c = 0; c < M; ++c) {
-            double a = 0.0;
-#pragma unroll
-            for (int j = 0; j < S; ++j) a += K[j][c] * T.A[r][j];
-            Y[c] = h * a + yi[c];
-        }
-        const double t = ti + T.c[r] * h;
-        if constexpr (JAC) {
-            Dual<M> Yd[M], Fd[M];
-#pragma unroll
-            for (int c = 0; c < M; ++c) {
-                Yd[c] = dconst<M>(Y[c]);
-                Yd[c].d[c] = 1.0;
-            }
-            f_eval<M, Dual<M>>(I.fam, I.P, t, Yd, Fd);
-#pragma unroll
-            for (int a = 0; a < M; ++a) {
-                G[r][a] = Fd[a].v - K[r][a];
-#pragma unroll
-                for (int c = 0; c < M; ++c) J[r][a][c] = Fd[a].d[c];
-            }
-        } else {
-            double F[M];
-            f_eval<M, double>(I.fam, I.P, t, Y, F);
-#pragma unroll
-            for (int a = 0; a < M; ++a) G[r][a] = F[a] - K[r][a];
-        }
+        for (int j = 0; j < S; ++j) a += K[j][c] * T.A[r][j];
+        Y[c] = h * a + yi[c];
     }
+    const double t = ti + T.c[r] * h;
+    if constexpr (JAC) f_jac<M>(I.fam, I.P, t, Y, F, Jr);
+    else f_eval<M, double>(I.fam, I.P, t, Y, F);
+}
+template <int M, int S>
+__device__ __forceinline__ void firk_phi(const FirkTab &T, double h, const double *yi, const double *yj,
+                                         const double (&K)[S][M], double (&Phi)[M]) {
 #pragma unroll
     for (int c = 0; c < M; ++c) {
         double a = 0.0;
@@ -195,39 +270,136 @@ __device__ inline void firk_interval(const Inst<M> &I, const FirkTab &T, double 
         Phi[c] = -h * a + (yj[c] - yi[c]);
     }
 }
+template <int M, int S, bool JAC>
+__device__ __noinline__ void firk_interval_big(const Inst<M> &I, const FirkTab &T, double ti, double h,
+                                               const double *yi, const double *yj, const double (&K)[S][M],
+                                               double (&G)[S][M], double (&Phi)[M], double (&J)[S][M][M]) {
+#pragma unroll 1
+    for (int r = 0; r < S; ++r) {
+        double F[M], Jr[M][M];
+        firk_stage<M, S, JAC>(I, T, r, ti, h, yi, K, F, Jr);
+#pragma unroll
+        for (int a = 0; a < M; ++a) {
+            G[r][a] = F[a] - K[r][a];
+            if constexpr (JAC)
+#pragma unroll
+                for (int c = 0; c < M; ++c) J[r][a][c] = Jr[a][c];
+        }
+    }
+    firk_phi<M, S>(T, h, yi, yj, K, Phi);
+}
+template <int M, int S, bool JAC, bool LD = kFirkSlotLds<M, S>>
+__device__ __forceinline__ void firk_interval(const Inst<M> &I, const FirkTab &T, double *sl, double ti, double h,
+                                              const double *yi, const double *yj, const double (&K)[S][M],
+                                              double (&G)[S][M], double (&Phi)[M], double (&J)[S][M][M]) {
+    if constexpr (!LD) {
+        firk_interval_big<M, S, JAC>(I, T, ti, h, yi, yj, K, G, Phi, J);
+    } else {
+        constexpr int NS = M + M * M;
+#pragma unroll 1
+        for (int r = 0; r < S; ++r) {
+            double F[M], Jr[M][M];
+            firk_stage<M, S, JAC>(I, T, r, ti, h, yi, K, F, Jr);
+            double *o = sl + r * (NS * WAVE);
+#pragma unroll
+            for (int a = 0; a < M; ++a) {
+                o[a * WAVE] = F[a];
+                if constexpr (JAC)
+#pragma unroll
+                    for (int c = 0; c < M; ++c) o[(M + a * M + c) * WAVE] = Jr[a][c];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            const double *o = sl + r * (NS * WAVE);
+#pragma unroll
+            for (int a = 0; a < M; ++a) {
+                G[r][a] = o[a * WAVE] - K[r][a];
+                if constexpr (JAC)
+#pragma unroll
+                    for (int c = 0; c < M; ++c) J[r][a][c] = o[(M + a * M + c) * WAVE];
+            }
+        }
+        firk_phi<M, S>(T, h, yi, yj, K, Phi);
+    }
+}
 
-// local record of an interval: kg [S M] then KJ [S M][M] (row (r, a), column c)
+// X = the solution of the local system W [kg | KJ] = [G | J] (NR = M + 1) or W x = G (NR = 1).
+// PIV false: without row exchanges; piv is set when a lane needs one (X is then undefined),
+// and the caller repeats its pass with PIV true.
+template <int M, int S, int NR>
+__device__ __noinline__ bool firk_local_big(const FirkTab &T, double h, const double (&G)[S][M],
+                                            const double (&J)[S][M][M], double (&X)[S * M][NR]) {
+    constexpr int NN = S * M;
+    double W[NN][NN];
+#pragma unroll 1
+    for (int r = 0; r < S; ++r)
+#pragma unroll 1
+        for (int a = 0; a < M; ++a) {
+#pragma unroll 1
+            for (int j = 0; j < S; ++j)
+#pragma unroll
+                for (int c = 0; c < M; ++c)
+                    W[r * M + a][j * M + c] = ((r == j && a == c) ? 1.0 : 0.0) - h * T.A[r][j] * J[r][a][c];
+            X[r * M + a][0] = G[r][a];
+            if constexpr (NR > 1)
+#pragma unroll
+                for (int c = 0; c < M; ++c) X[r * M + a][1 + c] = J[r][a][c];
+        }
+    return lu_solve<NN, NR>(W, X);
+}
+template <int M, int S, int NR, bool PIV>
+__device__ __forceinline__ bool firk_local(const FirkTab &T, double h, const double (&G)[S][M],
+                                           const double (&J)[S][M][M], double (&X)[S * M][NR], bool &piv) {
+    if constexpr (kFirkBig<M, S>) {
+        static_assert(PIV, "systems above 12 unknowns are solved with row exchanges");
+        return firk_local_big<M, S, NR>(T, h, G, J, X);
+    } else {
+        constexpr int NN = S * M;
+        double W[NN][NN];
+#pragma unroll
+        for (int r = 0; r < S; ++r)
+#pragma unroll
+            for (int a = 0; a < M; ++a) {
+#pragma unroll
+                for (int j = 0; j < S; ++j)
+#pragma unroll
+                    for (int c = 0; c < M; ++c)
+                        W[r * M + a][j * M + c] = ((r == j && a == c) ? 1.0 : 0.0) - h * T.A[r][j] * J[r][a][c];
+                X[r * M + a][0] = G[r][a];
+                if constexpr (NR > 1)
+#pragma unroll
+                    for (int c = 0; c < M; ++c) X[r * M + a][1 + c] = J[r][a][c];
+            }
+        if constexpr (PIV) {
+            return lu_solve<NN, NR>(W, X);
+        } else {
+            piv |= !lu_solve_diag<NN, NR>(W, X);
+            return true;
+        }
+    }
+}
+
+// local record of an interval: kg [S M] then KJ [S M][M] (row (r, a), column c), fields of
+// a lane-interleaved area
 template <int M, int S> constexpr int kFirkLoc = S * M * (M + 1);
 
 // Static condensation of interval k: solves W [kg | KJ] = [G | J], stores the record
 // at loc, and forms the two-node relation S_blk dy_i + dy_{i+1} = rhs.
 // nested: the stages are solved (G ~ 0 to the inner tolerance) and the relation is
 // the Newton step of the nested residual, rhs = -Phi.
-template <int M, int S>
-__device__ inline bool firk_condense(const FirkTab &T, double h, const double (&G)[S][M], const double (&Phi)[M],
-                                     const double (&J)[S][M][M], double *loc, double (&Sb)[M][M], double (&rhs)[M],
-                                     bool nested = false) {
+template <int M, int S, bool PIV>
+__device__ __forceinline__ bool firk_condense(const FirkTab &T, double h, const double (&G)[S][M],
+                                              const double (&Phi)[M], const double (&J)[S][M][M], double *loc,
+                                              double (&Sb)[M][M], double (&rhs)[M], bool nested, bool &piv) {
     constexpr int NN = S * M;
-    double W[NN][NN], X[NN][M + 1];
-#pragma unroll
-    for (int r = 0; r < S; ++r)
-#pragma unroll
-        for (int a = 0; a < M; ++a) {
-#pragma unroll
-            for (int j = 0; j < S; ++j)
-#pragma unroll
-                for (int c = 0; c < M; ++c)
-                    W[r * M + a][j * M + c] = ((r == j && a == c) ? 1.0 : 0.0) - h * T.A[r][j] * J[r][a][c];
-            X[r * M + a][0] = G[r][a];
-#pragma unroll
-            for (int c = 0; c < M; ++c) X[r * M + a][1 + c] = J[r][a][c];
-        }
-    const bool ok = lu_solve<NN, M + 1>(W, X);
+    double X[NN][M + 1];
+    const bool ok = firk_local<M, S, M + 1, PIV>(T, h, G, J, X, piv);
 #pragma unroll
     for (int q = 0; q < NN; ++q) {
-        loc[q] = X[q][0];
+        loc[q * WAVE] = X[q][0];
 #pragma unroll
-        for (int c = 0; c < M; ++c) loc[NN + q * M + c] = X[q][1 + c];
+        for (int c = 0; c < M; ++c) loc[(NN + q * M + c) * WAVE] = X[q][1 + c];
     }
 #pragma unroll
     for (int a = 0; a < M; ++a) {
@@ -246,12 +418,13 @@ __device__ inline bool firk_condense(const FirkTab &T, double h, const double (&
     return ok;
 }
 
+// the stage values at offset `off` of a lane-interleaved area
 template <int M, int S>
-__device__ inline void load_stages(const double *K, int k, double (&Kk)[S][M]) {
+__device__ __forceinline__ void load_stages(const double *K, size_t off, double (&Kk)[S][M]) {
 #pragma unroll
     for (int r = 0; r < S; ++r)
 #pragma unroll
-        for (int c = 0; c < M; ++c) Kk[r][c] = K[((size_t)k * S + r) * M + c];
+        for (int c = 0; c < M; ++c) Kk[r][c] = K[off + (size_t)(r * M + c) * WAVE];
 }
 
 // The nested form (nested_nlsolve = true, FIRK/firk.jl:114-288): the unknowns are the
@@ -278,17 +451,17 @@ __device__ inline FirkNest<M> firk_nest_of(const BatchDev &B, int b) {
     return n;
 }
 
-template <int M, int S>
-__device__ inline void firk_inner(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double ti, double h,
-                                  const double *yi, double (&K)[S][M]) {
-    constexpr int NN = S * M;
+// PIV false: stops with piv set where a lane's system needs row exchanges (K undefined).
+template <int M, int S, bool LD, bool PIV>
+__device__ __forceinline__ void firk_inner_body(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double *sl,
+                                           double ti, double h, const double *yi, double (&K)[S][M], bool &piv) {
 #pragma unroll
     for (int r = 0; r < S; ++r)
 #pragma unroll
         for (int c = 0; c < M; ++c) K[r][c] = nest.k0[c];
     for (int it = 0; it < 1000; ++it) {
         double G[S][M], Phi[M], J[S][M][M];
-        firk_interval<M, S, true>(I, T, ti, h, yi, yi, K, G, Phi, J);
+        firk_interval<M, S, true, LD>(I, T, sl, ti, h, yi, yi, K, G, Phi, J);
         double mx = 0.0;
         bool bad = false;
 #pragma unroll
@@ -299,19 +472,9 @@ __device__ inline void firk_inner(const Inst<M> &I, const FirkTab &T, const Firk
                 mx = fmax(mx, fabs(G[r][c]));
             }
         if (bad || !(mx > nest.tol)) break;
-        double W[NN][NN], X[NN][1];
-#pragma unroll
-        for (int r = 0; r < S; ++r)
-#pragma unroll
-            for (int a = 0; a < M; ++a) {
-#pragma unroll
-                for (int j = 0; j < S; ++j)
-#pragma unroll
-                    for (int c = 0; c < M; ++c)
-                        W[r * M + a][j * M + c] = ((r == j && a == c) ? 1.0 : 0.0) - h * T.A[r][j] * J[r][a][c];
-                X[r * M + a][0] = G[r][a];
-            }
-        if (!lu_solve<NN, 1>(W, X)) break;
+        double X[S * M][1];
+        if (!firk_local<M, S, 1, PIV>(T, h, G, J, X, piv)) break;
+        if (!PIV && piv) break;
 #pragma unroll
         for (int r = 0; r < S; ++r)
 #pragma unroll
@@ -320,11 +483,24 @@ __device__ inline void firk_inner(const Inst<M> &I, const FirkTab &T, const Firk
 }
 
 template <int M, int S>
-__device__ inline void store_stages(double *K, int k, const double (&Kk)[S][M]) {
+__device__ __noinline__ void firk_inner_big(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double ti,
+                                            double h, const double *yi, double (&K)[S][M]) {
+    bool piv = false;
+    firk_inner_body<M, S, false, true>(I, T, nest, nullptr, ti, h, yi, K, piv);
+}
+template <int M, int S, bool LD, bool PIV>
+__device__ __forceinline__ void firk_inner(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double *sl,
+                                           double ti, double h, const double *yi, double (&K)[S][M], bool &piv) {
+    if constexpr (kFirkBig<M, S>) firk_inner_big<M, S>(I, T, nest, ti, h, yi, K);
+    else firk_inner_body<M, S, LD, PIV>(I, T, nest, sl, ti, h, yi, K, piv);
+}
+
+template <int M, int S>
+__device__ __forceinline__ void store_stages(double *K, size_t off, const double (&Kk)[S][M]) {
 #pragma unroll
     for (int r = 0; r < S; ++r)
 #pragma unroll
-        for (int c = 0; c < M; ++c) K[((size_t)k * S + r) * M + c] = Kk[r][c];
+        for (int c = 0; c < M; ++c) K[off + (size_t)(r * M + c) * WAVE] = Kk[r][c];
 }
 
 // The quintic through value and slope at 0, h, h/2 (get_S_coeffs / s_constraints_block,
@@ -360,6 +536,10 @@ __device__ inline void firk_quintic(double h, const double (&bk)[6], double (&co
 template <int M> struct FirkShared : Shared<M> {
     double irow[M * (2 * M + 2)];
 };
+// this lane's column of the exchange area
+template <int M, int S> __device__ __forceinline__ double *firk_slot(Shared<M> &sh, int lane) {
+    return kFirkSlotLds<M, S> ? sh.stage + lane : nullptr;
+}
 
 // ------------------------------------------------------------------ interior boundary rows
 // A STANDARD row inside the span reads EvalSol of the FIRK cache (FIRK/interpolation.jl:
@@ -478,14 +658,14 @@ __device__ inline double firk_evalsol(const Inst<M> &I, const FirkTab &T, bool e
 // Residual of the boundary row k inside the span (interval j) at (y + alpha dy,
 // K + alpha dK) (dy, dK may be null: alpha 0; K unused by the nested form).  WANTG: also
 // its linearisation for the root solve into ir: [M] coefficients of dy_j, [M] of dy_{j+1},
-// the constant, with the stage corrections eliminated through the interval's record lk
-// (dK = kg + KJ dy_j).
+// the constant, with the stage corrections eliminated through the interval's record in loc
+// (dK = kg + KJ dy_j).  N: the mesh the lane-interleaved areas belong to.
 template <int M, int S, bool WANTG>
 __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest,
                                           const double *mesh, const double *y, const double *K, const double *dy,
-                                          const double *dK, double alpha, int k, int j, const double *lk,
-                                          double *ir, const double *dy2 = nullptr, const double *dK2 = nullptr,
-                                          double beta = 0.0, double *graw = nullptr) {
+                                          const double *dK, double alpha, int k, int j, const double *loc,
+                                          double *ir, int N, const double *dy2 = nullptr,
+                                          const double *dK2 = nullptr, double beta = 0.0, double *graw = nullptr) {
     const int comp = sel<M>(I.bcc, k);
     double yi[M], yj[M], Kk[S][M];
 #pragma unroll
@@ -505,13 +685,15 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
         FirkNest<M> z = nest;
 #pragma unroll
         for (int c = 0; c < M; ++c) z.k0[c] = 0.0;
-        firk_inner<M, S>(I, T, z, mesh[j], mesh[j + 1] - mesh[j], yi, Kk);
+        bool piv = false;
+        firk_inner<M, S, false, true>(I, T, z, nullptr, mesh[j], mesh[j + 1] - mesh[j], yi, Kk, piv);
     } else {
+        const size_t o = firk_off<S * M>(N, j, true);
 #pragma unroll
         for (int r = 0; r < S; ++r)
 #pragma unroll
             for (int c = 0; c < M; ++c) {
-                const size_t q = ((size_t)j * S + r) * M + c;
+                const size_t q = o + (size_t)(r * M + c) * WAVE;
                 Kk[r][c] = (dK ? K[q] + alpha * dK[q] : K[q]) + (dK2 ? beta * dK2[q] : 0.0);
             }
     }
@@ -529,12 +711,13 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
 #pragma unroll
         for (int c = 0; c < M; ++c) ca[c] = g[c];
         if (!nest.on) {
+            const double *lk = loc + firk_off<kFirkLoc<M, S>>(N, j, true);
 #pragma unroll
             for (int q = 0; q < NN; ++q) {
                 const double gq = g[2 * M + q];
-                cst += gq * lk[q];
+                cst += gq * lk[q * WAVE];
 #pragma unroll
-                for (int c = 0; c < M; ++c) ca[c] += gq * lk[NN + q * M + c];
+                for (int c = 0; c < M; ++c) ca[c] += gq * lk[(NN + q * M + c) * WAVE];
             }
         }
 #pragma unroll
@@ -548,14 +731,14 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
 template <int M, int S>
 __device__ inline double firk_bc_row(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, const double *mesh,
                                      const double *y, const double *K, const double *dy, const double *dK,
-                                     double alpha, int k, const BcLoc &L, const double *dy2 = nullptr,
+                                     double alpha, int k, const BcLoc &L, int N, const double *dy2 = nullptr,
                                      const double *dK2 = nullptr, double beta = 0.0) {
     if (L.iv < 0 || !nest.irows) {
         const size_t q = (size_t)L.node * M + sel<M>(I.bcc, k);
         return (dy ? y[q] + alpha * dy[q] : y[q]) + (dy2 ? beta * dy2[q] : 0.0) - sel<M>(I.bcv, k);
     }
-    return firk_bc_interior<M, S, false>(I, T, nest, mesh, y, K, dy, dK, alpha, k, L.iv, nullptr, nullptr, dy2, dK2,
-                                         beta);
+    return firk_bc_interior<M, S, false>(I, T, nest, mesh, y, K, dy, dK, alpha, k, L.iv, nullptr, nullptr, N, dy2,
+                                         dK2, beta);
 }
 
 // Boundary rows of the FIRK path at (y, K): residuals and nodes in sh.
@@ -565,60 +748,83 @@ __device__ inline void firk_bc_rows(const Inst<M> &I, const FirkTab &T, const Fi
     if (lane < M) {
         const BcLoc L = bc_locate<M>(I, lane, mesh, N);
         sh.bcnode[lane] = L.node;
-        sh.bcres[lane] = firk_bc_row<M, S>(I, T, nest, mesh, y, K, nullptr, nullptr, 0.0, lane, L);
+        sh.bcres[lane] = firk_bc_row<M, S>(I, T, nest, mesh, y, K, nullptr, nullptr, 0.0, lane, L, N);
     }
     __syncthreads();
 }
 
 // ------------------------------------------------------------------ Newton pieces
+// Largest |Phi| and (expanded) |G| of one interval's residual, folded into mx and bad.
+template <int M, int S>
+__device__ __forceinline__ void firk_fold(const double (&Phi)[M], const double (&G)[S][M], bool nested, double &mx,
+                                          bool &bad) {
+#pragma unroll
+    for (int c = 0; c < M; ++c) {
+        const double a = fabs(Phi[c]);
+        bad |= !(a <= 1.7976931348623157e308);
+        mx = fmax(mx, a);
+    }
+    if (nested) return;
+#pragma unroll
+    for (int r = 0; r < S; ++r)
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            const double a = fabs(G[r][c]);
+            bad |= !(a <= 1.7976931348623157e308);
+            mx = fmax(mx, a);
+        }
+}
+
 // Forward pass at (y, K): residual max (NaN-aware), per-interval records (loc) and the
 // chunk elimination (Back records in scr, the chunk relation in rel).  Returns
 // max|F| over Phi, G and the boundary rows in all lanes (NaN if not finite); *sing is
 // set when a local system was singular.  Nested form: K is written, not read (each
 // interval's stages solved from k0), and max|F| is over Phi and the boundary rows.
-template <int M, int S>
-__device__ inline double firk_forward(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
-                                      const double *mesh, const double *y, double *K, int N, int lane, double *scr,
-                                      double *loc, Rel<M> &rel, bool &sing) {
+// The chunk pass of one lane.  PIV: local systems with row exchanges; without, the pass
+// stops with piv set as soon as a lane needs one.
+template <int M> struct FirkPass {
+    double mx;
+    bool bad, sg, piv;
+};
+template <int M, int S, bool PIV>
+__device__ __forceinline__ void firk_chunk(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double *sl,
+                                           const double *mesh, const double *y, double *K, int N, int lane,
+                                           double *scr, double *loc, Rel<M> &rel, FirkPass<M> &ps) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
-    double mx = 0.0;
-    bool bad = false, sg = false;
-    for (int k = start; k < start + len; ++k) {
-        const double ti = mesh[k], h = mesh[k + 1] - ti;
-        double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
+    ps.mx = 0.0;
+    ps.bad = ps.sg = ps.piv = false;
+    // the left node of the next interval is this one's right node
+    double ti = 0.0, yi[M];
+    if (len > 0) {
+        ti = mesh[start];
 #pragma unroll
-        for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
+        for (int c = 0; c < M; ++c) yi[c] = y[(size_t)start * M + c];
+    }
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
+        const double tj = mesh[k + 1], h = tj - ti;
+        double yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
+#pragma unroll
+        for (int c = 0; c < M; ++c) yj[c] = y[(size_t)(k + 1) * M + c];
+        const size_t ko = firk_off<S * M>(lane, i);
         if (nest.on) {
-            firk_inner<M, S>(I, T, nest, ti, h, yi, Kk);
-            store_stages<M, S>(K, k, Kk);
+            firk_inner<M, S, kFirkSlotLds<M, S>, PIV>(I, T, nest, sl, ti, h, yi, Kk, ps.piv);
+            store_stages<M, S>(K, ko, Kk);
         } else {
-            load_stages<M, S>(K, k, Kk);
+            load_stages<M, S>(K, ko, Kk);
         }
-        firk_interval<M, S, true>(I, T, ti, h, yi, yj, Kk, G, Phi, J);
-#pragma unroll
-        for (int c = 0; c < M; ++c) {
-            const double a = fabs(Phi[c]);
-            bad |= !(a <= 1.7976931348623157e308);
-            mx = fmax(mx, a);
-        }
-        if (!nest.on) {
-#pragma unroll
-            for (int r = 0; r < S; ++r)
-#pragma unroll
-                for (int c = 0; c < M; ++c) {
-                    const double a = fabs(G[r][c]);
-                    bad |= !(a <= 1.7976931348623157e308);
-                    mx = fmax(mx, a);
-                }
-        }
+        firk_interval<M, S, true>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
+        firk_fold<M, S>(Phi, G, nest.on, ps.mx, ps.bad);
         double Sb[M][M], rhs[M], Rb[M][M];
-        sg |= !firk_condense<M, S>(T, h, G, Phi, J, loc + (size_t)k * kFirkLoc<M, S>, Sb, rhs, nest.on);
+        ps.sg |= !firk_condense<M, S, PIV>(T, h, G, Phi, J, loc + firk_off<kFirkLoc<M, S>>(lane, i), Sb, rhs, nest.on,
+                                           ps.piv);
+        if (!PIV && ps.piv) break;
 #pragma unroll
         for (int a = 0; a < M; ++a)
 #pragma unroll
             for (int c = 0; c < M; ++c) Rb[a][c] = (a == c) ? 1.0 : 0.0;
-        if (k == start) {
+        if (i == 0) {
 #pragma unroll
             for (int a = 0; a < M; ++a) {
 #pragma unroll
@@ -629,10 +835,93 @@ __device__ inline double firk_forward(const Inst<M> &I, const FirkTab &T, const 
             Rel<M> nr;
             Back<M> bk;
             eliminate<M>(rel, Sb, Rb, rhs, nr, bk);
-            put_rec<M, false>(scr, k - start - 1, lane, bk);
+            put_rec<M, false>(scr, i - 1, lane, bk);
             rel = nr;
         }
+        ti = tj;
+#pragma unroll
+        for (int c = 0; c < M; ++c) yi[c] = yj[c];
     }
+}
+
+// The chunk pass with row exchanges, out of line (in line, the exchanges cost the plain
+// pass hundreds of spill stores per interval); its relation comes back through LDS.  NEST:
+// the form, -1 for both.
+template <int M> struct FirkPivArgs {
+    const FirkTab *T;
+    const double *params, *mesh, *y;
+    double *sl, *K, *scr, *loc, *rel;
+    int pcnt, fam, N, lane;
+    FirkNest<M> nest;
+};
+template <int M, int S, int NEST>
+__device__ __noinline__ FirkPass<M> firk_chunk_pivoted(FirkPivArgs<M> a) {
+    Inst<M> I;
+    I.fam = a.fam;
+    I.minc = 1;
+#pragma unroll
+    for (int k = 0; k < Params<M>::MAXP; ++k) I.P.p[k] = k < a.pcnt ? a.params[k] : 0.0;
+    FirkNest<M> nest = a.nest;
+    if constexpr (NEST >= 0) nest.on = NEST != 0;
+    Rel<M> rel;
+    FirkPass<M> ps;
+    firk_chunk<M, S, true>(I, *a.T, nest, a.sl, a.mesh, a.y, a.K, a.N, a.lane, a.scr, a.loc, rel, ps);
+    __syncthreads();  // the exchange area shares its LDS with the relations
+    int f = 0;
+    double *o = a.rel + (size_t)a.lane * kRelFields<M>;
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int c = 0; c < M; ++c) o[f++] = rel.E[i][c];
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int c = 0; c < M; ++c) o[f++] = rel.F[i][c];
+#pragma unroll
+    for (int i = 0; i < M; ++i) o[f++] = rel.g[i];
+    return ps;
+}
+
+// Where the local systems run without row exchanges first (DIAG): from 6 unknowns (below, the
+// exchanges cost little) to 12 (above, the solve runs rolled over private arrays), in the
+// solve kernels of one wave per SIMD (the pivoted pass takes more registers than two leave).
+// Solve kernel at M = 2, one wave per SIMD: s = 5, 2,048 Bratu problems 12.6 ms before, 3.6 ms
+// (7.9 ms with the layout and the stage loop alone); nested s = 3, 4,096 problems 3.18 -> 2.50 ms.
+template <int M, int S> constexpr bool kFirkDiag = S * M >= 6 && S * M <= 12;
+
+// sticky: an earlier pass of this instance needed row exchanges (kept by the caller)
+template <int M, int S, bool DIAG>
+__device__ __forceinline__ double firk_forward(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest,
+                                               Shared<M> &sh, const double *mesh, const double *y, double *K, int N,
+                                               int lane, double *scr, double *loc, Rel<M> &rel, bool &sing,
+                                               bool &sticky) {
+    double *sl = firk_slot<M, S>(sh, lane);
+    FirkPass<M> ps;
+    if constexpr (kFirkBig<M, S>) {
+        FirkPivArgs<M> a{&T, I.params, mesh, y, sl, K, scr, loc, &sh.rel[0][0], I.pcnt, I.fam, N, lane, nest};
+        ps = firk_chunk_pivoted<M, S, -1>(a);
+        __syncthreads();
+        rel_from_lds<M>(sh, lane, rel);
+        __syncthreads();
+    } else if constexpr (DIAG) {
+        if (!sticky) {
+            firk_chunk<M, S, false>(I, T, nest, sl, mesh, y, K, N, lane, scr, loc, rel, ps);
+            sticky = wave_any(ps.piv);
+            __syncthreads();  // the exchange area's LDS is the tree's next
+        }
+        if (sticky) {
+            FirkPivArgs<M> a{&T, I.params, mesh, y, sl, K, scr, loc, &sh.rel[0][0], I.pcnt, I.fam, N, lane, nest};
+            ps = nest.on ? firk_chunk_pivoted<M, S, 1>(a) : firk_chunk_pivoted<M, S, 0>(a);
+            __syncthreads();
+            rel_from_lds<M>(sh, lane, rel);
+            __syncthreads();
+        }
+    } else {
+        firk_chunk<M, S, true>(I, T, nest, sl, mesh, y, K, N, lane, scr, loc, rel, ps);
+        __syncthreads();
+    }
+    double mx = ps.mx;
+    bool bad = ps.bad;
     firk_bc_rows<M, S>(I, T, nest, sh, mesh, y, K, N, lane);
 #pragma unroll
     for (int k = 0; k < M; ++k) {
@@ -641,87 +930,161 @@ __device__ inline double firk_forward(const Inst<M> &I, const FirkTab &T, const 
         mx = fmax(mx, a);
     }
     const bool anybad = wave_any(bad);
-    sing = wave_any(sg);
+    sing = wave_any(ps.sg);
     mx = wave_max(mx);
     __syncthreads();
-    return anybad ? NAN : mx;
+    return uniform(anybad ? NAN : mx);
 }
 
-// Tree solve and back-substitution of the condensed system: dy at the nodes, then
-// dK = kg + KJ dy_i per interval.  dy: [N+1][M], dK: [N][S][M].  Returns false when
-// the root system is singular.
-template <int M, int S, bool IR = true>
-__device__ inline bool firk_correction(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
-                                       const double *mesh, const double *y, const double *K, int N, int lane,
-                                       double *scr, const double *loc, Rel<M> &rel, double *dy, double *dK) {
-    const bool nested = nest.on;
+// What the back-substitution does with the corrections dy at the nodes and
+// dK = kg + KJ dy_i of the stages: store them (a line search or trust region follows), add
+// them to the state, or add them and evaluate max|F| there while the interval's new nodes
+// and stages are in registers.
+enum { FIRK_STORE = 0, FIRK_APPLY = 1, FIRK_CHECK = 2 };
+
+// Tree solve of the condensed system: the corrections at the chunk ends in sh.lo, sh.hi.
+// Returns false when the root system is singular.
+template <int M, int S, bool IR>
+__device__ __forceinline__ bool firk_tree(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+                                          const double *mesh, const double *y, const double *K, int N, int lane,
+                                          double *scr, const double *loc, Rel<M> &rel) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
-    // the linearisation of rows inside the span (rows read from a node carry a zero flag)
-    double *irow = static_cast<FirkShared<M> &>(sh).irow;
     if constexpr (IR) {
+        // the linearisation of rows inside the span (rows read from a node carry a zero flag)
+        double *irow = static_cast<FirkShared<M> &>(sh).irow;
         __syncthreads();  // the interval records are read across lanes
         if (lane < M) {
             const BcLoc L = bc_locate<M>(I, lane, mesh, N);
             double *ir = irow + lane * (2 * M + 2);
             ir[2 * M + 1] = L.iv >= 0 ? 1.0 : 0.0;
             if (L.iv >= 0)
-                firk_bc_interior<M, S, true>(I, T, nest, mesh, y, K, nullptr, nullptr, 0.0, lane, L.iv,
-                                             loc + (size_t)L.iv * kFirkLoc<M, S>, ir);
+                firk_bc_interior<M, S, true>(I, T, nest, mesh, y, K, nullptr, nullptr, 0.0, lane, L.iv, loc, ir, N);
         }
-        if (!tree_solve<M, false, true>(I, sh, N, lane, P, scr, rel, irow)) return false;
-    } else if (!tree_solve<M, false>(I, sh, N, lane, P, scr, rel)) {
-        return false;
+        return tree_solve<M, false, true>(I, sh, N, lane, P, scr, rel, irow);
+    } else {
+        return tree_solve<M, false>(I, sh, N, lane, P, scr, rel);
     }
+}
+
+// Back-substitution after firk_tree; fn receives max|F| at the new state (FIRK_CHECK; NaN if
+// not finite).
+template <int M, int S, bool DIAG, int MODE>
+__device__ __forceinline__ void firk_back(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+                                          const double *mesh, double *y, double *K, int N, int lane,
+                                          const double *scr, const double *loc, double *dy, double *dK,
+                                          double *fn = nullptr) {
+    constexpr int NN = S * M;
+    const bool nested = nest.on;
+    double *sl = firk_slot<M, S>(sh, lane);
+    int P, start, len;
+    chunk_of(N, lane, P, start, len);
+    double mx = 0.0;
+    bool bad = false, piv = false;
+    // tree_solve ends on a barrier; its lo and hi lie outside the exchange area's LDS
     if (len > 0) {
-        double ya[M], yn[M];
+        double ya[M], yn[M], yr[M], tr = 0.0;
 #pragma unroll
         for (int c = 0; c < M; ++c) { ya[c] = sh.lo[lane][c]; yn[c] = sh.hi[lane][c]; }
+        // the new state at the chunk's right end, read before any lane writes the state
+        if constexpr (MODE == FIRK_CHECK) {
+            tr = mesh[start + len];
+#pragma unroll
+            for (int c = 0; c < M; ++c) yr[c] = y[(size_t)(start + len) * M + c] + yn[c];
+        }
         if (lane == P - 1)
 #pragma unroll
-            for (int c = 0; c < M; ++c) dy[(size_t)N * M + c] = yn[c];
-        for (int k = start + len - 1; k > start; --k) {
-            Back<M> bk;
-            get_rec<M, false>(scr, k - start - 1, lane, bk);
-            double yk[M];
-            back_apply<M>(bk, ya, yn, yk);
+            for (int c = 0; c < M; ++c) {
+                if constexpr (MODE == FIRK_STORE) dy[(size_t)N * M + c] = yn[c];
+                else y[(size_t)N * M + c] += yn[c];
+            }
+        // intervals from the right: node k = start + i, its record in slot i - 1
+        for (int i = len - 1; i >= 0; --i) {
+            const int k = start + i;
+            const double *lk = loc + firk_off<kFirkLoc<M, S>>(lane, i);
+            const size_t ko = firk_off<NN>(lane, i);
+            double d[M], yl[M];
+            if (i > 0) {
+                Back<M> bk;
+                get_rec<M, false>(scr, i - 1, lane, bk);
+                back_apply<M>(bk, ya, yn, d);
+            } else {
 #pragma unroll
-            for (int c = 0; c < M; ++c) { dy[(size_t)k * M + c] = yk[c]; yn[c] = yk[c]; }
-        }
+                for (int c = 0; c < M; ++c) d[c] = ya[c];
+            }
 #pragma unroll
-        for (int c = 0; c < M; ++c) dy[(size_t)start * M + c] = ya[c];
-        // stage corrections of the chunk's intervals (dy of their left nodes: just written by
-        // this lane); the nested form has no stage unknowns
-        constexpr int NN = S * M;
-        for (int k = start; k < start + (nested ? 0 : len); ++k) {
-            const double *lk = loc + (size_t)k * kFirkLoc<M, S>;
-            double d[M];
+            for (int c = 0; c < M; ++c) {
+                if constexpr (MODE == FIRK_STORE) {
+                    dy[(size_t)k * M + c] = d[c];
+                } else {
+                    yl[c] = y[(size_t)k * M + c] + d[c];
+                    y[(size_t)k * M + c] = yl[c];
+                }
+                yn[c] = d[c];
+            }
+            // stage corrections (the nested form has no stage unknowns)
+            double Kk[S][M];
+            if (!nested) {
 #pragma unroll
-            for (int c = 0; c < M; ++c) d[c] = dy[(size_t)k * M + c];
+                for (int q = 0; q < NN; ++q) {
+                    double v = lk[q * WAVE];
 #pragma unroll
-            for (int q = 0; q < NN; ++q) {
-                double v = lk[q];
+                    for (int c = 0; c < M; ++c) v += lk[(NN + q * M + c) * WAVE] * d[c];
+                    if constexpr (MODE == FIRK_STORE) {
+                        dK[ko + (size_t)q * WAVE] = v;
+                    } else {
+                        Kk[q / M][q % M] = K[ko + (size_t)q * WAVE] + v;
+                        K[ko + (size_t)q * WAVE] = Kk[q / M][q % M];
+                    }
+                }
+            }
+            if constexpr (MODE == FIRK_CHECK) {
+                const double tl = mesh[k], h = tr - tl;
+                if (nested) {
+                    firk_inner<M, S, kFirkSlotLds<M, S>, !DIAG>(I, T, nest, sl, tl, h, yl, Kk, piv);
+                    store_stages<M, S>(K, ko, Kk);
+                }
+                double G[S][M], Phi[M], J[S][M][M];
+                firk_interval<M, S, false>(I, T, sl, tl, h, yl, yr, Kk, G, Phi, J);
+                firk_fold<M, S>(Phi, G, nested, mx, bad);
+                tr = tl;
 #pragma unroll
-                for (int c = 0; c < M; ++c) v += lk[NN + q * M + c] * d[c];
-                dK[(size_t)k * NN + q] = v;
+                for (int c = 0; c < M; ++c) yr[c] = yl[c];
             }
         }
     }
     __syncthreads();
-    return true;
+    if constexpr (MODE == FIRK_CHECK) {
+        firk_bc_rows<M, S>(I, T, nest, sh, mesh, y, K, N, lane);
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+            const double a = fabs(sh.bcres[k]);
+            bad |= !(a <= 1.7976931348623157e308);
+            mx = fmax(mx, a);
+        }
+        const bool anybad = wave_any(bad);
+        mx = wave_max(mx);
+        // an inner solve that needs row exchanges: not known to have converged, the next
+        // forward pass decides
+        *fn = wave_any(piv) ? 1.7976931348623157e308 : uniform(anybad ? NAN : mx);
+        __syncthreads();
+    }
 }
+
 
 // Sum of squares of the residual at (y + alpha dy, K + alpha dK) (the line search's
 // merit, times 2) in all lanes; NaN if not finite.
 template <int M, int S>
-__device__ inline double firk_trial_sumsq(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest,
+__device__ inline double firk_trial_sumsq(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
                                           const double *mesh, const double *y, const double *K, const double *dy,
                                           const double *dK, double alpha, int N, int lane) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
+    double *sl = firk_slot<M, S>(sh, lane);
     double ss = 0.0;
-    bool bad = false;
-    for (int k = start; k < start + len; ++k) {
+    bool bad = false, piv = false;
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
         const double ti = mesh[k], h = mesh[k + 1] - ti;
         double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
@@ -730,17 +1093,18 @@ __device__ inline double firk_trial_sumsq(const Inst<M> &I, const FirkTab &T, co
             yj[c] = y[(size_t)(k + 1) * M + c] + alpha * dy[(size_t)(k + 1) * M + c];
         }
         if (nest.on) {
-            firk_inner<M, S>(I, T, nest, ti, h, yi, Kk);
+            firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
         } else {
+            const size_t ko = firk_off<S * M>(lane, i);
 #pragma unroll
             for (int r = 0; r < S; ++r)
 #pragma unroll
                 for (int c = 0; c < M; ++c) {
-                    const size_t q = ((size_t)k * S + r) * M + c;
+                    const size_t q = ko + (size_t)(r * M + c) * WAVE;
                     Kk[r][c] = K[q] + alpha * dK[q];
                 }
         }
-        firk_interval<M, S, false>(I, T, ti, h, yi, yj, Kk, G, Phi, J);
+        firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
 #pragma unroll
         for (int c = 0; c < M; ++c) ss += Phi[c] * Phi[c];
         if (!nest.on) {
@@ -752,13 +1116,13 @@ __device__ inline double firk_trial_sumsq(const Inst<M> &I, const FirkTab &T, co
     }
     if (lane < M) {
         const BcLoc L = bc_locate<M>(I, lane, mesh, N);
-        const double v = firk_bc_row<M, S>(I, T, nest, mesh, y, K, dy, dK, alpha, lane, L);
+        const double v = firk_bc_row<M, S>(I, T, nest, mesh, y, K, dy, dK, alpha, lane, L, N);
         ss += v * v;
     }
     bad = !(fabs(ss) <= 1.7976931348623157e308);
     const bool anybad = wave_any(bad);
     ss = wave_sum(ss);
-    return anybad ? NAN : uniform(ss);
+    return uniform(anybad ? NAN : ss);
 }
 
 // x += alpha d over the nodes and stages of the lane's chunk (node N by the last lane)
@@ -767,12 +1131,14 @@ __device__ inline void firk_apply(double *y, double *K, const double *dy, const 
                                   int lane, bool nested) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
-    for (int k = start; k < start + len; ++k) {
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
+        const size_t ko = firk_off<S * M>(lane, i);
 #pragma unroll
         for (int c = 0; c < M; ++c) y[(size_t)k * M + c] += alpha * dy[(size_t)k * M + c];
         if (!nested) {
 #pragma unroll
-            for (int q = 0; q < S * M; ++q) K[(size_t)k * S * M + q] += alpha * dK[(size_t)k * S * M + q];
+            for (int q = 0; q < S * M; ++q) K[ko + (size_t)q * WAVE] += alpha * dK[ko + (size_t)q * WAVE];
         }
     }
     if (lane == P - 1)
@@ -784,7 +1150,10 @@ __device__ inline void firk_apply(double *y, double *K, const double *dy, const 
 template <int M, int S>
 __device__ inline void firk_copy_state(double *yd, double *Kd, const double *ys, const double *Ks, int N, int lane) {
     for (int q = lane; q < (N + 1) * M; q += WAVE) yd[q] = ys[q];
-    for (int q = lane; q < N * S * M; q += WAVE) Kd[q] = Ks[q];
+    firk_each<S * M>(N, lane, [&](size_t o) {
+#pragma unroll
+        for (int q = 0; q < S * M; ++q) Kd[o + (size_t)q * WAVE] = Ks[o + (size_t)q * WAVE];
+    });
     __syncthreads();
 }
 
@@ -808,18 +1177,21 @@ template <int M> __device__ inline FirkNest<M> firk_expanded_rows() {
 // (the Jacobian of FIRK/collocation.jl:59-93 that the oracle assembles), stage
 // Jacobians J_r evaluated at (y, K).  firk_jt_f: g = J'F into (gy [N+1][M], gK [N][S][M]).
 template <int M, int S>
-__device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, const double *mesh, const double *y,
-                                 const double *K, int N, int lane, double *gy, double *gK) {
+__device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
+                                 const double *y, const double *K, int N, int lane, double *gy, double *gK) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
+    double *sl = firk_slot<M, S>(sh, lane);
     // pass 1: each interval's terms on y_i and K_i (node N: zero)
-    for (int k = start; k < start + len; ++k) {
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
+        const size_t ko = firk_off<S * M>(lane, i);
         const double ti = mesh[k], h = mesh[k + 1] - ti;
         double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
         for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
-        load_stages<M, S>(K, k, Kk);
-        firk_interval<M, S, true>(I, T, ti, h, yi, yj, Kk, G, Phi, J);
+        load_stages<M, S>(K, ko, Kk);
+        firk_interval<M, S, true>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
 #pragma unroll
         for (int c = 0; c < M; ++c) {
             double v = -Phi[c];
@@ -838,7 +1210,7 @@ __device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, const doubl
                 for (int r = 0; r < S; ++r)
 #pragma unroll
                     for (int a = 0; a < M; ++a) v += h * T.A[r][j] * J[r][a][c] * G[r][a];
-                gK[((size_t)k * S + j) * M + c] = v;
+                gK[ko + (size_t)(j * M + c) * WAVE] = v;
             }
     }
     if (lane == P - 1)
@@ -846,10 +1218,11 @@ __device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, const doubl
         for (int c = 0; c < M; ++c) gy[(size_t)N * M + c] = 0.0;
     __syncthreads();
     // pass 2: Phi_i on y_{i+1}
-    for (int k = start; k < start + len; ++k) {
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
         const double h = mesh[k + 1] - mesh[k];
         double Kk[S][M];
-        load_stages<M, S>(K, k, Kk);
+        load_stages<M, S>(K, firk_off<S * M>(lane, i), Kk);
 #pragma unroll
         for (int c = 0; c < M; ++c) {
             double a = 0.0;
@@ -870,13 +1243,14 @@ __device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, const doubl
                 const int j = L.iv;
                 double g[(S + 2) * M];
                 const double v = firk_bc_interior<M, S, true>(I, T, firk_expanded_rows<M>(), mesh, y, K, nullptr,
-                                                              nullptr, 0.0, r, j, nullptr, nullptr, nullptr, nullptr,
+                                                              nullptr, 0.0, r, j, nullptr, nullptr, N, nullptr, nullptr,
                                                               0.0, g);
                 for (int c = 0; c < M; ++c) {
                     gy[(size_t)j * M + c] += v * g[c];
                     gy[(size_t)(j + 1) * M + c] += v * g[M + c];
                 }
-                for (int q = 0; q < S * M; ++q) gK[(size_t)j * S * M + q] += v * g[2 * M + q];
+                const size_t jo = firk_off<S * M>(N, j, true);
+                for (int q = 0; q < S * M; ++q) gK[jo + (size_t)q * WAVE] += v * g[2 * M + q];
             }
         }
     __syncthreads();
@@ -884,19 +1258,23 @@ __device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, const doubl
 
 // |J g|^2 for g = (gy, gK), in all lanes
 template <int M, int S>
-__device__ inline double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, const double *mesh, const double *y,
-                                        const double *K, const double *gy, const double *gK, int N, int lane) {
+__device__ inline double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
+                                        const double *y, const double *K, const double *gy, const double *gK, int N,
+                                        int lane) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
+    double *sl = firk_slot<M, S>(sh, lane);
     double acc = 0.0;
-    for (int k = start; k < start + len; ++k) {
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
+        const size_t ko = firk_off<S * M>(lane, i);
         const double ti = mesh[k], h = mesh[k + 1] - ti;
         double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M], gk[S][M];
 #pragma unroll
         for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
-        load_stages<M, S>(K, k, Kk);
-        load_stages<M, S>(gK, k, gk);
-        firk_interval<M, S, true>(I, T, ti, h, yi, yj, Kk, G, Phi, J);
+        load_stages<M, S>(K, ko, Kk);
+        load_stages<M, S>(gK, ko, gk);
+        firk_interval<M, S, true>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
 #pragma unroll
         for (int a = 0; a < M; ++a) {
             double v = gy[(size_t)(k + 1) * M + a] - gy[(size_t)k * M + a];
@@ -929,10 +1307,11 @@ __device__ inline double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, cons
                 const int j = L.iv;
                 double g[(S + 2) * M];
                 firk_bc_interior<M, S, true>(I, T, firk_expanded_rows<M>(), mesh, y, K, nullptr, nullptr, 0.0, r, j,
-                                             nullptr, nullptr, nullptr, nullptr, 0.0, g);
+                                             nullptr, nullptr, N, nullptr, nullptr, 0.0, g);
                 v = 0.0;
                 for (int c = 0; c < M; ++c) v += g[c] * gy[(size_t)j * M + c] + g[M + c] * gy[(size_t)(j + 1) * M + c];
-                for (int q = 0; q < S * M; ++q) v += g[2 * M + q] * gK[(size_t)j * S * M + q];
+                const size_t jo = firk_off<S * M>(N, j, true);
+                for (int q = 0; q < S * M; ++q) v += g[2 * M + q] * gK[jo + (size_t)q * WAVE];
             }
             acc += v * v;
         }
@@ -943,13 +1322,16 @@ __device__ inline double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, cons
 
 // |F|^2 and max|F| at (y + a dy + b gy, K + a dK + b gK), in all lanes (NaN if not finite)
 template <int M, int S>
-__device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, const double *mesh, const double *y,
-                                     const double *K, const double *dy, const double *dK, double a, const double *gy,
+__device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
+                                     const double *y, const double *K, const double *dy, const double *dK, double a, const double *gy,
                                      const double *gK, double b, int N, int lane, double &mx) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
+    double *sl = firk_slot<M, S>(sh, lane);
     double ss = 0.0, m = 0.0;
-    for (int k = start; k < start + len; ++k) {
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
+        const size_t ko = firk_off<S * M>(lane, i);
         const double ti = mesh[k], h = mesh[k + 1] - ti;
         double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
@@ -962,10 +1344,10 @@ __device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, const d
         for (int r = 0; r < S; ++r)
 #pragma unroll
             for (int c = 0; c < M; ++c) {
-                const size_t q = ((size_t)k * S + r) * M + c;
+                const size_t q = ko + (size_t)(r * M + c) * WAVE;
                 Kk[r][c] = K[q] + a * dK[q] + b * gK[q];
             }
-        firk_interval<M, S, false>(I, T, ti, h, yi, yj, Kk, G, Phi, J);
+        firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
 #pragma unroll
         for (int c = 0; c < M; ++c) { ss += Phi[c] * Phi[c]; m = fmax(m, fabs(Phi[c])); }
 #pragma unroll
@@ -976,7 +1358,7 @@ __device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, const d
     if (lane < M) {
         const BcLoc L = bc_locate<M>(I, lane, mesh, N);
         const double v =
-            firk_bc_row<M, S>(I, T, firk_expanded_rows<M>(), mesh, y, K, dy, dK, a, lane, L, gy, gK, b);
+            firk_bc_row<M, S>(I, T, firk_expanded_rows<M>(), mesh, y, K, dy, dK, a, lane, L, N, gy, gK, b);
         ss += v * v;
         m = fmax(m, fabs(v));
     }
@@ -993,22 +1375,27 @@ __device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, const d
 // radius update; the restatement the oracle follows, Core/default_internal_solve.jl:
 // 37-43).  Boundary rows anywhere in the span.
 // gy, gK: work areas for J'F.
-template <int M, int S>
+template <int M, int S, bool DIAG>
 __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, const FirkTab &T,
                                         const FirkNest<M> &nest, Shared<M> &sh, const double *mesh, double *y,
                                         double *K, int N, int lane, double *scr, double *loc, double *dy, double *dK,
                                         double *gy, double *gK, FirkNewtonOut &out) {
     double mx;
-    double ss = firk_trial2<M, S>(I, T, mesh, y, K, y, K, 0.0, y, K, 0.0, N, lane, mx);
+    double ss = firk_trial2<M, S>(I, T, sh, mesh, y, K, y, K, 0.0, y, K, 0.0, N, lane, mx);
     double xmax = -INFINITY, xmin = INFINITY;
     for (int q = lane; q < (N + 1) * M; q += WAVE) { xmax = fmax(xmax, y[q]); xmin = fmin(xmin, y[q]); }
-    for (int q = lane; q < N * S * M; q += WAVE) { xmax = fmax(xmax, K[q]); xmin = fmin(xmin, K[q]); }
+    firk_each<S * M>(N, lane, [&](size_t o) {
+        for (int q = 0; q < S * M; ++q) {
+            xmax = fmax(xmax, K[o + (size_t)q * WAVE]);
+            xmin = fmin(xmin, K[o + (size_t)q * WAVE]);
+        }
+    });
     xmax = uniform(wave_max(xmax));
     xmin = uniform(-wave_max(-xmin));
     __syncthreads();
     double radius = fmax(sqrt(ss), xmax - xmin) / 11.0;
     int shrinks = 0;
-    bool fresh = true;
+    bool fresh = true, sticky = false;
     double dn2 = 0.0, l2 = 0.0, gdn = 0.0, jg2 = 0.0;
     for (int it = 0;; ++it) {
         out.fn = mx;
@@ -1018,26 +1405,29 @@ __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, con
         if (fresh) {
             Rel<M> rel;
             bool sing = false;
-            firk_forward<M, S>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing);
-            if (sing || !firk_correction<M, S, false>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, dy, dK))
-                return BVP_RET_FAILURE;
-            firk_jt_f<M, S>(I, T, mesh, y, K, N, lane, gy, gK);
+            firk_forward<M, S, DIAG>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing, sticky);
+            if (sing || !firk_tree<M, S, false>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel)) return BVP_RET_FAILURE;
+            firk_back<M, S, DIAG, FIRK_STORE>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
+            firk_jt_f<M, S>(I, T, sh, mesh, y, K, N, lane, gy, gK);
             double a = 0.0, b = 0.0, c = 0.0;
             for (int q = lane; q < (N + 1) * M; q += WAVE) {
                 a += dy[q] * dy[q];
                 b += gy[q] * gy[q];
                 c += gy[q] * dy[q];
             }
-            for (int q = lane; q < N * S * M; q += WAVE) {
-                a += dK[q] * dK[q];
-                b += gK[q] * gK[q];
-                c += gK[q] * dK[q];
-            }
+            firk_each<S * M>(N, lane, [&](size_t o) {
+                for (int q = 0; q < S * M; ++q) {
+                    const double d = dK[o + (size_t)q * WAVE], g = gK[o + (size_t)q * WAVE];
+                    a += d * d;
+                    b += g * g;
+                    c += g * d;
+                }
+            });
             dn2 = uniform(wave_sum(a));
             l2 = uniform(wave_sum(b));
             gdn = uniform(wave_sum(c));
             __syncthreads();
-            jg2 = firk_jac_norm2<M, S>(I, T, mesh, y, K, gy, gK, N, lane);
+            jg2 = firk_jac_norm2<M, S>(I, T, sh, mesh, y, K, gy, gK, N, lane);
             fresh = false;
         }
         out.iters++;
@@ -1061,11 +1451,14 @@ __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, con
             }
         }
         double mxt;
-        const double sst = firk_trial2<M, S>(I, T, mesh, y, K, dy, dK, cn, gy, gK, cg, N, lane, mxt);
+        const double sst = firk_trial2<M, S>(I, T, sh, mesh, y, K, dy, dK, cn, gy, gK, cg, N, lane, mxt);
         const double rho = (ss - sst) / pred;
         if (rho > 1e-4) {
             for (int q = lane; q < (N + 1) * M; q += WAVE) y[q] += cn * dy[q] + cg * gy[q];
-            for (int q = lane; q < N * S * M; q += WAVE) K[q] += cn * dK[q] + cg * gK[q];
+            firk_each<S * M>(N, lane, [&](size_t o) {
+                for (int q = 0; q < S * M; ++q)
+                    K[o + (size_t)q * WAVE] += cn * dK[o + (size_t)q * WAVE] + cg * gK[o + (size_t)q * WAVE];
+            });
             __syncthreads();
             ss = sst;
             mx = mxt;
@@ -1086,7 +1479,7 @@ __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, con
 // plain, then with the BackTracking line search, each from the same start, stopping
 // when max|F| <= tol (checked before every step).  Work areas: dy [cap][M], dK, the
 // start copy y0 [cap][M], K0, loc.
-template <int M, int S, bool IR = true>
+template <int M, int S, bool IR, bool DIAG>
 __device__ inline FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I, const FirkTab &T,
                                             const FirkNest<M> &nest, Shared<M> &sh, const double *mesh, double *y,
                                             double *K, int N, int lane, double *scr, double *loc, double *dy,
@@ -1094,7 +1487,7 @@ __device__ inline FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I,
     FirkNewtonOut out{BVP_RET_MAXITERS, 0, -1, NAN};
     // the TrustRegion stage: compiled into the general kernels (IR) only
     const int stages = B.stages & (IR ? 7 : 3);
-    bool first = true;
+    bool first = true, sticky = false;
     if (__popc(stages) > 1) firk_copy_state<M, S>(y0, K0, y, K, N, lane);
     for (int st = 0; st < 3; ++st) {
         if (!(stages & (1 << st))) continue;
@@ -1104,7 +1497,7 @@ __device__ inline FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I,
         if constexpr (IR) {
             if (st == 2 && !nest.on) {
                 // the last stage: the start copy is free for J'F
-                out.ret = firk_trust_region<M, S>(B, I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, y0, K0,
+                out.ret = firk_trust_region<M, S, DIAG>(B, I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, y0, K0,
                                                   out);
                 break;
             }
@@ -1112,24 +1505,38 @@ __device__ inline FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I,
         for (int it = 0;; ++it) {
             Rel<M> rel;
             bool sing = false;
-            const double fn = firk_forward<M, S>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing);
+            const double fn = firk_forward<M, S, DIAG>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing, sticky);
             out.fn = fn;
             if (!(fabs(fn) <= 1.7976931348623157e308)) { out.ret = BVP_RET_UNSTABLE; break; }
             if (fn <= B.newton_tol) { out.ret = BVP_RET_SUCCESS; break; }
             if (it >= B.max_newton) { out.ret = BVP_RET_MAXITERS; break; }
-            if (sing || !firk_correction<M, S, IR>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, dy, dK)) {
+            if (sing || !firk_tree<M, S, IR>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel)) {
                 out.ret = BVP_RET_FAILURE;
                 break;
             }
             out.iters++;
-            double alpha = 1.0;
-            if (st == 1) {
-                const double ss = firk_trial_sumsq<M, S>(I, T, nest, mesh, y, K, dy, dK, 0.0, N, lane);
-                auto phi = [&](double a) {
-                    return 0.5 * firk_trial_sumsq<M, S>(I, T, nest, mesh, y, K, dy, dK, a, N, lane);
-                };
-                if (!backtracking(phi, 0.5 * ss, -ss, alpha)) { out.ret = BVP_RET_FAILURE; break; }
+            if (st == 0 && fn <= 100.0 * sqrt(B.newton_tol)) {
+                // a step predicted to converge (as in the MIRK path: quadratic convergence with
+                // a constant of 1e-4): the residual at the new state is evaluated with the
+                // update, which spares the forward pass that would only find it converged
+                double fn2 = NAN;
+                firk_back<M, S, DIAG, FIRK_CHECK>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, &fn2);
+                out.fn = fn2;
+                if (!(fabs(fn2) <= 1.7976931348623157e308)) { out.ret = BVP_RET_UNSTABLE; break; }
+                if (fn2 <= B.newton_tol) { out.ret = BVP_RET_SUCCESS; break; }
+                continue;
             }
+            if (st == 0) {
+                firk_back<M, S, DIAG, FIRK_APPLY>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
+                continue;
+            }
+            firk_back<M, S, DIAG, FIRK_STORE>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
+            double alpha = 1.0;
+            const double ss = firk_trial_sumsq<M, S>(I, T, nest, sh, mesh, y, K, dy, dK, 0.0, N, lane);
+            auto phi = [&](double a) {
+                return 0.5 * firk_trial_sumsq<M, S>(I, T, nest, sh, mesh, y, K, dy, dK, a, N, lane);
+            };
+            if (!backtracking(phi, 0.5 * ss, -ss, alpha)) { out.ret = BVP_RET_FAILURE; break; }
             firk_apply<M, S>(y, K, dy, dK, alpha, N, lane, nest.on);
         }
         if (out.ret == BVP_RET_SUCCESS) break;
@@ -1177,12 +1584,13 @@ __device__ inline double firk_defect_pass(const Inst<M> &I, const FirkTab &T, co
     double dmx = 0.0, s1 = 0.0, s2 = 0.0;
     bool bad = false;
     const double expo = 1.0 / (T.order + 1);
-    for (int k = start; k < start + len; ++k) {
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
         const double ti = mesh[k], h = mesh[k + 1] - ti;
         double yi[M], Kk[S][M], z[M], zp[M], f[M], d1[M], d2[M];
 #pragma unroll
         for (int c = 0; c < M; ++c) yi[c] = y[(size_t)k * M + c];
-        load_stages<M, S>(K, k, Kk);
+        load_stages<M, S>(K, firk_off<S * M>(lane, i), Kk);
         firk_eval_q<M, S>(T, yi, T.tau, h, Kk, z, zp);
         f_eval<M, double>(I.fam, I.P, ti + T.tau * h, z, f);
         double e1 = 0.0, e2 = 0.0;
@@ -1225,7 +1633,9 @@ __device__ inline double firk_defect_pass(const Inst<M> &I, const FirkTab &T, co
 // interval's step in the stage polynomial and the quintic (the nested form's transfer
 // passes the reference's growth factor, FIRK/adaptivity.jl:98-104); with nest.on the
 // stages come from the inner solve (at the unscaled step), else from K.
-template <int M, int S>
+// K: the stages in [interval][S][M] order (PLAIN: the dense output's packed input), or the
+// lane-interleaved state.
+template <int M, int S, bool PLAIN>
 __device__ inline void firk_interp_at(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, const double *mesh,
                                       const double *y, const double *K, int N, double t, double *u, double *du,
                                       double hscale = 1.0) {
@@ -1234,8 +1644,17 @@ __device__ inline void firk_interp_at(const Inst<M> &I, const FirkTab &T, const 
     double yi[M], yj[M], fi[M], fj[M], z[M], zp[M], Kk[S][M];
 #pragma unroll
     for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)j * M + c]; yj[c] = y[(size_t)(j + 1) * M + c]; }
-    if (nest.on && !K) firk_inner<M, S>(I, T, nest, tj, h0, yi, Kk);
-    else load_stages<M, S>(K, j, Kk);
+    if (nest.on && !K) {
+        bool piv = false;
+        firk_inner<M, S, false, true>(I, T, nest, nullptr, tj, h0, yi, Kk, piv);
+    } else if constexpr (PLAIN) {
+#pragma unroll
+        for (int r = 0; r < S; ++r)
+#pragma unroll
+            for (int c = 0; c < M; ++c) Kk[r][c] = K[((size_t)j * S + r) * M + c];
+    } else {
+        load_stages<M, S>(K, firk_off<S * M>(N, j, true), Kk);
+    }
     f_eval<M, double>(I.fam, I.P, tj, yi, fi);
     f_eval<M, double>(I.fam, I.P, mesh[j + 1], yj, fj);
     firk_eval_q<M, S>(T, yi, 0.5, h, Kk, z, zp);
@@ -1260,11 +1679,56 @@ __device__ inline void firk_interp_at(const Inst<M> &I, const FirkTab &T, const 
 // extend_y (FIRK/firk.jl:76-83): every stage of interval i set to y_{i+1}
 template <int M, int S>
 __device__ inline void firk_extend(const double *y, double *K, int N, int lane) {
-    for (int q = lane; q < N * S * M; q += WAVE) {
-        const int i = q / (S * M), c = q % M;
-        K[q] = y[(size_t)(i + 1) * M + c];
+    int P, start, len;
+    chunk_of(N, lane, P, start, len);
+    for (int i = 0; i < len; ++i) {
+        const size_t ko = firk_off<S * M>(lane, i);
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            const double v = y[(size_t)(start + i + 1) * M + c];
+#pragma unroll
+            for (int r = 0; r < S; ++r) K[ko + (size_t)(r * M + c) * WAVE] = v;
+        }
     }
     __syncthreads();
+}
+
+// max|F| at (y, K) (NaN if not finite); the nested form's stages are solved into K
+template <int M, int S>
+__device__ inline double firk_residual_max(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+                                           const double *mesh, const double *y, double *K, int N, int lane) {
+    int P, start, len;
+    chunk_of(N, lane, P, start, len);
+    double *sl = firk_slot<M, S>(sh, lane);
+    double mx = 0.0;
+    bool bad = false, piv = false;
+    for (int i = 0; i < len; ++i) {
+        const int k = start + i;
+        const size_t ko = firk_off<S * M>(lane, i);
+        const double ti = mesh[k], h = mesh[k + 1] - ti;
+        double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
+#pragma unroll
+        for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
+        if (nest.on) {
+            firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
+            store_stages<M, S>(K, ko, Kk);
+        } else {
+            load_stages<M, S>(K, ko, Kk);
+        }
+        firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
+        firk_fold<M, S>(Phi, G, nest.on, mx, bad);
+    }
+    __syncthreads();
+    firk_bc_rows<M, S>(I, T, nest, sh, mesh, y, K, N, lane);
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+        const double a = fabs(sh.bcres[k]);
+        bad |= !(a <= 1.7976931348623157e308);
+        mx = fmax(mx, a);
+    }
+    const bool anybad = wave_any(bad);
+    mx = wave_max(mx);
+    return uniform(anybad ? NAN : mx);
 }
 
 // ------------------------------------------------------------------ full solve of one instance
@@ -1272,7 +1736,7 @@ __device__ inline void firk_extend(const double *y, double *K, int N, int lane) 
 // the transfer of the solution (the old quintic interpolant at the new nodes, stages as
 // extend_y sets them for a new problem), or halving with a zero restart when Newton or
 // the defect threshold failed.
-template <int M, int S, bool NEST, bool IR>
+template <int M, int S, bool NEST, bool IR, bool DIAG>
 __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, int b, Shared<M> &sh, int lane,
                                            double *scr, double *aux) {
     Inst<M> I;
@@ -1283,15 +1747,16 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
     FirkNest<M> nest = firk_nest_of<M>(B, b);
     nest.on = NEST;  // compile-time forms: the expanded kernels carry no inner-solve code,
     nest.irows = IR;  // and kernels for batches without interior rows no EvalSol code
-    const size_t cap = (size_t)B.cap;
-    double *dy = aux;                          // [cap][M]
-    double *dK = dy + cap * M;                 // [cap][S][M]
-    double *y0 = dK + cap * S * M;             // [cap][M]
-    double *K0 = y0 + cap * M;                 // [cap][S][M]
-    double *loc = K0 + cap * S * M;            // [cap][kFirkLoc]
+    // node areas [cap][M]; interval areas lane-interleaved
+    const size_t cap = (size_t)B.cap, icap = firk_pad(B.cap);
+    double *dy = aux;
+    double *y0 = dy + cap * M;
+    double *dK = y0 + cap * M;
+    double *K0 = dK + icap * S * M;
+    double *loc = K0 + icap * S * M;
     double *shat = as_global(B.shat + (size_t)b * B.cap);
     int cur = 0;
-    int N = B.N0[b];
+    int N = __builtin_amdgcn_readfirstlane(B.N0[b]);
     {
         const long long off = B.init_off[b];
         for (int k = lane; k <= N; k += WAVE) {
@@ -1312,7 +1777,7 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
         const double *mesh = bf.mesh[cur];
         double *y = bf.y_of(cur);
         double *mesh_o = bf.mesh[1 - cur], *y_o = bf.y_of(1 - cur);
-        FirkNewtonOut nl = firk_newton<M, S, IR>(B, I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, y0, K0);
+        FirkNewtonOut nl = firk_newton<M, S, IR, DIAG>(B, I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, y0, K0);
         iters += nl.iters;
         rn = nl.fn;
         rn_valid = true;
@@ -1332,7 +1797,8 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
         }
         if (info == BVP_RET_SUCCESS) {
             if (error_norm > B.abstol) {
-                const int Nn = mesh_select(mesh, N, shat, r1, r2, B.max_sub, mesh_o, lane, sh);
+                const int Nn =
+                    __builtin_amdgcn_readfirstlane(mesh_select(mesh, N, shat, r1, r2, B.max_sub, mesh_o, lane, sh));
                 if (Nn < 0) {
                     info = BVP_RET_FAILURE;
                 } else {
@@ -1341,7 +1807,7 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
                     // restart is the interpolated nodes with extend_y's stages
                     const double hs = (nest.on && Nn > N) ? (double)Nn / (double)N : 1.0;
                     for (int j = lane; j <= Nn; j += WAVE)
-                        firk_interp_at<M, S>(I, T, nest, mesh, y, K, N, mesh_o[j], y_o + (size_t)j * M, nullptr, hs);
+                        firk_interp_at<M, S, false>(I, T, nest, mesh, y, K, N, mesh_o[j], y_o + (size_t)j * M, nullptr, hs);
                     __syncthreads();
                     if (!nest.on) firk_extend<M, S>(y_o, K, Nn, lane);
                     cnt_tr += N + Nn;
@@ -1356,7 +1822,10 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
             } else {
                 half_mesh_into(mesh, N, mesh_o, lane);
                 for (int q = lane; q <= 2 * N * M + M - 1; q += WAVE) y_o[q] = 0.0;
-                for (int q = lane; q < 2 * N * S * M; q += WAVE) K[q] = 0.0;
+                firk_each<S * M>(2 * N, lane, [&](size_t o) {
+#pragma unroll
+                    for (int q = 0; q < S * M; ++q) K[o + (size_t)q * WAVE] = 0.0;
+                });
                 __syncthreads();
                 N = 2 * N;
                 cur = 1 - cur;
@@ -1368,9 +1837,7 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
         if (outer >= 64) { info = BVP_RET_FAILURE; break; }
     }
     if (!rn_valid) {
-        Rel<M> rel;
-        bool sing = false;
-        rn = firk_forward<M, S>(I, T, nest, sh, bf.mesh[cur], bf.y_of(cur), K, N, lane, scr, loc, rel, sing);
+        rn = firk_residual_max<M, S>(I, T, nest, sh, bf.mesh[cur], bf.y_of(cur), K, N, lane);
     }
     if (lane == 0) {
         B.err[b] = NAN;
@@ -1393,17 +1860,19 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
 // ------------------------------------------------------------------ kernels
 // Persistent FIRK solve: each wave pulls instances from the queue.  NEST: the nested form;
 // IR: the general kernels (STANDARD rows inside the span, the TrustRegion stage).
-template <int M, int S, bool NEST, bool IR>
+template <int M, int S, bool NEST, bool IR, bool DIAG>
 __device__ __forceinline__ void firk_solve_queue(const BatchDev &B) {
     __shared__ FirkShared<M> sh;
     const int lane = threadIdx.x;
-    const FirkTab &T = *reinterpret_cast<const FirkTab *>(B.firk_tab);
+    const FirkTab &T = firk_tab_of(B);
     double *scr = as_global(B.scratch + (size_t)blockIdx.x * B.scratch_per_slot);
     double *aux = as_global(B.aux + (size_t)blockIdx.x * B.aux_per_slot);
     for (;;) {
-        const int item = next_item<M>(B.counter, sh, lane);
+        // the item and its instance in scalar registers: loop bounds, the family and the
+        // parameters are then the same for all lanes
+        const int item = __builtin_amdgcn_readfirstlane(next_item<M>(B.counter, sh, lane));
         if (item >= B.n) break;
-        firk_solve_instance<M, S, NEST, IR>(B, T, B.order[item], sh, lane, scr, aux);
+        firk_solve_instance<M, S, NEST, IR, DIAG>(B, T, __builtin_amdgcn_readfirstlane(B.order[item]), sh, lane, scr, aux);
     }
 }
 
@@ -1411,11 +1880,11 @@ __device__ __forceinline__ void firk_solve_queue(const BatchDev &B) {
 // (few spills) and two waves per SIMD (twice the waves to hide latency, more spills).
 template <int M, int S, bool NEST, bool IR = false>
 __global__ __launch_bounds__(64, 1) void k_firk_solve(BatchDev B) {
-    firk_solve_queue<M, S, NEST, IR>(B);
+    firk_solve_queue<M, S, NEST, IR, kFirkDiag<M, S>>(B);
 }
 template <int M, int S, bool NEST>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_firk_solve_w2(BatchDev B) {
-    firk_solve_queue<M, S, NEST, false>(B);
+    firk_solve_queue<M, S, NEST, false, false>(B);
 }
 
 // Component kernels at the packed state (mesh, guess and the packed stages init_K; the
@@ -1429,7 +1898,7 @@ template <int M, int S>
 __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
     __shared__ FirkShared<M> sh;
     const int lane = threadIdx.x;
-    const FirkTab &T = *reinterpret_cast<const FirkTab *>(B.firk_tab);
+    const FirkTab &T = firk_tab_of(B);
     double *scr = as_global(B.scratch + (size_t)blockIdx.x * B.scratch_per_slot);
     double *aux = as_global(B.aux + (size_t)blockIdx.x * B.aux_per_slot);
     const size_t cap = (size_t)B.cap;
@@ -1444,11 +1913,21 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
         const long long ioff = off - b;  // interval offset
         const double *mesh = as_global(B.init_mesh + off);
         const double *y = as_global(B.init_y + off * M);
-        double *dy = aux, *dK = dy + cap * M, *loc = dK + cap * S * M;
+        const size_t icap = firk_pad(B.cap);
+        double *dy = aux, *dK = dy + 2 * cap * M, *K = dK + icap * S * M, *loc = K + icap * S * M;
         const FirkNest<M> nest = firk_nest_of<M>(B, b);
-        // the stage state: the packed input, or (nested) the inner solves' stages in the
-        // slot's dK area, which the nested correction does not use
-        double *K = nest.on ? dK : const_cast<double *>(as_global(B.init_K + ioff * S * M));
+        double *sl = firk_slot<M, S>(sh, lane);
+        // the stage state in the slot: the packed input lane-interleaved, or (nested) the
+        // inner solves' stages
+        if (!nest.on) {
+            const double *Ki = as_global(B.init_K + ioff * S * M);
+            int P, start, len;
+            chunk_of(N, lane, P, start, len);
+            for (int i = 0; i < len; ++i)
+                for (int q = 0; q < S * M; ++q)
+                    K[firk_off<S * M>(lane, i) + (size_t)q * WAVE] = Ki[(size_t)(start + i) * S * M + q];
+            __syncthreads();
+        }
         const size_t xo = nest.on ? (size_t)M * off : (size_t)M * ((size_t)(S + 1) * ioff + b);  // slot offset
         const int rowlen = nest.on ? M : (S + 1) * M;  // residual entries per interval
         if (op == OP_RESIDUAL) {
@@ -1460,14 +1939,16 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
                 nbca = M;
             int P, start, len;
             chunk_of(N, lane, P, start, len);
-            for (int k = start; k < start + len; ++k) {
+            bool piv = false;
+            for (int i = 0; i < len; ++i) {
+                const int k = start + i;
                 const double ti = mesh[k], h = mesh[k + 1] - ti;
                 double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
                 for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
-                if (nest.on) firk_inner<M, S>(I, T, nest, ti, h, yi, Kk);
-                else load_stages<M, S>(K, k, Kk);
-                firk_interval<M, S, false>(I, T, ti, h, yi, yj, Kk, G, Phi, J);
+                if (nest.on) firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
+                else load_stages<M, S>(K, firk_off<S * M>(lane, i), Kk);
+                firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
                 double *o = out + nbca + (size_t)k * rowlen;
 #pragma unroll
                 for (int c = 0; c < M; ++c) o[c] = Phi[c];
@@ -1483,7 +1964,7 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
                 int ia = 0, ib = 0;
                 for (int k = 0; k < M; ++k) {
                     const BcLoc L = bc_locate<M>(I, k, mesh, N);
-                    const double v = firk_bc_row<M, S>(I, T, nest, mesh, y, K, nullptr, nullptr, 0.0, k, L);
+                    const double v = firk_bc_row<M, S>(I, T, nest, mesh, y, K, nullptr, nullptr, 0.0, k, L, N);
                     if (I.bc_kind == BVP_BC_TWO_POINT && sel<M>(I.bct, k) != I.t0)
                         out[nbca + (size_t)N * rowlen + (ib++)] = v;
                     else
@@ -1492,9 +1973,12 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
             }
         } else if (op == OP_NEWTON_STEP) {
             Rel<M> rel;
-            bool sing = false;
-            firk_forward<M, S>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing);
-            const bool ok = !sing && firk_correction<M, S>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, dy, dK);
+            bool sing = false, sticky = false;
+            firk_forward<M, S, false>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing, sticky);
+            const bool ok = !sing && firk_tree<M, S, true>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel);
+            if (ok)
+                firk_back<M, S, false, FIRK_STORE>(I, T, nest, sh, mesh, const_cast<double *>(y), K, N, lane, scr, loc, dy,
+                                                   dK);
             double *out = B.out0 + xo;
             for (int q = lane; q < (N + 1) * M; q += WAVE) {
                 const int i = q / M, c = q % M;
@@ -1502,18 +1986,23 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
             }
             for (int q = lane; q < (nest.on ? 0 : N * S * M); q += WAVE) {
                 const int i = q / (S * M), rc = q % (S * M);
-                out[(size_t)i * (S + 1) * M + M + rc] = ok ? dK[q] : NAN;
+                out[(size_t)i * (S + 1) * M + M + rc] =
+                    ok ? dK[firk_off<S * M>(N, i, true) + (size_t)rc * WAVE] : NAN;
             }
         } else if (op == OP_DEFECT) {
             if (nest.on) {
                 // the stages from the inner solves, as defect_estimate! solves them
                 // (FIRK/adaptivity.jl:465-517)
-                for (int k = lane; k < N; k += WAVE) {
+                int P, start, len;
+                chunk_of(N, lane, P, start, len);
+                bool piv = false;
+                for (int i = 0; i < len; ++i) {
+                    const int k = start + i;
                     double yi[M], Kk[S][M];
 #pragma unroll
                     for (int c = 0; c < M; ++c) yi[c] = y[(size_t)k * M + c];
-                    firk_inner<M, S>(I, T, nest, mesh[k], mesh[k + 1] - mesh[k], yi, Kk);
-                    store_stages<M, S>(K, k, Kk);
+                    firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, mesh[k], mesh[k + 1] - mesh[k], yi, Kk, piv);
+                    store_stages<M, S>(K, firk_off<S * M>(lane, i), Kk);
                 }
                 __syncthreads();
             }
@@ -1532,7 +2021,7 @@ __global__ __launch_bounds__(256) void k_firk_interp(BatchDev B, const int *qins
                                                      double *duo, long long nq) {
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
     if (q >= nq) return;
-    const FirkTab &T = *reinterpret_cast<const FirkTab *>(B.firk_tab);
+    const FirkTab &T = firk_tab_of(B);
     const int b = qinst[q];
     Inst<M> I;
     load_inst<M>(B, b, I);
@@ -1545,7 +2034,7 @@ __global__ __launch_bounds__(256) void k_firk_interp(BatchDev B, const int *qins
     const FirkNest<M> nest = firk_nest_of<M>(B, b);
     const double *K = nest.on ? nullptr : as_global(B.init_K + ioff * S * M);
     double u[M], du[M];
-    firk_interp_at<M, S>(I, T, nest, mesh, y, K, N, t, u, du);
+    firk_interp_at<M, S, true>(I, T, nest, mesh, y, K, N, t, u, du);
 #pragma unroll
     for (int c = 0; c < M; ++c) {
         uo[q * M + c] = u[c];
@@ -1562,7 +2051,8 @@ __global__ __launch_bounds__(256) void k_firk_gather(BatchDev B, const long long
     const int N = B.N_final[b];
     const double *K = firk_stages_of<M, S>(B, b);
     const long long o = out_off[b] * S * M;
-    for (int q = threadIdx.x; q < N * S * M; q += blockDim.x) out[o + q] = K[q];
+    for (int q = threadIdx.x; q < N * S * M; q += blockDim.x)
+        out[o + q] = K[firk_off<S * M>(N, q / (S * M), true) + (size_t)(q % (S * M)) * WAVE];
 }
 
 // The two-waves-per-SIMD register variant where the compiler reaches that occupancy

@@ -302,6 +302,77 @@ __device__ inline void f_eval(int fam, const Params<M> &P, double t, const T *y,
     }
 }
 
+// f and its Jacobian J[a][c] = df_a/dy_c; f is the arithmetic of f_eval, J what its dual
+// numbers carry.
+template <int M>
+__device__ __forceinline__ void f_jac(int fam, const Params<M> &P, double t, const double *y, double *f,
+                                      double (&J)[M][M]) {
+    if constexpr (M == 2) {
+        if (fam == BVP_FAMILY_BRATU) {
+            const double e = exp(y[0]);
+            f[0] = y[1];
+            f[1] = -P.p[0] * e;
+            J[0][0] = 0.0; J[0][1] = 1.0;
+            J[1][0] = -P.p[0] * e; J[1][1] = 0.0;
+            return;
+        }
+        if (fam == BVP_FAMILY_PENDULUM) {
+            double s, c;
+            sincos(y[0], &s, &c);
+            f[0] = y[1];
+            f[1] = -P.p[0] * s;
+            J[0][0] = 0.0; J[0][1] = 1.0;
+            J[1][0] = -P.p[0] * c; J[1][1] = 0.0;
+            return;
+        }
+        if (fam == BVP_FAMILY_SINGPERT) {
+            f[0] = y[1];
+            f[1] = (y[0] - t * y[1]) / P.p[0];
+            J[0][0] = 0.0; J[0][1] = 1.0;
+            J[1][0] = 1.0 / P.p[0]; J[1][1] = -t / P.p[0];
+            return;
+        }
+        if (fam == BVP_FAMILY_TURNING) {
+            f_eval<M, double>(fam, P, t, y, f);
+            J[0][0] = 0.0; J[0][1] = 1.0;
+            J[1][0] = 0.0; J[1][1] = -t / P.p[0];
+            return;
+        }
+    }
+    if constexpr (M == 1) {
+        if (fam == BVP_FAMILY_SCALAR_TU) {
+            f[0] = t * y[0];
+            J[0][0] = t;
+            return;
+        }
+    }
+    if constexpr (M == 6) {
+        if (fam == BVP_FAMILY_SWIRL) {
+            f_eval<M, double>(fam, P, t, y, f);
+#pragma unroll
+            for (int a = 0; a < M; ++a)
+#pragma unroll
+                for (int c = 0; c < M; ++c) J[a][c] = 0.0;
+            J[0][1] = J[2][3] = J[3][4] = J[4][5] = 1.0;
+            J[1][0] = y[3] / P.p[0]; J[1][1] = -y[2] / P.p[0]; J[1][2] = -y[1] / P.p[0]; J[1][3] = y[0] / P.p[0];
+            J[5][0] = -y[1] / P.p[0]; J[5][1] = -y[0] / P.p[0]; J[5][2] = -y[5] / P.p[0]; J[5][5] = -y[2] / P.p[0];
+            return;
+        }
+    }
+    // BVP_FAMILY_LINEAR_TANH
+    const double c = P.p[0];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        double acc = P.p[1 + i * M] * y[0];
+#pragma unroll
+        for (int j = 1; j < M; ++j) acc = acc + P.p[1 + i * M + j] * y[j];
+        const double th = tanh(y[i]);
+        f[i] = acc + c * th;
+#pragma unroll
+        for (int j = 0; j < M; ++j) J[i][j] = P.p[1 + i * M + j] + (i == j ? c * (1.0 - th * th) : 0.0);
+    }
+}
+
 template <int M>
 __host__ __device__ inline bool family_supported(int fam) {
     if (fam == BVP_FAMILY_LINEAR_TANH) return true;

@@ -87,7 +87,7 @@ struct BatchDev {
     size_t ge_per_slot;
 
     // FIRK methods (expanded form): the tableau (a FirkTab in device memory), the stage
-    // values of every instance [n][cap][s][M], and for the component kernels the packed
+    // values of every instance (cap + 64 intervals each, lane-interleaved), and for the component kernels the packed
     // input stages [sum N][s][M] (interval offset = init_off[b] - b)
     const void *firk_tab;
     double *stK;
@@ -144,7 +144,8 @@ hipError_t firk_launch_gather(const BatchDev &B, int S, const long long *out_off
 int firk_blocks_per_cu(int M, int S, int variant, int nested);  // resident solve waves per CU
 // doubles per slot of the FIRK work area for node capacity cap
 inline size_t firk_aux_doubles(int cap, int M, int S) {
-    return (size_t)cap * (2 * M + 2 * S * M + S * M * (M + 1));
+    // node areas of cap nodes, lane-interleaved interval areas of cap + 64 intervals
+    return (size_t)cap * (2 * M) + ((size_t)cap + 64) * (2 * S * M + S * M * (M + 1));
 }
 
 hipError_t launch_copy_probe(const double *src, double *dst, size_t n, hipStream_t s);

@@ -399,7 +399,8 @@ template <int M> constexpr int kRelFields = 2 * M * M + M;
 // Eliminate the shared node b of  L: E1 dy_a + F1 dy_b = g1  and  S dy_b + R dy_c = r
 // by Gaussian elimination with partial pivoting on the stacked 2M x M column
 // block [F1; S].  Produces the relation for (a, c) and the back-substitution
-// rows of b.
+// rows of b.  (All unrolled loops have constant trip counts with a condition inside:
+// triangular bounds leave the arrays in private memory, with a store for every update.)
 template <int M>
 __device__ inline void eliminate(const Rel<M> &L, const double (&S)[M][M], const double (&R)[M][M],
                                  const double *r, Rel<M> &out, Back<M> &bk) {
@@ -421,13 +422,15 @@ __device__ inline void eliminate(const Rel<M> &L, const double (&S)[M][M], const
         int p = j;
         double best = fabs(A[j][j]);
 #pragma unroll
-        for (int i = j + 1; i < M2; ++i) {
+        for (int i = 0; i < M2; ++i) {
+            if (i <= j) continue;
             const double v = fabs(A[i][j]);
             if (v > best) { best = v; p = i; }
         }
         // swap rows j and p by selects (keeps the arrays in registers)
 #pragma unroll
-        for (int i = j + 1; i < M2; ++i) {
+        for (int i = 0; i < M2; ++i) {
+            if (i <= j) continue;
             const bool sw = (i == p);
 #pragma unroll
             for (int c = 0; c < M; ++c) {
@@ -442,10 +445,12 @@ __device__ inline void eliminate(const Rel<M> &L, const double (&S)[M][M], const
         }
         const double inv = 1.0 / A[j][j];
 #pragma unroll
-        for (int i = j + 1; i < M2; ++i) {
+        for (int i = 0; i < M2; ++i) {
+            if (i <= j) continue;
             const double m = A[i][j] * inv;
 #pragma unroll
-            for (int c = j + 1; c < M; ++c) A[i][c] -= m * A[j][c];
+            for (int c = 0; c < M; ++c)
+                if (c > j) A[i][c] -= m * A[j][c];
 #pragma unroll
             for (int c = 0; c < M; ++c) { B1[i][c] -= m * B1[j][c]; B2[i][c] -= m * B2[j][c]; }
             q[i] -= m * q[j];
@@ -453,19 +458,22 @@ __device__ inline void eliminate(const Rel<M> &L, const double (&S)[M][M], const
     }
     // back-substitution rows: solve U [X Z h] = [B1 B2 q] (top M rows)
 #pragma unroll
-    for (int i = M - 1; i >= 0; --i) {
+    for (int ii = 0; ii < M; ++ii) {
+        const int i = M - 1 - ii;
         const double inv = 1.0 / A[i][i];
 #pragma unroll
         for (int c = 0; c < M; ++c) {
             double x = B1[i][c], z = B2[i][c];
 #pragma unroll
-            for (int k = i + 1; k < M; ++k) { x -= A[i][k] * bk.X[k][c]; z -= A[i][k] * bk.Z[k][c]; }
+            for (int k = 0; k < M; ++k)
+                if (k > i) { x -= A[i][k] * bk.X[k][c]; z -= A[i][k] * bk.Z[k][c]; }
             bk.X[i][c] = x * inv;
             bk.Z[i][c] = z * inv;
         }
         double hh = q[i];
 #pragma unroll
-        for (int k = i + 1; k < M; ++k) hh -= A[i][k] * bk.h[k];
+        for (int k = 0; k < M; ++k)
+            if (k > i) hh -= A[i][k] * bk.h[k];
         bk.h[i] = hh * inv;
     }
 #pragma unroll
@@ -581,9 +589,11 @@ __device__ inline bool dense_solve(double (&A)[NN][NN], double (&b)[NN]) {
         int p = j;
         double best = fabs(A[j][j]);
 #pragma unroll
-        for (int i = j + 1; i < NN; ++i) if (fabs(A[i][j]) > best) { best = fabs(A[i][j]); p = i; }
+        for (int i = 0; i < NN; ++i)
+            if (i > j && fabs(A[i][j]) > best) { best = fabs(A[i][j]); p = i; }
 #pragma unroll
-        for (int i = j + 1; i < NN; ++i) {
+        for (int i = 0; i < NN; ++i) {
+            if (i <= j) continue;
             const bool sw = (i == p);
 #pragma unroll
             for (int c = 0; c < NN; ++c) {
@@ -598,18 +608,22 @@ __device__ inline bool dense_solve(double (&A)[NN][NN], double (&b)[NN]) {
         if (A[j][j] == 0.0) return false;
         const double inv = 1.0 / A[j][j];
 #pragma unroll
-        for (int i = j + 1; i < NN; ++i) {
+        for (int i = 0; i < NN; ++i) {
+            if (i <= j) continue;
             const double m = A[i][j] * inv;
 #pragma unroll
-            for (int c = j + 1; c < NN; ++c) A[i][c] -= m * A[j][c];
+            for (int c = 0; c < NN; ++c)
+                if (c > j) A[i][c] -= m * A[j][c];
             b[i] -= m * b[j];
         }
     }
 #pragma unroll
-    for (int i = NN - 1; i >= 0; --i) {
+    for (int ii = 0; ii < NN; ++ii) {
+        const int i = NN - 1 - ii;
         double v = b[i];
 #pragma unroll
-        for (int c = i + 1; c < NN; ++c) v -= A[i][c] * b[c];
+        for (int c = 0; c < NN; ++c)
+            if (c > i) v -= A[i][c] * b[c];
         b[i] = v / A[i][i];
     }
     return true;
@@ -620,6 +634,8 @@ template <int M> struct Inst {
     int fam;
     int minc;  // chunk_of's minimum intervals per lane
     Params<M> P;
+    const double *params;  // where P was read from, and how many
+    int pcnt;
     int bc_kind;
     double bct[M], bcv[M];
     int bcc[M];
@@ -631,6 +647,8 @@ __device__ inline void load_inst(const BatchDev &B, int b, Inst<M> &I) {
     I.fam = B.family[b];
     I.minc = B.min_chunk > 0 ? B.min_chunk : 1;
     const int po = B.param_off[b], pn = B.param_cnt[b];
+    I.params = B.params + po;
+    I.pcnt = pn;
 #pragma unroll
     for (int k = 0; k < Params<M>::MAXP; ++k) I.P.p[k] = k < pn ? B.params[po + k] : 0.0;
     I.bc_kind = B.bc_kind[b];
