@@ -1355,7 +1355,7 @@ int bvp_mlp_train(bvp_mlp *m, int64_t n, const float *x, const float *y, const b
     int rc;
     if ((rc = dalloc(ctx, A, dx, (size_t)n * mlp::NIN)) || (rc = dalloc(ctx, A, dy, (size_t)n * mlp::NOUT)) ||
         (rc = dalloc(ctx, A, dpart, (size_t)tiles * mlp::NSLOT)) || (rc = dalloc(ctx, A, dloss, (size_t)total)) ||
-        (rc = upload(ctx, A, dperm, perm)) || (rc = dalloc(ctx, A, dstep, 1)))
+        (rc = upload(ctx, A, dperm, perm)) || (rc = dalloc(ctx, A, dstep, 2)))
         return rc;
     HIP_TRY(ctx, hipMemcpyAsync(dx, x, sizeof(float) * n * mlp::NIN, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(dy, y, sizeof(float) * n * mlp::NOUT, hipMemcpyHostToDevice, ctx->stream));

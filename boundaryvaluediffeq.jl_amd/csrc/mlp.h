@@ -59,7 +59,7 @@ struct TrainDev {
     int steps_per_epoch;
     int total_steps;
     const unsigned long long *perm; // per epoch: (a, c) of the index permutation j -> (a j + c) mod n
-    int *step;                      // device step counter
+    int *step;                      // device step counter; step[1]: the step k_adam works on
     float *partial;                 // [batch_tiles][NSLOT]
     float *loss;                    // [steps of this call], indexed by step - step0
     int step0;                      // first step of this call

@@ -46,27 +46,25 @@ struct __align__(16) Tile {
     int valid[T];
 };
 
-// acc[rt][ct] (rows 16rt.., columns 64*wave + 16ct..) = A (LDS, T x H) times the
-// matrix whose column c is row c of G (global BF16, H x H, row-major).
-__device__ inline void gemm_tile(const uint16_t *A, const uint16_t *G, int wave, int lane, f4 acc[4][4]) {
+// Training runs a tile with 16 waves: TW threads, four waves per SIMD.
+constexpr int TW = 1024;
+
+// acc[rt] (rows 16rt.., columns 16*wave..) = A (LDS, T x H) times the matrix whose column
+// c is row c of G (global BF16, H x H, row-major).  All of the wave's operands of G are
+// loaded at once, before the products.
+__device__ inline void gemm_tile(const uint16_t *A, const uint16_t *G, int wave, int lane, f4 acc[4]) {
     const int i = lane & 15, g = lane >> 4;
+    bf8 b[H / 32];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int ks = 0; ks < H / 32; ++ks) b[ks] = *(const bf8 *)(G + (size_t)(16 * wave + i) * H + 32 * ks + 8 * g);
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k0 = 0; k0 < H; k0 += 32) {
-        bf8 a[4], b[4];
+    for (int rt = 0; rt < 4; ++rt) acc[rt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) a[rt] = *(const bf8 *)(A + (size_t)(16 * rt + i) * HP + k0 + 8 * g);
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) b[ct] = *(const bf8 *)(G + (size_t)(64 * wave + 16 * ct + i) * H + k0 + 8 * g);
+    for (int ks = 0; ks < H / 32; ++ks)
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < 4; ++ct)
-                acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], b[ct], acc[rt][ct], 0, 0, 0);
-    }
+            acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                *(const bf8 *)(A + (size_t)(16 * rt + i) * HP + 32 * ks + 8 * g), b[ks], acc[rt], 0, 0, 0);
 }
 
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
@@ -81,61 +79,45 @@ __device__ inline bf8 gather8(const uint16_t *p, int stride) {
     return __builtin_bit_cast(bf8, r);
 }
 
-// dW[k][n] = sum_p Hin[p][k] dz[p][n] for this tile, written output-major to
-// part[n*H + k] (four consecutive k per lane: one 16-byte store); wave w owns
-// rows k in [64w, 64w+64).
+// dW[k][n] = sum_p Hin[p][k] dz[p][n] for this tile, written input-major (the parameters'
+// order) to part[k*H + n], four consecutive n per lane: one 16-byte store; a wave owns a
+// 64 x 64 block.
 __device__ inline void wgrad_tile(const uint16_t *Hin, const uint16_t *dz, float *part, int wave, int lane) {
-    const int i = lane & 15, g = lane >> 4;
+    const int i = lane & 15, g = lane >> 4, n0 = 64 * (wave >> 2), k0 = 64 * (wave & 3);
     bf8 a[4][2];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) a[rt][ks] = gather8(Hin + (size_t)(32 * ks + 8 * g) * HP + 64 * wave + 16 * rt + i, HP);
-    for (int np = 0; np < 4; ++np) {
-        f4 acc[4][4];
+        for (int ks = 0; ks < 2; ++ks) a[rt][ks] = gather8(dz + (size_t)(32 * ks + 8 * g) * HP + n0 + 16 * rt + i, HP);
+#pragma unroll 2
+    for (int ct = 0; ct < 4; ++ct) {
+        f4 acc[4];
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int rt = 0; rt < 4; ++rt) acc[rt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            bf8 b[4];
-#pragma unroll
-            for (int ct = 0; ct < 4; ++ct) b[ct] = gather8(dz + (size_t)(32 * ks + 8 * g) * HP + 64 * np + 16 * ct + i, HP);
+            const bf8 b = gather8(Hin + (size_t)(32 * ks + 8 * g) * HP + k0 + 16 * ct + i, HP);
 #pragma unroll
             for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-                for (int ct = 0; ct < 4; ++ct)
-                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt][ks], b[ct], acc[rt][ct], 0, 0, 0);
+                acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt][ks], b, acc[rt], 0, 0, 0);
         }
+        f4 *dst = (f4 *)(part + (size_t)(k0 + 16 * ct + i) * H + n0 + 4 * g);
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            f4 *dst = (f4 *)(part + (size_t)(64 * np + 16 * ct + i) * H + 64 * wave + 4 * g);
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt) dst[4 * rt] = acc[rt][ct];
-        }
+        for (int rt = 0; rt < 4; ++rt) dst[4 * rt] = acc[rt];
     }
-}
-
-// Index in the parameter vector of slot entry j (the hidden matrices are
-// stored output-major in the per-tile slots, input-major in the parameters).
-__device__ inline int slot_param(int j) {
-    if (j >= OW2 && j < OW2 + H * H) return OW2 + ((j - OW2) % H) * H + (j - OW2) / H;
-    if (j >= OW3 && j < OW3 + H * H) return OW3 + ((j - OW3) % H) * H + (j - OW3) / H;
-    return j;
 }
 
 // Forward pass of the tile (S.x filled): hidden activations into S.h, output into S.out.
 __device__ void forward_tile(Tile &S, const Net &net, int tid) {
     const int wave = tid >> 6, lane = tid & 63;
-    {  // layer 1 (4 -> 256): thread tid owns column n = tid
-        const int n = tid;
+    {  // layer 1 (4 -> 256): a thread owns column n and 16 points
+        const int n = tid & (H - 1), p0 = (tid / H) * 16;
         float w[NIN];
 #pragma unroll
         for (int i = 0; i < NIN; ++i) w[i] = net.q[OW1 + i * H + n];
         const float b = net.q[OB1 + n];
 #pragma unroll 8
-        for (int p = 0; p < T; ++p) {
+        for (int p = p0; p < p0 + 16; ++p) {
             float z = b;
 #pragma unroll
             for (int i = 0; i < NIN; ++i) z += S.x[p][i] * w[i];
@@ -146,33 +128,31 @@ __device__ void forward_tile(Tile &S, const Net &net, int tid) {
     const int i = lane & 15, g = lane >> 4;
 #pragma unroll 1
     for (int l = 0; l < 2; ++l) {  // layers 2 and 3 (256 -> 256) on the matrix cores
-        f4 acc[4][4];
+        f4 acc[4];
+        const int n = 16 * wave + i;
+        const float bn = net.q[(l == 0 ? OB2 : OB3) + n];
         gemm_tile(&S.h[l][0][0], l == 0 ? net.w2f : net.w3f, wave, lane, acc);
-        const float *bias = net.q + (l == 0 ? OB2 : OB3);
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct) {
-                const int n = 64 * wave + 16 * ct + i;
-                const float bn = bias[n];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) S.h[l + 1][16 * rt + 4 * g + j][n] = f2bf(tanh_f(acc[rt][ct][j] + bn));
-            }
+            for (int j = 0; j < 4; ++j) S.h[l + 1][16 * rt + 4 * g + j][n] = f2bf(tanh_f(acc[rt][j] + bn));
         __syncthreads();
     }
-    {  // output layer (256 -> 2): four threads per point, 64 inputs each
-        const int p = tid >> 2, part = tid & 3;
+    {  // output layer (256 -> 2): sixteen threads per point, every sixteenth input each
+        const int p = tid >> 4, part = tid & 15;
         float o0 = 0.f, o1 = 0.f;
-#pragma unroll 16
-        for (int k = 64 * part; k < 64 * part + 64; ++k) {
+#pragma unroll
+        for (int it = 0; it < H / 16; ++it) {
+            const int k = 16 * it + part;
             const float hk = bf2f(S.h[2][p][k]);
             o0 += hk * net.q[OW4 + 2 * k];
             o1 += hk * net.q[OW4 + 2 * k + 1];
         }
-        o0 += __shfl_xor(o0, 1);
-        o1 += __shfl_xor(o1, 1);
-        o0 += __shfl_xor(o0, 2);
-        o1 += __shfl_xor(o1, 2);
+#pragma unroll
+        for (int m = 1; m < 16; m *= 2) {
+            o0 += __shfl_xor(o0, m);
+            o1 += __shfl_xor(o1, m);
+        }
         if (part == 0) {
             S.out[p][0] = o0 + net.q[OB4];
             S.out[p][1] = o1 + net.q[OB4 + 1];
@@ -182,89 +162,101 @@ __device__ void forward_tile(Tile &S, const Net &net, int tid) {
 }
 
 // Backward pass of the tile after forward_tile; inv_b = 1 / (points in the step).
-// Writes the tile's gradient and loss into part[NSLOT].
+// Writes the tile's gradient and loss into part[NSLOT].  Sums over the tile's points: four
+// threads per unit, every fourth point each (pt = 4 it + sub), combined by shuffles.
 __device__ void backward_tile(Tile &S, const Net &net, int tid, float inv_b, float *part) {
     const int wave = tid >> 6, lane = tid & 63;
     const int i = lane & 15, g = lane >> 4;
-    // dL/dout and the loss (L = sum 0.5 (out - y)^2 / B)
+    const int unit = tid >> 2, sub = tid & 3;
+    auto sum4 = [](float v) {
+        v += __shfl_xor(v, 1);
+        return v + __shfl_xor(v, 2);
+    };
+    // dL/dout and the loss (L = sum 0.5 (out - y)^2 / B): one wave, a point per lane
     if (tid < T) {
         const int p = tid;
-        float l = 0.f;
+        float l = 0.f, d[NOUT];
 #pragma unroll
         for (int o = 0; o < NOUT; ++o) {
-            const float d = S.valid[p] ? (S.out[p][o] - S.tgt[p][o]) : 0.f;
-            l += 0.5f * d * d;
-            S.out[p][o] = d * inv_b;
+            d[o] = S.valid[p] ? (S.out[p][o] - S.tgt[p][o]) : 0.f;
+            l += 0.5f * d[o] * d[o];
+            d[o] *= inv_b;
+            S.out[p][o] = d[o];
         }
-        S.lossv[p] = l * inv_b;
+        l *= inv_b;
+#pragma unroll
+        for (int m = 1; m < T; m *= 2) {
+            l += __shfl_xor(l, m);
+#pragma unroll
+            for (int o = 0; o < NOUT; ++o) d[o] += __shfl_xor(d[o], m);
+        }
+        if (p == 0) {
+            part[NPARAM] = l;
+#pragma unroll
+            for (int o = 0; o < NOUT; ++o) part[OB4 + o] = d[o];
+        }
     }
     __syncthreads();
-    {  // output layer: dW4, db4, and dz3 = (dout W4^T) * (1 - h3^2); thread tid owns hidden unit k
-        const int k = tid;
-        const float w0 = net.q[OW4 + 2 * k], w1 = net.q[OW4 + 2 * k + 1];
+    {  // output layer: dW4, and dz3 = (dout W4^T) * (1 - h3^2)
+        const float w0 = net.q[OW4 + 2 * unit], w1 = net.q[OW4 + 2 * unit + 1];
         float g0 = 0.f, g1 = 0.f;
-        for (int p = 0; p < T; ++p) {
-            const float hk = bf2f(S.h[2][p][k]);
+#pragma unroll 8
+        for (int it = 0; it < T / 4; ++it) {
+            const int p = 4 * it + sub;
+            const float hk = bf2f(S.h[2][p][unit]);
             const float d0 = S.out[p][0], d1 = S.out[p][1];
             g0 += hk * d0;
             g1 += hk * d1;
-            S.dz[p][k] = f2bf((d0 * w0 + d1 * w1) * (1.f - hk * hk));
+            S.dz[p][unit] = f2bf((d0 * w0 + d1 * w1) * (1.f - hk * hk));
         }
-        part[OW4 + 2 * k] = g0;
-        part[OW4 + 2 * k + 1] = g1;
-        if (tid < NOUT) {
-            float s = 0.f;
-            for (int p = 0; p < T; ++p) s += S.out[p][tid];
-            part[OB4 + tid] = s;
-        }
-        if (tid == 0) {
-            float s = 0.f;
-            for (int p = 0; p < T; ++p) s += S.lossv[p];
-            part[NPARAM] = s;
-        }
+        g0 = sum4(g0);
+        g1 = sum4(g1);
+        if (sub < NOUT) part[OW4 + 2 * unit + sub] = sub == 0 ? g0 : g1;
     }
     __syncthreads();
 #pragma unroll 1
     for (int l = 1; l >= 0; --l) {  // hidden layer l + 2 (weights W3 for l = 1, W2 for l = 0)
-        const uint16_t *hin = &S.h[l][0][0];
-        wgrad_tile(hin, &S.dz[0][0], part + (l == 1 ? OW3 : OW2), wave, lane);
+        wgrad_tile(&S.h[l][0][0], &S.dz[0][0], part + (l == 1 ? OW3 : OW2), wave, lane);
         {
-            const int n = tid;
             float s = 0.f;
-            for (int p = 0; p < T; ++p) s += bf2f(S.dz[p][n]);
-            part[(l == 1 ? OB3 : OB2) + n] = s;
+#pragma unroll
+            for (int it = 0; it < T / 4; ++it) s += bf2f(S.dz[4 * it + sub][unit]);
+            s = sum4(s);
+            if (sub == 0) part[(l == 1 ? OB3 : OB2) + unit] = s;
         }
-        f4 acc[4][4];
+        f4 acc[4];
         gemm_tile(&S.dz[0][0], l == 1 ? net.w3b : net.w2b, wave, lane, acc);
         __syncthreads();
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct) {
-                const int k = 64 * wave + 16 * ct + i;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int p = 16 * rt + 4 * g + j;
-                    const float hk = bf2f(S.h[l][p][k]);
-                    S.dz[p][k] = f2bf(acc[rt][ct][j] * (1.f - hk * hk));
-                }
+            for (int j = 0; j < 4; ++j) {
+                const int p = 16 * rt + 4 * g + j, k = 16 * wave + i;
+                const float hk = bf2f(S.h[l][p][k]);
+                S.dz[p][k] = f2bf(acc[rt][j] * (1.f - hk * hk));
             }
         __syncthreads();
     }
     {  // input layer: dW1, db1
-        const int n = tid;
         float gw[NIN] = {0.f, 0.f, 0.f, 0.f}, gb = 0.f;
-        for (int p = 0; p < T; ++p) {
-            const float d = bf2f(S.dz[p][n]);
+#pragma unroll 8
+        for (int it = 0; it < T / 4; ++it) {
+            const int p = 4 * it + sub;
+            const float d = bf2f(S.dz[p][unit]);
             gb += d;
 #pragma unroll
             for (int q = 0; q < NIN; ++q) gw[q] += S.x[p][q] * d;
         }
 #pragma unroll
-        for (int q = 0; q < NIN; ++q) part[OW1 + q * H + n] = gw[q];
-        part[OB1 + n] = gb;
+        for (int q = 0; q < NIN; ++q) gw[q] = sum4(gw[q]);
+        gb = sum4(gb);
+#pragma unroll
+        for (int q = 0; q < NIN; ++q)
+            if (sub == q) part[OW1 + q * H + unit] = gw[q];
+        if (sub == 0) part[OB1 + unit] = gb;
     }
 }
+static_assert(NIN == 4 && TW == 4 * H && TW == 16 * T, "the thread splits of a training tile");
 
 __device__ inline void load_point(Tile &S, const Net &net, int p, bool valid, const float *xr, const float *yr) {
 #pragma unroll
@@ -276,10 +268,11 @@ __device__ inline void load_point(Tile &S, const Net &net, int p, bool valid, co
 }
 
 // ------------------------------------------------------------------ kernels
-__global__ __launch_bounds__(256) void k_train_tile(Net net, TrainDev td) {
+__global__ __launch_bounds__(TW) void k_train_tile(Net net, TrainDev td) {
     __shared__ Tile S;
     const int tid = threadIdx.x;
     const int step = td.step[0];
+    if (blockIdx.x == 0 && tid == 0) td.step[1] = step;  // for k_adam
     const int epoch = step / td.steps_per_epoch, sin = step % td.steps_per_epoch;
     const unsigned long long a = td.perm[2 * epoch], c = td.perm[2 * epoch + 1];
     const long long bsz = (long long)td.batch_tiles * T;
@@ -293,7 +286,7 @@ __global__ __launch_bounds__(256) void k_train_tile(Net net, TrainDev td) {
     backward_tile(S, net, tid, 1.0f / (float)bsz, td.partial + (size_t)blockIdx.x * NSLOT);
 }
 
-__global__ __launch_bounds__(256) void k_grad_tile(Net net, const float *x, const float *y, int n, float *partial) {
+__global__ __launch_bounds__(TW) void k_grad_tile(Net net, const float *x, const float *y, int n, float *partial) {
     __shared__ Tile S;
     const int tid = threadIdx.x;
     if (tid < T) {
@@ -306,28 +299,42 @@ __global__ __launch_bounds__(256) void k_grad_tile(Net net, const float *x, cons
     backward_tile(S, net, tid, 1.0f / (float)n, partial + (size_t)blockIdx.x * NSLOT);
 }
 
-// sum of the per-tile slots, in parameter order: grad[0..NPARAM) and the loss in grad[NPARAM]
-// Sum of value j over the per-tile gradient slots, in a fixed order (the same bits
-// on every run): eight independent partial sums, so that eight loads of a thread
-// are in flight at a time, combined pairwise.
-__device__ inline float sum_slots(const float *partial, int tiles, int j) {
-    float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int t = 0;
-    for (; t + 8 <= tiles; t += 8) {
-        float v[8];
+// Sum over the per-tile gradient slots of value j = 256 blockIdx + threadIdx (gradient at
+// [0, NPARAM), the loss at NPARAM), in a fixed order (the same bits on every run).  Each of
+// the block's four waves sums a quarter of the slots for all 256 values, 16 bytes per lane
+// and eight loads in flight (with 4 bytes per lane the bytes in flight bounded the sum).
+__device__ inline float sum_slots(const float *partial, int tiles) {
+    __shared__ f4 red[4][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int j4 = blockIdx.x * 256 + 4 * lane;
+    const int per = (tiles + 3) / 4, t0 = min(tiles, wave * per), t1 = min(tiles, t0 + per);
+    f4 s = f4{0.f, 0.f, 0.f, 0.f};
+    if (j4 < NSLOT) {
+        const float *src = partial + j4;
+        f4 a[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = partial[(size_t)(t + u) * NSLOT + j];
+        for (int u = 0; u < 8; ++u) a[u] = s;
+        int t = t0;
+        for (; t + 8 <= t1; t += 8) {
+            f4 v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] += v[u];
+            for (int u = 0; u < 8; ++u) v[u] = *(const f4 *)(src + (size_t)(t + u) * NSLOT);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[u] += v[u];
+        }
+        for (; t < t1; ++t) a[0] += *(const f4 *)(src + (size_t)t * NSLOT);
+        s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
     }
-    for (; t < tiles; ++t) a[0] += partial[(size_t)t * NSLOT + j];
-    return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+    red[wave][lane] = s;
+    __syncthreads();
+    const float *r = (const float *)red + threadIdx.x;
+    return (r[0] + r[256]) + (r[512] + r[768]);
 }
 
-__global__ void k_sum_slots(const float *partial, int tiles, float *grad) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j > NPARAM) return;
-    grad[j == NPARAM ? j : slot_param(j)] = sum_slots(partial, tiles, j);
+__global__ __launch_bounds__(256) void k_sum_slots(const float *partial, int tiles, float *grad) {
+    const float g = sum_slots(partial, tiles);
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (j <= NPARAM) grad[j] = g;
 }
 
 __device__ inline void requant(const NetBufs &nb, int j, float w) {
@@ -351,16 +358,18 @@ __global__ void k_quantize(NetBufs nb) {
 
 // Adam on the summed tile gradients (decoupled weight decay on matrices only),
 // learning rate: linear warm-up then cosine decay to lr_min.
-__global__ void k_adam(NetBufs nb, TrainDev td) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+// The step it works on is step[1], written by k_train_tile; the thread of the loss advances
+// step[0], which nothing else reads meanwhile.
+__global__ __launch_bounds__(256) void k_adam(NetBufs nb, TrainDev td) {
+    const int step = td.step[1];
+    const float g = sum_slots(td.partial, td.batch_tiles);
+    const int j = blockIdx.x * 256 + threadIdx.x;
     if (j > NPARAM) return;
-    const int step = td.step[0];
-    const float g = sum_slots(td.partial, td.batch_tiles, j);
     if (j == NPARAM) {
         td.loss[step - td.step0] = g;
+        td.step[0] = step + 1;
         return;
     }
-    const int pj = slot_param(j);
     float lr;
     if (step < td.warmup) lr = td.lr * (float)(step + 1) / (float)td.warmup;
     else {
@@ -368,19 +377,15 @@ __global__ void k_adam(NetBufs nb, TrainDev td) {
         lr = td.lr_min + 0.5f * (td.lr - td.lr_min) * (1.f + cosf(3.14159265358979f * fminf(f, 1.f)));
     }
     const float t = (float)(step + 1);
-    const float m = nb.m[pj] = td.beta1 * nb.m[pj] + (1.f - td.beta1) * g;
-    const float v = nb.v[pj] = td.beta2 * nb.v[pj] + (1.f - td.beta2) * g * g;
+    const float m = nb.m[j] = td.beta1 * nb.m[j] + (1.f - td.beta1) * g;
+    const float v = nb.v[j] = td.beta2 * nb.v[j] + (1.f - td.beta2) * g * g;
     const float mh = m / (1.f - powf(td.beta1, t)), vh = v / (1.f - powf(td.beta2, t));
-    const bool matrix = (pj < OB1) || (pj >= OW2 && pj < OB2) || (pj >= OW3 && pj < OB3) || (pj >= OW4 && pj < OB4);
-    float w = nb.w[pj];
+    const bool matrix = (j < OB1) || (j >= OW2 && j < OB2) || (j >= OW3 && j < OB3) || (j >= OW4 && j < OB4);
+    float w = nb.w[j];
     if (matrix) w -= lr * td.weight_decay * w;
     w -= lr * mh / (sqrtf(vh) + td.eps);
-    nb.w[pj] = w;
-    requant(nb, pj, w);
-}
-
-__global__ void k_advance(int *step) {
-    if (threadIdx.x == 0) step[0] += 1;
+    nb.w[j] = w;
+    requant(nb, j, w);
 }
 
 // last instance whose first node is <= gidx
@@ -402,8 +407,12 @@ __device__ inline int instance_of_node(const BatchDev &B, long long gidx) {
 // what a source keeps of a point between reading its features and storing its
 // output (the anchor source: the instance's parameters, time and family)
 constexpr int kStash = 8;
-// the features of kAhead tiles are read together, by all 256 threads
-constexpr int kAhead = 4;
+// threads of an inference workgroup: two waves per SIMD, each with 32 columns of both hidden
+// matrices (128 registers), so that one wave's LDS reads and exponentials hide the other's
+constexpr int TI = 512;
+constexpr int CT = H / (16 * (TI / 64));
+// the features of kAhead tiles are read together, by all threads
+constexpr int kAhead = TI / T;
 struct InferTile {
     uint16_t h[2][T][HP];
     float w4[H][NOUT];
@@ -413,14 +422,14 @@ struct InferTile {
     int valid[kAhead][T];
 };
 
-__device__ inline void hidden_reg(const uint16_t *A, uint16_t *Hout, const bf8 (&w)[4][8], const float (&bias)[4],
+__device__ inline void hidden_reg(const uint16_t *A, uint16_t *Hout, const bf8 (&w)[CT][8], const float (&bias)[CT],
                                   int wave, int lane) {
     const int i = lane & 15, g = lane >> 4;
-    f4 acc[4][4];
+    f4 acc[4][CT];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
         bf8 a[4];
@@ -429,28 +438,28 @@ __device__ inline void hidden_reg(const uint16_t *A, uint16_t *Hout, const bf8 (
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct)
+            for (int ct = 0; ct < CT; ++ct)
                 acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], w[ct][ks], acc[rt][ct], 0, 0, 0);
     }
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
+        for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                Hout[(size_t)(16 * rt + 4 * g + j) * HP + 64 * wave + 16 * ct + i] =
+                Hout[(size_t)(16 * rt + 4 * g + j) * HP + 16 * CT * wave + 16 * ct + i] =
                     f2bf(tanh_f(acc[rt][ct][j] + bias[ct]));
 }
 
 template <class Src>
-__global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts) {
+__global__ __launch_bounds__(TI) void k_infer(Net net, Src src, long long npts) {
     __shared__ InferTile S;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
-    bf8 w2[4][8], w3[4][8];
-    float b2[4], b3[4];
+    bf8 w2[CT][8], w3[CT][8];
+    float b2[CT], b3[CT];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-        const int n = 64 * wave + 16 * ct + i;
+    for (int ct = 0; ct < CT; ++ct) {
+        const int n = 16 * CT * wave + 16 * ct + i;
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
             w2[ct][ks] = *(const bf8 *)(net.w2f + (size_t)n * H + 32 * ks + 8 * g);
@@ -461,13 +470,13 @@ __global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts)
     }
     float w1[NIN];
 #pragma unroll
-    for (int q = 0; q < NIN; ++q) w1[q] = net.q[OW1 + q * H + tid];
-    const float b1 = net.q[OB1 + tid];
-    S.w4[tid][0] = net.q[OW4 + 2 * tid];
-    S.w4[tid][1] = net.q[OW4 + 2 * tid + 1];
+    for (int q = 0; q < NIN; ++q) w1[q] = net.q[OW1 + q * H + (tid & (H - 1))];
+    const float b1 = net.q[OB1 + (tid & (H - 1))];
+    static_assert(NOUT * H == TI, "one output weight per thread");
+    S.w4[tid / NOUT][tid % NOUT] = net.q[OW4 + tid];
     const float b40 = net.q[OB4], b41 = net.q[OB4 + 1];
     const long long ntiles = (npts + T - 1) / T;
-    static_assert(kAhead * T == 256, "one feature point per thread");
+    static_assert(kAhead * T == TI, "one feature point per thread");
     for (long long tile0 = blockIdx.x; tile0 < ntiles; tile0 += (long long)kAhead * gridDim.x) {
         {  // features of this workgroup's next kAhead tiles (tile0 + qa * gridDim.x)
             const int qa = tid / T, pa = tid % T;
@@ -484,12 +493,15 @@ __global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts)
         for (int qa = 0; qa < kAhead; ++qa) {
         const long long tile = tile0 + (long long)qa * gridDim.x;
         if (tile >= ntiles) break;
+        // layer 1: a thread owns a column and a half of the points
+        const int n1 = tid & (H - 1), p0 = (tid / H) * (T * H / TI);
 #pragma unroll 8
-        for (int p = 0; p < T; ++p) {
+        for (int it = 0; it < T * H / TI; ++it) {
+            const int p = p0 + it;
             float z = b1;
 #pragma unroll
             for (int q = 0; q < NIN; ++q) z += S.x[qa][p][q] * w1[q];
-            S.h[0][p][tid] = f2bf(tanh_f(z));
+            S.h[0][p][n1] = f2bf(tanh_f(z));
         }
         __syncthreads();
         hidden_reg(&S.h[0][0][0], &S.h[1][0][0], w2, b2, wave, lane);
@@ -497,18 +509,22 @@ __global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts)
         hidden_reg(&S.h[1][0][0], &S.h[0][0][0], w3, b3, wave, lane);
         __syncthreads();
         {
-            const int p = tid >> 2, part = tid & 3;
+            // output layer: eight threads per point, every eighth input each
+            constexpr int TP = TI / T;
+            const int p = tid / TP, part = tid % TP;
             float o0 = 0.f, o1 = 0.f;
 #pragma unroll 16
-            for (int k = 64 * part; k < 64 * part + 64; ++k) {
+            for (int it = 0; it < H / TP; ++it) {
+                const int k = TP * it + part;
                 const float hk = bf2f(S.h[0][p][k]);
                 o0 += hk * S.w4[k][0];
                 o1 += hk * S.w4[k][1];
             }
-            o0 += __shfl_xor(o0, 1);
-            o1 += __shfl_xor(o1, 1);
-            o0 += __shfl_xor(o0, 2);
-            o1 += __shfl_xor(o1, 2);
+#pragma unroll
+            for (int m = 1; m < TP; m *= 2) {
+                o0 += __shfl_xor(o0, m);
+                o1 += __shfl_xor(o1, m);
+            }
             if (part == 0) {
                 S.out[p][0] = (o0 + b40) * net.out_scale[0] + net.out_shift[0];
                 S.out[p][1] = (o1 + b41) * net.out_scale[1] + net.out_shift[1];
@@ -614,16 +630,15 @@ hipError_t launch_quantize(const NetBufs &nb, hipStream_t s) {
 }
 
 hipError_t launch_train_step(const NetBufs &nb, const Net &net, const TrainDev &td, hipStream_t s) {
-    k_train_tile<<<td.batch_tiles, 256, 0, s>>>(net, td);
+    k_train_tile<<<td.batch_tiles, TW, 0, s>>>(net, td);
     k_adam<<<(NSLOT + 255) / 256, 256, 0, s>>>(nb, td);
-    k_advance<<<1, 64, 0, s>>>(td.step);
     return hipGetLastError();
 }
 
 hipError_t launch_grad(const Net &net, const float *x, const float *y, int n, float *partial, float *grad,
                        hipStream_t s) {
     const int tiles = (n + T - 1) / T;
-    k_grad_tile<<<tiles, 256, 0, s>>>(net, x, y, n, partial);
+    k_grad_tile<<<tiles, TW, 0, s>>>(net, x, y, n, partial);
     k_sum_slots<<<(NSLOT + 255) / 256, 256, 0, s>>>(partial, tiles, grad);
     return hipGetLastError();
 }
@@ -634,19 +649,19 @@ static unsigned infer_grid(long long npts, int num_cus) {
 }
 
 hipError_t launch_predict(const Net &net, const float *x, int n, float *out, int num_cus, hipStream_t s) {
-    k_infer<PredictSrc><<<infer_grid(n, num_cus), 256, 0, s>>>(net, PredictSrc{x, out}, n);
+    k_infer<PredictSrc><<<infer_grid(n, num_cus), TI, 0, s>>>(net, PredictSrc{x, out}, n);
     return hipGetLastError();
 }
 
 hipError_t launch_batch_guess(const Net &net, const BatchDev &B, double *init_y, long long total_nodes,
                               int feature_kind, int anchors, double *anc, int num_cus, hipStream_t s) {
     if (anchors == 0) {
-        k_infer<NodeSrc><<<infer_grid(total_nodes, num_cus), 256, 0, s>>>(net, NodeSrc{B, init_y, feature_kind},
+        k_infer<NodeSrc><<<infer_grid(total_nodes, num_cus), TI, 0, s>>>(net, NodeSrc{B, init_y, feature_kind},
                                                                           total_nodes);
         return hipGetLastError();
     }
     const long long pts = (long long)B.n * anchors;
-    k_infer<AnchorSrc><<<infer_grid(pts, num_cus), 256, 0, s>>>(net, AnchorSrc{B, anc, anchors, feature_kind}, pts);
+    k_infer<AnchorSrc><<<infer_grid(pts, num_cus), TI, 0, s>>>(net, AnchorSrc{B, anc, anchors, feature_kind}, pts);
     return hipGetLastError();
 }
 
