@@ -14,7 +14,7 @@
 namespace mlp {
 
 constexpr int NIN = 4, H = 256, NOUT = 2;
-constexpr int T = 64;        // points per tile (one workgroup of 4 waves)
+constexpr int T = 64;        // points per tile (one workgroup)
 constexpr int HP = H + 8;    // LDS row stride of the activation tiles (bf16 elements)
 
 // offsets in the FP32 parameter vector; matrices are input-major: W[i][o]
