@@ -411,8 +411,13 @@ __device__ inline int instance_of_node(const BatchDev &B, long long gidx) {
 // what a source keeps of a point between reading its features and storing its
 // output (the anchor source: the instance's parameters, time and family)
 constexpr int kStash = 8;
-// the features of kAhead tiles are read together, by all 256 threads
-constexpr int kAhead = 4;
+// threads of an inference workgroup: two waves per SIMD, each with 32 columns of both hidden
+// matrices (128 registers), so that one wave's LDS reads and exponentials hide the other's
+// (262,144 points: 270 us with one wave per SIMD and 64 columns, 151 us)
+constexpr int TI = 512;
+constexpr int CT = H / (16 * (TI / 64));
+// the features of kAhead tiles are read together, by all threads
+constexpr int kAhead = TI / T;
 struct InferTile {
     uint16_t h[2][T][HP];
     float w4[H][NOUT];
@@ -422,14 +427,14 @@ struct InferTile {
     int valid[kAhead][T];
 };
 
-__device__ inline void hidden_reg(const uint16_t *A, uint16_t *Hout, const bf8 (&w)[4][8], const float (&bias)[4],
+__device__ inline void hidden_reg(const uint16_t *A, uint16_t *Hout, const bf8 (&w)[CT][8], const float (&bias)[CT],
                                   int wave, int lane) {
     const int i = lane & 15, g = lane >> 4;
-    f4 acc[4][4];
+    f4 acc[4][CT];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
         bf8 a[4];
@@ -438,28 +443,28 @@ __device__ inline void hidden_reg(const uint16_t *A, uint16_t *Hout, const bf8 (
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct)
+            for (int ct = 0; ct < CT; ++ct)
                 acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], w[ct][ks], acc[rt][ct], 0, 0, 0);
     }
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
+        for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                Hout[(size_t)(16 * rt + 4 * g + j) * HP + 64 * wave + 16 * ct + i] =
+                Hout[(size_t)(16 * rt + 4 * g + j) * HP + 16 * CT * wave + 16 * ct + i] =
                     f2bf(tanh_f(acc[rt][ct][j] + bias[ct]));
 }
 
 template <class Src>
-__global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts) {
+__global__ __launch_bounds__(TI) void k_infer(Net net, Src src, long long npts) {
     __shared__ InferTile S;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
-    bf8 w2[4][8], w3[4][8];
-    float b2[4], b3[4];
+    bf8 w2[CT][8], w3[CT][8];
+    float b2[CT], b3[CT];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-        const int n = 64 * wave + 16 * ct + i;
+    for (int ct = 0; ct < CT; ++ct) {
+        const int n = 16 * CT * wave + 16 * ct + i;
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
             w2[ct][ks] = *(const bf8 *)(net.w2f + (size_t)n * H + 32 * ks + 8 * g);
@@ -470,13 +475,13 @@ __global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts)
     }
     float w1[NIN];
 #pragma unroll
-    for (int q = 0; q < NIN; ++q) w1[q] = net.q[OW1 + q * H + tid];
-    const float b1 = net.q[OB1 + tid];
-    S.w4[tid][0] = net.q[OW4 + 2 * tid];
-    S.w4[tid][1] = net.q[OW4 + 2 * tid + 1];
+    for (int q = 0; q < NIN; ++q) w1[q] = net.q[OW1 + q * H + (tid & (H - 1))];
+    const float b1 = net.q[OB1 + (tid & (H - 1))];
+    static_assert(NOUT * H == TI, "one output weight per thread");
+    S.w4[tid / NOUT][tid % NOUT] = net.q[OW4 + tid];
     const float b40 = net.q[OB4], b41 = net.q[OB4 + 1];
     const long long ntiles = (npts + T - 1) / T;
-    static_assert(kAhead * T == 256, "one feature point per thread");
+    static_assert(kAhead * T == TI, "one feature point per thread");
     for (long long tile0 = blockIdx.x; tile0 < ntiles; tile0 += (long long)kAhead * gridDim.x) {
         {  // features of this workgroup's next kAhead tiles (tile0 + qa * gridDim.x)
             const int qa = tid / T, pa = tid % T;
@@ -493,12 +498,15 @@ __global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts)
         for (int qa = 0; qa < kAhead; ++qa) {
         const long long tile = tile0 + (long long)qa * gridDim.x;
         if (tile >= ntiles) break;
+        // layer 1: a thread owns a column and a half of the points
+        const int n1 = tid & (H - 1), p0 = (tid / H) * (T * H / TI);
 #pragma unroll 8
-        for (int p = 0; p < T; ++p) {
+        for (int it = 0; it < T * H / TI; ++it) {
+            const int p = p0 + it;
             float z = b1;
 #pragma unroll
             for (int q = 0; q < NIN; ++q) z += S.x[qa][p][q] * w1[q];
-            S.h[0][p][tid] = f2bf(tanh_f(z));
+            S.h[0][p][n1] = f2bf(tanh_f(z));
         }
         __syncthreads();
         hidden_reg(&S.h[0][0][0], &S.h[1][0][0], w2, b2, wave, lane);
@@ -506,18 +514,22 @@ __global__ __launch_bounds__(256) void k_infer(Net net, Src src, long long npts)
         hidden_reg(&S.h[1][0][0], &S.h[0][0][0], w3, b3, wave, lane);
         __syncthreads();
         {
-            const int p = tid >> 2, part = tid & 3;
+            // output layer: eight threads per point, every eighth input each
+            constexpr int TP = TI / T;
+            const int p = tid / TP, part = tid % TP;
             float o0 = 0.f, o1 = 0.f;
 #pragma unroll 16
-            for (int k = 64 * part; k < 64 * part + 64; ++k) {
+            for (int it = 0; it < H / TP; ++it) {
+                const int k = TP * it + part;
                 const float hk = bf2f(S.h[0][p][k]);
                 o0 += hk * S.w4[k][0];
                 o1 += hk * S.w4[k][1];
             }
-            o0 += __shfl_xor(o0, 1);
-            o1 += __shfl_xor(o1, 1);
-            o0 += __shfl_xor(o0, 2);
-            o1 += __shfl_xor(o1, 2);
+#pragma unroll
+            for (int m = 1; m < TP; m *= 2) {
+                o0 += __shfl_xor(o0, m);
+                o1 += __shfl_xor(o1, m);
+            }
             if (part == 0) {
                 S.out[p][0] = (o0 + b40) * net.out_scale[0] + net.out_shift[0];
                 S.out[p][1] = (o1 + b41) * net.out_scale[1] + net.out_shift[1];
@@ -642,19 +654,19 @@ static unsigned infer_grid(long long npts, int num_cus) {
 }
 
 hipError_t launch_predict(const Net &net, const float *x, int n, float *out, int num_cus, hipStream_t s) {
-    k_infer<PredictSrc><<<infer_grid(n, num_cus), 256, 0, s>>>(net, PredictSrc{x, out}, n);
+    k_infer<PredictSrc><<<infer_grid(n, num_cus), TI, 0, s>>>(net, PredictSrc{x, out}, n);
     return hipGetLastError();
 }
 
 hipError_t launch_batch_guess(const Net &net, const BatchDev &B, double *init_y, long long total_nodes,
                               int feature_kind, int anchors, double *anc, int num_cus, hipStream_t s) {
     if (anchors == 0) {
-        k_infer<NodeSrc><<<infer_grid(total_nodes, num_cus), 256, 0, s>>>(net, NodeSrc{B, init_y, feature_kind},
+        k_infer<NodeSrc><<<infer_grid(total_nodes, num_cus), TI, 0, s>>>(net, NodeSrc{B, init_y, feature_kind},
                                                                           total_nodes);
         return hipGetLastError();
     }
     const long long pts = (long long)B.n * anchors;
-    k_infer<AnchorSrc><<<infer_grid(pts, num_cus), 256, 0, s>>>(net, AnchorSrc{B, anc, anchors, feature_kind}, pts);
+    k_infer<AnchorSrc><<<infer_grid(pts, num_cus), TI, 0, s>>>(net, AnchorSrc{B, anc, anchors, feature_kind}, pts);
     return hipGetLastError();
 }
 
