@@ -7,7 +7,7 @@ import pathlib
 import numpy as np
 
 from . import _abi
-from .problems import instance_array
+from .problems import _struct_dtype, instance_array
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "_build" / "libbvp_mirk.so"
 
@@ -372,27 +372,35 @@ class RawSolution:
         self.stages = None
 
 
+_RESULT = _struct_dtype(_abi.Result)
+
+
 def _result_array(specs, cap, stages=0):
-    n = len(specs)
+    """bvp_result rows with room for cap nodes each, and the arrays they point into: meshes
+    (n, cap), solutions (n, cap * M) and stages (n, cap * stages * M or None)."""
+    n, M = len(specs), max((s.M for s in specs), default=0)
     res = (_abi.Result * n)()
-    bufs = []
-    for i, s in enumerate(specs):
-        m, u = np.zeros(cap), np.zeros(cap * s.M)
-        k = np.zeros(max(1, cap * stages * s.M)) if stages else None
-        bufs.append((m, u, k))
-        res[i].capacity = cap
-        res[i].mesh = m.ctypes.data_as(_dp)
-        res[i].u = u.ctypes.data_as(_dp)
-        if stages:
-            res[i].stages = k.ctypes.data_as(_dp)
+    if n == 0:
+        return res, ((), (), ())
+    # one lazily zeroed block per kind, a row per instance
+    bufs = (np.zeros((n, cap)), np.zeros((n, cap * M)), np.zeros((n, cap * stages * M)) if stages else None)
+    v = np.frombuffer(res, dtype=_RESULT, count=n)
+    v["capacity"] = cap
+    row = np.arange(n, dtype=np.uint64)
+    for name, b in zip(("mesh", "u", "stages"), bufs):
+        if b is not None:
+            v[name] = np.uint64(b.ctypes.data) + row * np.uint64(b.strides[0])
     return res, bufs
 
 
-def _raw(res, spec, buf, stages):
-    r = RawSolution(res, spec.M, buf[0], buf[1])
-    if stages:
-        r.stages = buf[2][:r.N * stages * spec.M].reshape(r.N, stages, spec.M).copy()
-    return r
+def _raws(res, specs, bufs, stages):
+    out = []
+    for i, spec in enumerate(specs):
+        r = RawSolution(res[i], spec.M, bufs[0][i], bufs[1][i])
+        if stages:
+            r.stages = bufs[2][i, :r.N * stages * spec.M].reshape(r.N, stages, spec.M).copy()
+        out.append(r)
+    return out
 
 
 def solve_batch(ctx, opts, specs):
@@ -403,7 +411,7 @@ def solve_batch(ctx, opts, specs):
     st = _abi.firk_stages(opts.method) if _abi.is_firk(opts.method) else 0
     res, bufs = _result_array(specs, cap, st)
     ctx.check(lib().bvp_mirk_solve_batch(ctx.handle, C.byref(opts), len(specs), arr, res), "solve_batch")
-    return [_raw(res[i], specs[i], bufs[i], st) for i in range(len(specs))]
+    return _raws(res, specs, bufs, st)
 
 
 def solve_batch_noalloc(ctx, opts, specs):
@@ -415,7 +423,7 @@ def solve_batch_noalloc(ctx, opts, specs):
     res, bufs = _result_array(specs, cap, st)
     ctx.check(lib().bvp_mirk_solve_batch_noalloc(ctx.handle, C.byref(opts), len(specs), arr, res),
               "solve_batch_noalloc")
-    return [_raw(res[i], specs[i], bufs[i], st) for i in range(len(specs))]
+    return _raws(res, specs, bufs, st)
 
 
 class Batch:
@@ -443,7 +451,7 @@ class Batch:
         st = _abi.firk_stages(self.opts.method) if _abi.is_firk(self.opts.method) else 0
         res, bufs = _result_array(self.specs, cap, st)
         self.ctx.check(lib().bvp_batch_results(self.ctx.handle, self._h, res), "batch_results")
-        return [_raw(res[i], self.specs[i], bufs[i], st) for i in range(len(self.specs))]
+        return _raws(res, self.specs, bufs, st)
 
     def learned_guess(self):
         """The attached network's guess at every node, one (N+1, M) array per instance."""

@@ -13,6 +13,8 @@
 #include <cstring>
 #include <numeric>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/bvp_mirk.h"
@@ -53,31 +55,45 @@ int validate(bvp_ctx *ctx, int32_t n, const bvp_instance *inst, int &M) {
     return rc;
 }
 
-template <typename T>
-int dalloc(bvp_ctx *ctx, DevArena &arena, T *&p, size_t count) {
-    p = nullptr;
-    if (count == 0) count = 1;
+// bytes of device memory from the arena (aligned to 256), or null with the context's error set
+void *arena_bytes(bvp_ctx *ctx, DevArena &arena, size_t count) {
+    const size_t bytes = (std::max<size_t>(count, 1) + 255) & ~(size_t)255;
     if (arena.bump) {
-        const size_t bytes = (count * sizeof(T) + 255) & ~(size_t)255;
         if (arena.bump_used + bytes > arena.bump_cap) {
             set_err(ctx, "the call needs more than the %zu bytes of the no-allocation scratch (%zu more bytes "
                          "requested with %zu in use): solve fewer instances per call or lower "
                          "max_num_subintervals", arena.bump_cap, bytes, arena.bump_used);
-            return BVP_ENOMEM;
+            return nullptr;
         }
-        p = (T *)(arena.bump + arena.bump_used);
         arena.bump_used += bytes;
-        return 0;
+        return arena.bump + arena.bump_used - bytes;
     }
-    void *q = nullptr;
-    hipError_t e = hipMalloc(&q, count * sizeof(T));
-    if (e != hipSuccess) {
-        set_err(ctx, "hipMalloc(%zu bytes) failed: %s", count * sizeof(T), hipGetErrorString(e));
-        return BVP_ENOMEM;
+    constexpr size_t kShared = (size_t)1 << 20;  // small allocations share blocks of this size
+    if (bytes > arena.cur_left || bytes > kShared / 4) {
+        if (!arena.pool) arena.pool = ctx->pool;
+        size_t got = 0;
+        const bool own = bytes > kShared / 4;
+        void *q = arena.pool->take(own ? bytes : kShared, got);
+        if (!q) {
+            set_err(ctx, "hipMalloc(%zu bytes) failed: out of memory", own ? bytes : kShared);
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        arena.blocks.emplace_back(q, got);
+        if (own) return q;
+        arena.cur = (char *)q;
+        arena.cur_left = got;
     }
-    arena.ptrs.push_back(q);
-    p = (T *)q;
-    return 0;
+    char *p = arena.cur;
+    arena.cur += bytes;
+    arena.cur_left -= bytes;
+    return p;
+}
+
+template <typename T>
+int dalloc(bvp_ctx *ctx, DevArena &arena, T *&p, size_t count) {
+    p = (T *)arena_bytes(ctx, arena, count * sizeof(T));
+    return p ? 0 : BVP_ENOMEM;
 }
 
 template <typename T>
@@ -88,10 +104,225 @@ int upload(bvp_ctx *ctx, DevArena &arena, T *&p, const std::vector<T> &v) {
     return 0;
 }
 
+// Several host arrays to one device region: a single copy through the pinned staging area
+// where they fit it, else one copy per array.  The arrays must stay until the stream is
+// synchronised.
+class Uploads {
+  public:
+    template <typename T> void add(T *&p, const std::vector<T> &v) {
+        items_.push_back({(void **)&p, v.data(), v.size() * sizeof(T), total_});
+        total_ += (std::max<size_t>(v.size() * sizeof(T), 1) + 255) & ~(size_t)255;
+    }
+    int commit(bvp_ctx *ctx, DevArena &arena) {
+        char *d = (char *)arena_bytes(ctx, arena, total_);
+        if (!d) return BVP_ENOMEM;
+        char *h = arena.bump ? nullptr : ctx->pin.take(total_);
+        for (const Item &it : items_) {
+            *it.dst = d + it.off;
+            if (!it.bytes) continue;
+            if (h) std::memcpy(h + it.off, it.src, it.bytes);
+            else HIP_TRY(ctx, hipMemcpyAsync(d + it.off, it.src, it.bytes, hipMemcpyHostToDevice, ctx->stream));
+        }
+        if (h) HIP_TRY(ctx, hipMemcpyAsync(d, h, total_, hipMemcpyHostToDevice, ctx->stream));
+        return 0;
+    }
+
+  private:
+    struct Item {
+        void **dst;
+        const void *src;
+        size_t bytes, off;
+    };
+    std::vector<Item> items_;
+    size_t total_ = 0;
+};
+
+// A device array of consecutive per-instance pieces (piece i: off[i] .. off[i + 1] in units
+// of `unit` bytes) and where each piece goes on the host (null: dropped).
+struct Pieces {
+    const void *dev = nullptr;
+    size_t unit = 0;
+    const long long *off = nullptr;  // [n + 1]
+    std::vector<char *> dst;
+    size_t bytes() const { return (size_t)off[dst.size()] * unit; }
+    // host copy of bytes [a, b) of the array at src
+    void scatter(size_t a, size_t b, const char *src) const {
+        const size_t n = dst.size();
+        size_t i = std::upper_bound(off, off + n + 1, (long long)(a / unit)) - off;
+        i = i ? i - 1 : 0;
+        for (; i < n && (size_t)off[i] * unit < b; ++i) {
+            const size_t lo = std::max((size_t)off[i] * unit, a), hi = std::min((size_t)off[i + 1] * unit, b);
+            if (dst[i] && hi > lo) std::memcpy(dst[i] + (lo - (size_t)off[i] * unit), src + (lo - a), hi - lo);
+        }
+    }
+};
+
+// Copies the pieces back, all device work of the stream done on return.  Up to the small
+// staging area in one go; larger results stream through two pinned chunks, each scattered
+// by a few host threads while the next one is on its way (pageable copies of the whole and
+// one thread's scatter: 32 ms for 8,192 Bratu solutions of 560 nodes, 110 MB).
+int fetch(bvp_ctx *ctx, const std::vector<Pieces> &ps, bool pinned) {
+    size_t total = 0;
+    for (const Pieces &p : ps) total += (p.bytes() + 255) & ~(size_t)255;
+    char *h = pinned ? ctx->pin.take(total) : nullptr;
+    if (h || !pinned || !ctx->pin.chunks()) {
+        std::vector<char> own;
+        if (!h) {
+            own.resize(total);
+            h = own.data();
+        }
+        size_t o = 0;
+        for (const Pieces &p : ps) {
+            if (p.bytes()) HIP_TRY(ctx, hipMemcpyAsync(h + o, p.dev, p.bytes(), hipMemcpyDeviceToHost, ctx->stream));
+            o += (p.bytes() + 255) & ~(size_t)255;
+        }
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        o = 0;
+        for (const Pieces &p : ps) {
+            p.scatter(0, p.bytes(), h + o);
+            o += (p.bytes() + 255) & ~(size_t)255;
+        }
+        return 0;
+    }
+    struct Chunk {
+        const Pieces *p;
+        size_t a, b;
+    };
+    std::vector<Chunk> cs;
+    for (const Pieces &p : ps) {
+        const size_t step = PinnedStage::kChunk / p.unit * p.unit;
+        for (size_t a = 0; a < p.bytes(); a += step) cs.push_back({&p, a, std::min(a + step, p.bytes())});
+    }
+    const unsigned hw = std::thread::hardware_concurrency();
+    const int nt = (int)std::min(8u, std::max(1u, hw / 2));
+    auto enqueue = [&](size_t c) -> int {
+        HIP_TRY(ctx, hipMemcpyAsync(ctx->pin.chunk[c & 1], (const char *)cs[c].p->dev + cs[c].a, cs[c].b - cs[c].a,
+                                    hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(ctx, hipEventRecord(ctx->pin.ev[c & 1], ctx->stream));
+        return 0;
+    };
+    if (cs.empty()) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    else if (int rc = enqueue(0)) return rc;
+    for (size_t c = 0; c < cs.size(); ++c) {
+        if (c + 1 < cs.size())
+            if (int rc = enqueue(c + 1)) return rc;
+        HIP_TRY(ctx, hipEventSynchronize(ctx->pin.ev[c & 1]));
+        const Chunk &k = cs[c];
+        const char *src = ctx->pin.chunk[c & 1];
+        const size_t len = k.b - k.a, part = (len / nt + 63) & ~(size_t)63;
+        auto work = [&k, src, len, part](int t) {
+            const size_t lo = std::min(len, part * t), hi = std::min(len, part * (t + 1));
+            if (hi > lo) k.p->scatter(k.a + lo, k.a + hi, src + lo);
+        };
+        std::vector<std::thread> th;
+        int t = 1;
+        if (len > PinnedStage::kSmall) {
+            try {
+                for (; t < nt; ++t) th.emplace_back(work, t);
+            } catch (const std::system_error &) {  // no more threads: the rest runs here
+            }
+        }
+        work(0);
+        for (; t < nt; ++t) work(t);
+        for (std::thread &x : th) x.join();
+    }
+    return 0;
+}
+
 }  // namespace
 
 DevArena::~DevArena() {
-    for (void *p : ptrs) (void)hipFree(p);
+    for (auto &b : blocks) pool->give(b.first, b.second);
+}
+
+void *DevPool::take(size_t bytes, size_t &got) {
+    // sizes in steps of an eighth of their power of two, so that blocks of nearly the same
+    // calls fit each other
+    size_t step = 4096;
+    while (step * 16 < bytes) step *= 2;
+    got = (bytes + step - 1) / step * step;
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        auto it = held_.lower_bound(got);
+        if (it != held_.end() && it->first <= got + got / 4) {
+            void *p = it->second;
+            got = it->first;
+            held_bytes_ -= got;
+            held_.erase(it);
+            return p;
+        }
+    }
+    void *q = nullptr;
+    if (hipMalloc(&q, got) == hipSuccess) return q;
+    release();  // the held blocks may be what is missing
+    (void)hipGetLastError();
+    return hipMalloc(&q, got) == hipSuccess ? q : nullptr;
+}
+
+void DevPool::give(void *p, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        if (!closed_ && bytes <= kMaxBlock && held_bytes_ + bytes <= kMaxHeld) {
+            held_.emplace(bytes, p);
+            held_bytes_ += bytes;
+            return;
+        }
+    }
+    (void)hipFree(p);
+}
+
+void DevPool::release() {
+    std::multimap<size_t, void *> out;
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        out.swap(held_);
+        held_bytes_ = 0;
+    }
+    for (auto &b : out) (void)hipFree(b.second);
+}
+
+void DevPool::close() {
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        closed_ = true;
+    }
+    release();
+}
+
+char *PinnedStage::take(size_t bytes) {
+    if (bytes > kSmall) return nullptr;
+    if (!small && hipHostMalloc((void **)&small, kSmall, hipHostMallocDefault) != hipSuccess) {
+        small = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const size_t b = (bytes + 255) & ~(size_t)255;
+    if (used + b > kSmall) return nullptr;
+    used += b;
+    return small + used - b;
+}
+
+bool PinnedStage::chunks() {
+    for (int k = 0; k < 2; ++k) {
+        if (!chunk[k] && hipHostMalloc((void **)&chunk[k], kChunk, hipHostMallocDefault) != hipSuccess) chunk[k] = nullptr;
+        if (!ev[k] && hipEventCreateWithFlags(&ev[k], hipEventDisableTiming) != hipSuccess) ev[k] = nullptr;
+        if (!chunk[k] || !ev[k]) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    return true;
+}
+
+void PinnedStage::free_all() {
+    if (small) (void)hipHostFree(small);
+    small = nullptr;
+    for (int k = 0; k < 2; ++k) {
+        if (chunk[k]) (void)hipHostFree(chunk[k]);
+        if (ev[k]) (void)hipEventDestroy(ev[k]);
+        chunk[k] = nullptr;
+        ev[k] = nullptr;
+    }
 }
 
 // ------------------------------------------------------------------ no-allocation scratch
@@ -103,12 +334,31 @@ DevArena::~DevArena() {
 constexpr size_t kNoAllocBytes = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
+// The per-instance scalars of a batch's results, back to back (on the device and in the
+// host copy alike).
+struct ResultHead {
+    double *dn, *rn, *er;
+    int *ret, *N, *it, *outer, *fb;
+    static size_t bytes(int n) { return (size_t)n * (3 * sizeof(double) + 5 * sizeof(int)); }
+    ResultHead(char *p, int n) {
+        dn = (double *)p;
+        rn = dn + n;
+        er = rn + n;
+        ret = (int *)(er + n);
+        N = ret + n;
+        it = N + n;
+        outer = it + n;
+        fb = outer + n;
+    }
+};
+
 // ------------------------------------------------------------------ batch build
 int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *inst, int cap_req, bvp_batch **out,
                 char *bump, size_t bump_cap) {
     int M;
     int rc = validate(ctx, n, inst, M);
     if (rc) return rc;
+    ctx->pin.used = 0;  // every call leaves the stream's copies through it done
     const bool blk = !wave_supports(M, inst[0].family);
     if (blk && bump) {
         set_err(ctx, "the no-allocation entry point serves the wave-kernel state dimensions (M = 1..4, 6)");
@@ -181,12 +431,23 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
     int *dfam, *dpoff, *dpcnt, *dbck, *dbcc, *dN0, *dorder;
     double *dt0, *dt1, *dparams, *dbct, *dbcv, *dim, *diy, *du0c;
     long long *dioff;
-    if ((rc = upload(ctx, A, dfam, fam)) || (rc = upload(ctx, A, dpoff, poff)) || (rc = upload(ctx, A, dpcnt, pcnt)) ||
-        (rc = upload(ctx, A, dbck, bck)) || (rc = upload(ctx, A, dbcc, bcc)) || (rc = upload(ctx, A, dN0, N0)) ||
-        (rc = upload(ctx, A, dorder, order)) || (rc = upload(ctx, A, dt0, t0)) || (rc = upload(ctx, A, dt1, t1)) ||
-        (rc = upload(ctx, A, dparams, params)) || (rc = upload(ctx, A, dbct, bct)) || (rc = upload(ctx, A, dbcv, bcv)) ||
-        (rc = upload(ctx, A, dim, imesh)) || (rc = upload(ctx, A, diy, iy)) || (rc = upload(ctx, A, dioff, ioff)) ||
-        (rc = upload(ctx, A, du0c, u0c))) {
+    FirkTab *dtab = nullptr;
+    std::vector<FirkTab> tab(firk ? 1 : 0);
+    if (firk) {
+        std::memcpy(tab[0].A, ftab.A, sizeof tab[0].A);
+        std::memcpy(tab[0].b, ftab.b, sizeof tab[0].b);
+        std::memcpy(tab[0].c, ftab.c, sizeof tab[0].c);
+        std::memcpy(tab[0].Q, ftab.Q, sizeof tab[0].Q);
+        tab[0].tau = ftab.tau;
+        tab[0].s = ftab.s;
+        tab[0].order = ftab.order;
+    }
+    Uploads up;
+    up.add(dfam, fam); up.add(dpoff, poff); up.add(dpcnt, pcnt); up.add(dbck, bck); up.add(dbcc, bcc);
+    up.add(dN0, N0); up.add(dorder, order); up.add(dt0, t0); up.add(dt1, t1); up.add(dparams, params);
+    up.add(dbct, bct); up.add(dbcv, bcv); up.add(dim, imesh); up.add(diy, iy); up.add(dioff, ioff);
+    up.add(du0c, u0c); up.add(dtab, tab);
+    if ((rc = up.commit(ctx, A))) {
         delete B;
         return rc;
     }
@@ -195,17 +456,20 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
     D.init_mesh = dim; D.init_y = diy; D.init_off = dioff;
     D.u0c = du0c;
     D.warm = (o->warm_start == BVP_WARM_MLP) ? 1 : 0;
-    // working state and results
+    // working state; the per-instance results in one region, in the order batch_results
+    // copies them back
+    char *res = nullptr;
     if ((rc = dalloc(ctx, A, D.mesh, (size_t)n * 2 * cap)) || (rc = dalloc(ctx, A, D.y, (size_t)n * 2 * cap * M)) ||
-        (rc = dalloc(ctx, A, D.shat, (size_t)n * cap)) || (rc = dalloc(ctx, A, D.retcode, n)) ||
-        (rc = dalloc(ctx, A, D.N_final, n)) || (rc = dalloc(ctx, A, D.newton_iters, n)) ||
-        (rc = dalloc(ctx, A, D.outer_iters, n)) || (rc = dalloc(ctx, A, D.fallback, n)) ||
-        (rc = dalloc(ctx, A, D.cur_buf, n)) || (rc = dalloc(ctx, A, D.defect_norm, n)) ||
-        (rc = dalloc(ctx, A, D.resid_norm, n)) || (rc = dalloc(ctx, A, D.err, n)) ||
-        (rc = dalloc(ctx, A, D.cnt, (size_t)n * 4)) ||
+        (rc = dalloc(ctx, A, D.shat, (size_t)n * cap)) || (rc = dalloc(ctx, A, res, ResultHead::bytes(n))) ||
+        (rc = dalloc(ctx, A, D.cnt, (size_t)n * 4)) || (rc = dalloc(ctx, A, D.cur_buf, n)) ||
         (rc = dalloc(ctx, A, D.counter, 1))) {
         delete B;
         return rc;
+    }
+    {
+        const ResultHead h(res, n);
+        D.defect_norm = h.dn; D.resid_norm = h.rn; D.err = h.er;
+        D.retcode = h.ret; D.N_final = h.N; D.newton_iters = h.it; D.outer_iters = h.outer; D.fallback = h.fb;
     }
     // persistent slots: the kernel variant and waves per CU from an earlier tuning
     // of this kind of plan, else variant 0 at its occupancy; scratch is sized for
@@ -292,17 +556,7 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
         return rc;
     }
     if (firk) {
-        FirkTab tab{};
-        std::memcpy(tab.A, ftab.A, sizeof tab.A);
-        std::memcpy(tab.b, ftab.b, sizeof tab.b);
-        std::memcpy(tab.c, ftab.c, sizeof tab.c);
-        std::memcpy(tab.Q, ftab.Q, sizeof tab.Q);
-        tab.tau = ftab.tau;
-        tab.s = ftab.s;
-        tab.order = ftab.order;
-        FirkTab *dtab = nullptr;
-        if ((rc = upload(ctx, A, dtab, std::vector<FirkTab>(1, tab))) ||
-            (rc = dalloc(ctx, A, D.stK, (size_t)n * ((size_t)cap + 64) * ftab.s * M))) {
+        if ((rc = dalloc(ctx, A, D.stK, (size_t)n * ((size_t)cap + 64) * ftab.s * M))) {
             delete B;
             return rc;
         }
@@ -441,81 +695,81 @@ int batch_sync(bvp_ctx *ctx, bvp_batch *B, float *ms) {
 }
 
 int batch_results(bvp_ctx *ctx, bvp_batch *B, bvp_result *res) {
-    const int n = B->n, M = B->M;
+    const int n = B->n, M = B->M, S = B->firk_s;
     const BatchDev &D = B->dev;
-    std::vector<int> ret(n), Nf(n), it(n), ou(n), fb(n);
-    std::vector<double> dn(n), rn(n), er(n);
-    HIP_TRY(ctx, hipMemcpy(ret.data(), D.retcode, n * sizeof(int), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(Nf.data(), D.N_final, n * sizeof(int), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(it.data(), D.newton_iters, n * sizeof(int), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(ou.data(), D.outer_iters, n * sizeof(int), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(fb.data(), D.fallback, n * sizeof(int), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(dn.data(), D.defect_norm, n * sizeof(double), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(rn.data(), D.resid_norm, n * sizeof(double), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(er.data(), D.err, n * sizeof(double), hipMemcpyDeviceToHost));
-    std::vector<long long> off(n);
-    long long tot = 0;
-    int maxn = 0;
-    for (int i = 0; i < n; ++i) {
-        off[i] = tot;
-        tot += Nf[i] + 1;
-        maxn = std::max(maxn, Nf[i] + 1);
+    const bool pinned = !B->arena.bump;  // the no-allocation entry point allocates no pinned memory either
+    ctx->pin.used = 0;
+    char *hh = pinned ? ctx->pin.take(ResultHead::bytes(n)) : nullptr;
+    std::vector<char> own;
+    if (!hh) {
+        own.resize(ResultHead::bytes(n));
+        hh = own.data();
     }
+    HIP_TRY(ctx, hipMemcpyAsync(hh, D.defect_norm, ResultHead::bytes(n), hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    const ResultHead h(hh, n);
+    std::vector<long long> off((size_t)n + 1), ioff((size_t)n + 1);
+    int maxn = 0;
+    bool bad = false, want_stages = false;
+    for (int i = 0; i < n; ++i) {
+        off[i + 1] = off[i] + h.N[i] + 1;
+        ioff[i + 1] = ioff[i] + h.N[i];
+        maxn = std::max(maxn, h.N[i] + 1);
+        bvp_result &r = res[i];
+        r.retcode = h.ret[i];
+        r.N_final = h.N[i];
+        r.newton_iters = h.it[i];
+        r.outer_iters = h.outer[i];
+        r.fallback_used = h.fb[i];
+        r.defect_norm = h.dn[i];
+        r.resid_norm = h.rn[i];
+        r.err_vs_fp64 = h.er[i];
+        bad |= r.capacity < h.N[i] + 1;
+        want_stages |= B->firk && r.stages != nullptr;
+    }
+    want_stages &= !bad;
+    const long long tot = off[n], nint = ioff[n];
     DevArena tmp;
     if (B->arena.bump) {  // the gather buffers follow the plan's own part of the region
         tmp.bump = B->arena.bump + B->arena.bump_used;
         tmp.bump_cap = B->arena.bump_cap - B->arena.bump_used;
     }
-    long long *doff;
-    double *dm, *dy;
+    long long *doff = nullptr, *dio = nullptr;
+    double *dm = nullptr, *dy = nullptr, *dk = nullptr;
+    Uploads up;
+    up.add(doff, off);
+    if (want_stages) up.add(dio, ioff);
     int rc;
-    if ((rc = upload(ctx, tmp, doff, off)) || (rc = dalloc(ctx, tmp, dm, (size_t)tot)) ||
-        (rc = dalloc(ctx, tmp, dy, (size_t)tot * M)))
+    if ((rc = up.commit(ctx, tmp)) || (rc = dalloc(ctx, tmp, dm, (size_t)tot)) ||
+        (rc = dalloc(ctx, tmp, dy, (size_t)tot * M)) ||
+        (want_stages && (rc = dalloc(ctx, tmp, dk, (size_t)std::max(1LL, nint) * S * M))))
         return rc;
     HIP_TRY(ctx, wave_launch_gather(D, doff, dm, dy, maxn, ctx->stream));
-    std::vector<double> hm((size_t)tot), hy((size_t)tot * M);
-    HIP_TRY(ctx, hipMemcpyAsync(hm.data(), dm, hm.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(hy.data(), dy, hy.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    int bad = 0;
-    for (int i = 0; i < n; ++i) {
-        bvp_result &r = res[i];
-        r.retcode = ret[i];
-        r.N_final = Nf[i];
-        r.newton_iters = it[i];
-        r.outer_iters = ou[i];
-        r.fallback_used = fb[i];
-        r.defect_norm = dn[i];
-        r.resid_norm = rn[i];
-        r.err_vs_fp64 = er[i];
-        if (r.capacity < Nf[i] + 1) { bad = 1; continue; }
-        if (r.mesh) std::memcpy(r.mesh, &hm[(size_t)off[i]], sizeof(double) * (Nf[i] + 1));
-        if (r.u) std::memcpy(r.u, &hy[(size_t)off[i] * M], sizeof(double) * (size_t)M * (Nf[i] + 1));
+    if (want_stages) HIP_TRY(ctx, firk_launch_gather(D, S, dio, dk, ctx->stream));
+    std::vector<Pieces> ps(want_stages ? 3 : 2);
+    ps[0].dev = dm;
+    ps[0].unit = sizeof(double);
+    ps[1].dev = dy;
+    ps[1].unit = sizeof(double) * M;
+    for (int k = 0; k < 2; ++k) {
+        ps[k].off = off.data();
+        ps[k].dst.resize(n);
     }
-    if (bad) { set_err(ctx, "result capacity smaller than the final mesh"); return BVP_EINVAL; }
-    bool want_stages = false;
-    for (int i = 0; i < n; ++i) want_stages |= B->firk && res[i].stages != nullptr;
     if (want_stages) {
-        // final stage values, instances back to back at interval offsets
-        const int S = B->firk_s;
-        std::vector<long long> ioff(n);
-        long long nint = 0;
-        for (int i = 0; i < n; ++i) {
-            ioff[i] = nint;
-            nint += Nf[i];
-        }
-        long long *dio;
-        double *dk;
-        if ((rc = upload(ctx, tmp, dio, ioff)) || (rc = dalloc(ctx, tmp, dk, (size_t)std::max(1LL, nint) * S * M)))
-            return rc;
-        HIP_TRY(ctx, firk_launch_gather(D, S, dio, dk, ctx->stream));
-        std::vector<double> hk((size_t)nint * S * M);
-        HIP_TRY(ctx, hipMemcpyAsync(hk.data(), dk, hk.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-        for (int i = 0; i < n; ++i)
-            if (res[i].stages)
-                std::memcpy(res[i].stages, &hk[(size_t)ioff[i] * S * M], sizeof(double) * (size_t)Nf[i] * S * M);
+        ps[2].dev = dk;
+        ps[2].unit = sizeof(double) * S * M;
+        ps[2].off = ioff.data();
+        ps[2].dst.resize(n);
     }
+    for (int i = 0; i < n; ++i) {
+        const bvp_result &r = res[i];
+        const bool fits = r.capacity >= r.N_final + 1;
+        ps[0].dst[i] = fits ? (char *)r.mesh : nullptr;
+        ps[1].dst[i] = fits ? (char *)r.u : nullptr;
+        if (want_stages) ps[2].dst[i] = (char *)r.stages;
+    }
+    if ((rc = fetch(ctx, ps, pinned))) return rc;
+    if (bad) { set_err(ctx, "result capacity smaller than the final mesh"); return BVP_EINVAL; }
     return 0;
 }
 
@@ -582,6 +836,8 @@ void bvp_ctx_destroy(bvp_ctx *c) {
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->evm) (void)hipEventDestroy(c->evm);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    c->pin.free_all();
+    c->pool->close();  // blocks of arenas that outlive the context go straight back
     delete c;
 }
 
@@ -593,6 +849,7 @@ int bvp_mirk_solve_batch(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_i
     bvp_batch *B = nullptr;
     int rc = batch_build(ctx, o, n, inst, 0, &B, nullptr, 0);
     if (rc) return rc;
+    B->use_graph = false;  // run once: capturing and instantiating a graph costs more than its launch saves
     if ((rc = batch_run(ctx, B)) == 0 && (rc = batch_sync(ctx, B, nullptr)) == 0) rc = batch_results(ctx, B, res);
     delete B;
     return rc;
@@ -789,6 +1046,20 @@ int bvp_mirk_global_error(bvp_ctx *ctx, const bvp_opts *opts, int32_t n, const b
     return rc;
 }
 
+// nq points of M values each to u, and their derivatives to du when it is set
+static int fetch_points(bvp_ctx *ctx, long long nq, int M, const double *dev_u, double *u, const double *dev_du,
+                        double *du) {
+    const long long off[2] = {0, nq};
+    std::vector<Pieces> ps(du ? 2 : 1);
+    for (size_t k = 0; k < ps.size(); ++k) {
+        ps[k].dev = k ? dev_du : dev_u;
+        ps[k].unit = sizeof(double) * M;
+        ps[k].off = off;
+        ps[k].dst.assign(1, (char *)(k ? du : u));
+    }
+    return fetch(ctx, ps, true);
+}
+
 int bvp_mirk_interpolate(bvp_ctx *ctx, int32_t method, int32_t n, const bvp_instance *inst, const int32_t *n_t,
                          const double *t, double *u, double *du) {
     if (!ctx || !n_t || !u) return BVP_EINVAL;
@@ -818,18 +1089,19 @@ int bvp_mirk_interpolate(bvp_ctx *ctx, int32_t method, int32_t n, const bvp_inst
     int *dqi = nullptr;
     double *dt = nullptr, *du_ = nullptr, *ddu = nullptr;
     const int M = B->M;
+    Uploads up;
+    up.add(dqi, qi);
+    up.add(dt, tv);
     if (nq > 0 &&
-        ((rc = upload(ctx, B->arena, dqi, qi)) || (rc = upload(ctx, B->arena, dt, tv)) ||
+        ((rc = up.commit(ctx, B->arena)) ||
          (rc = dalloc(ctx, B->arena, du_, (size_t)nq * M)) || (du && (rc = dalloc(ctx, B->arena, ddu, (size_t)nq * M))))) {
         delete B;
         return rc;
     }
     if (nq > 0) {
         hipError_t e = wave_launch_interp(B->dev, method, dqi, dt, du_, ddu, nq, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        if (e == hipSuccess) e = hipMemcpy(u, du_, (size_t)nq * M * sizeof(double), hipMemcpyDeviceToHost);
-        if (e == hipSuccess && du) e = hipMemcpy(du, ddu, (size_t)nq * M * sizeof(double), hipMemcpyDeviceToHost);
         if (e != hipSuccess) { set_err(ctx, "interpolate: %s", hipGetErrorString(e)); rc = BVP_EHIP; }
+        else rc = fetch_points(ctx, nq, M, du_, u, ddu, du);
     }
     delete B;
     return rc;
@@ -937,18 +1209,19 @@ int bvp_firk_interpolate(bvp_ctx *ctx, int32_t method, int32_t n, const bvp_inst
     int *dqi = nullptr;
     double *dt = nullptr, *du_ = nullptr, *ddu = nullptr;
     const int M = B->M;
+    Uploads up;
+    up.add(dqi, qi);
+    up.add(dt, tv);
     if (nq > 0 &&
-        ((rc = upload(ctx, B->arena, dqi, qi)) || (rc = upload(ctx, B->arena, dt, tv)) ||
+        ((rc = up.commit(ctx, B->arena)) ||
          (rc = dalloc(ctx, B->arena, du_, (size_t)nq * M)) || (du && (rc = dalloc(ctx, B->arena, ddu, (size_t)nq * M))))) {
         delete B;
         return rc;
     }
     if (nq > 0) {
         hipError_t e = firk_launch_interp(B->dev, B->firk_s, dqi, dt, du_, ddu, nq, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        if (e == hipSuccess) e = hipMemcpy(u, du_, (size_t)nq * M * sizeof(double), hipMemcpyDeviceToHost);
-        if (e == hipSuccess && du) e = hipMemcpy(du, ddu, (size_t)nq * M * sizeof(double), hipMemcpyDeviceToHost);
         if (e != hipSuccess) { set_err(ctx, "FIRK interpolate: %s", hipGetErrorString(e)); rc = BVP_EHIP; }
+        else rc = fetch_points(ctx, nq, M, du_, u, ddu, du);
     }
     delete B;
     return rc;

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <utility>
@@ -12,6 +14,44 @@
 #include "../../include/bvp_mirk.h"
 #include "mirk_wave.h"
 #include "mlp.h"
+
+// Device blocks of a context that freed arenas leave for later ones (hipMalloc and hipFree
+// cost tens of microseconds each, and a call needs a handful of blocks: a lone pendulum solve
+// takes 0.46 ms, 0.89 ms with some 35 allocations and 17 small uploads per call).  At most kMaxHeld
+// bytes are held, no block above kMaxBlock; the rest, and everything when the context is
+// destroyed, goes back to the device.  All work on pooled memory is enqueued on the
+// context's one stream, so a block handed on is rewritten only after its last reader.
+class DevPool {
+  public:
+    static constexpr size_t kMaxHeld = (size_t)1 << 30, kMaxBlock = (size_t)256 << 20;
+    DevPool() = default;
+    DevPool(const DevPool &) = delete;
+    DevPool &operator=(const DevPool &) = delete;
+    ~DevPool() { close(); }
+    // a block of at least `bytes` (its true size in got), or null
+    void *take(size_t bytes, size_t &got);
+    void give(void *p, size_t bytes);
+    void release();  // frees the held blocks
+    void close();    // release(), and hold nothing from now on
+
+  private:
+    std::mutex mu_;
+    std::multimap<size_t, void *> held_;
+    size_t held_bytes_ = 0;
+    bool closed_ = false;
+};
+
+// Pinned host memory of a context: a small area that uploads and small results are staged
+// in, and two chunks that large results stream through (allocated when first needed).
+struct PinnedStage {
+    static constexpr size_t kSmall = (size_t)1 << 20, kChunk = (size_t)16 << 20;
+    char *small = nullptr, *chunk[2] = {nullptr, nullptr};
+    size_t used = 0;  // of `small`, since the stream was last idle
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    char *take(size_t bytes);  // from `small`; null when it does not fit
+    bool chunks();             // makes sure the large chunks exist
+    void free_all();
+};
 
 struct bvp_ctx {
     int device = 0;
@@ -25,6 +65,8 @@ struct bvp_ctx {
     // device address of the no-allocation entry point's scratch array on this
     // context's device (hipGetSymbolAddress at creation)
     char *noalloc = nullptr;
+    std::shared_ptr<DevPool> pool = std::make_shared<DevPool>();
+    PinnedStage pin;
     // autotuner choices, (M, method, precision, kernel kind (0 wave, 1 block, 2 wave
     // under a global-error controller), family or -1) -> (variant,
     // waves per CU, FP32 records, minimum intervals per lane); later plans of the same
@@ -32,10 +74,14 @@ struct bvp_ctx {
     std::map<std::tuple<int, int, int, int, int>, std::tuple<int, int, int, int>> tuned;
 };
 
-// device allocations owned by one batch; freed together.  In bump mode (bump set)
-// allocations are carved from a region the arena does not own and nothing is freed.
+// device allocations owned by one batch; given back together.  Small allocations share
+// blocks.  In bump mode (bump set) allocations are carved from a region the arena does not
+// own and nothing is freed.
 struct DevArena {
-    std::vector<void *> ptrs;
+    std::shared_ptr<DevPool> pool;
+    std::vector<std::pair<void *, size_t>> blocks;
+    char *cur = nullptr;  // the block small allocations come from
+    size_t cur_left = 0;
     char *bump = nullptr;
     size_t bump_cap = 0, bump_used = 0;
     DevArena() = default;

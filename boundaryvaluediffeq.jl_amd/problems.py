@@ -11,6 +11,7 @@ Problem details are extracted as the reference does in
 ``__extract_problem_details`` / ``__extract_mesh`` / ``__initial_guess_on_mesh``
 (Core/utils.jl:330-388, 694-704, 750-777).
 """
+import ctypes
 from fractions import Fraction
 import inspect
 import math
@@ -208,11 +209,37 @@ class InstanceSpec:
         return s
 
 
+def _struct_dtype(cls):
+    """numpy dtype of a ctypes structure (pointers as addresses), to fill many of them by column."""
+    names = [f[0] for f in cls._fields_]
+    code = {4: "i4", 8: "u8"}
+    formats = ["f8" if t is ctypes.c_double else code[ctypes.sizeof(t)] for _, t in cls._fields_]
+    return np.dtype({"names": names, "formats": formats, "offsets": [getattr(cls, k).offset for k in names],
+                     "itemsize": ctypes.sizeof(cls)})
+
+
+_INSTANCE = _struct_dtype(_abi.Instance)
+
+
+def _addresses(arrays):
+    return [0 if a is None else a.__array_interface__["data"][0] for a in arrays]
+
+
 def instance_array(specs):
-    """ctypes array of ``_abi.Instance`` for a list of specs."""
-    arr = (_abi.Instance * len(specs))()
-    for i, s in enumerate(specs):
-        arr[i] = s.ctypes()
+    """ctypes array of ``_abi.Instance`` for a list of specs (keep them alive)."""
+    n = len(specs)
+    arr = (_abi.Instance * n)()
+    if n < 8:
+        for i, s in enumerate(specs):
+            arr[i] = s.ctypes()
+        return arr
+    v = np.frombuffer(arr, dtype=_INSTANCE, count=n)
+    for k in ("family", "M", "t0", "t1", "bc_kind", "N"):
+        v[k] = [getattr(s, k) for s in specs]
+    v["n_params"] = [s.params.shape[0] for s in specs]
+    v["n_bc"] = [s.bc_t.shape[0] for s in specs]
+    for k in ("params", "bc_t", "bc_comp", "bc_val", "mesh", "guess", "u0"):
+        v[k] = _addresses([getattr(s, k) for s in specs])
     return arr
 
 

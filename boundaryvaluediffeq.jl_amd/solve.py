@@ -205,7 +205,7 @@ class BVPSolution:
         self.prob = prob
         self.alg = alg
         self.t = raw.t
-        self.u = [raw.u[i].copy() for i in range(raw.u.shape[0])]
+        self.u = list(raw.u)  # one array per node (rows of the solution's own copy)
         self.stages = raw.stages  # FIRK: the stage values (N, s, M) of the solution
         self.retcode = _abi.RETCODE_NAMES.get(raw.retcode, str(raw.retcode))
         self.resid = raw.resid_norm
