@@ -1798,7 +1798,7 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
         if (info == BVP_RET_SUCCESS) {
             if (error_norm > B.abstol) {
                 const int Nn =
-                    __builtin_amdgcn_readfirstlane(mesh_select(mesh, N, shat, r1, r2, B.max_sub, mesh_o, lane, sh));
+                    __builtin_amdgcn_readfirstlane(mesh_select(mesh, N, shat, r1, r2, B.max_sub, mesh_o, lane));
                 if (Nn < 0) {
                     info = BVP_RET_FAILURE;
                 } else {

@@ -1262,7 +1262,7 @@ __device__ void bsolve_instance(const BatchDev &B, int b, int tid,
         if (info == BVP_RET_SUCCESS) {
             if (error_norm > B.abstol) {
                 if (tid < WAVE) {
-                    const int n = mesh_select<decltype(sh), WaveSync>(mesh, N, shat, r1, r2, B.max_sub, mesh_o, tid, sh);
+                    const int n = mesh_select<WaveSync>(mesh, N, shat, r1, r2, B.max_sub, mesh_o, tid);
                     if (tid == 0) sh.flag = n;
                 }
                 __syncthreads();
@@ -1415,7 +1415,7 @@ __global__ __launch_bounds__((kBlockWaves<M, LT> * WAVE)) void k_bcomponent(Batc
             __syncthreads();
             double *nm = mesh + B.cap, *ny = y + (size_t)B.cap * M;
             if (tid < WAVE) {
-                const int n = mesh_select<decltype(sh), WaveSync>(mesh, N, shat, df.r1, df.r2, B.max_sub, nm, tid, sh);
+                const int n = mesh_select<WaveSync>(mesh, N, shat, df.r1, df.r2, B.max_sub, nm, tid);
                 if (tid == 0) sh.flag = n;
             }
             __syncthreads();

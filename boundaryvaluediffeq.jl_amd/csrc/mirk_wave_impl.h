@@ -63,6 +63,14 @@ __device__ inline double uniform(double v) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// v of lane l (the same l in all lanes)
+__device__ inline double read_lane(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffLL), l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((unsigned long long)b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // p as a pointer into global memory.  Pointers that reach the compiler as
 // generic (flat) pointers -- read back from a runtime-indexed array, or derived
 // in ways it cannot follow -- compile to flat_* accesses, and the use of any
@@ -1794,9 +1802,9 @@ __device__ inline void half_mesh_into(const double *mesh, int N, double *out, in
 struct BlockSync {
     __device__ void operator()() const { __syncthreads(); }
 };
-template <typename SH, class Sync = BlockSync>
+template <class Sync = BlockSync>
 __device__ inline int mesh_select(const double *mesh, int N, double *shat, double r1, double r2, int max_sub,
-                                  double *new_mesh, int lane, SH &sh, double rho = 1.0) {
+                                  double *new_mesh, int lane, double rho = 1.0) {
     const int n = N;
     const double r3 = r2 / (double)n;
     long long npred = round_even(1.3 * r2 + 1.0);
@@ -1822,36 +1830,44 @@ __device__ inline int mesh_select(const double *mesh, int N, double *shat, doubl
         shat[k] = s;
         acc += s * h;
     }
-    const double zeta = wave_sum(acc) / (double)Ns;
+    const double zeta = uniform(wave_sum(acc) / (double)Ns);
     Sync()();
-    if (lane == 0) {
-        // sequential equidistribution walk (MIRK/adaptivity.jl:254-273)
-        new_mesh[0] = mesh[0];
-        double t = mesh[0], integral = 0.0;
-        int k = 0;
-        long long i = 0;
-        int ok = 1;
-        while (k < n) {
-            const double next_piece = shat[k] * (mesh[k + 1] - t);
-            const double int_next = integral + next_piece;
-            if (int_next > zeta) {
-                const double tn = (zeta - integral) / shat[k] + t;
-                if (i + 1 > Ns) { ok = 0; break; }
-                new_mesh[i + 1] = tn;
-                t = tn;
-                ++i;
-                integral = 0.0;
-            } else {
-                integral = int_next;
-                t = mesh[k + 1];
-                ++k;
-            }
+    // sequential equidistribution walk (MIRK/adaptivity.jl:254-273), the same in all lanes:
+    // 64 intervals at a time in the lanes' registers, read by lane number, so that a step
+    // of the walk waits for arithmetic only (one lane with two dependent loads per step
+    // before: with the transfer's chain below, 512 singular perturbations refined to 152
+    // intervals on average took 743 us in the solve kernel, 416 us now)
+    double t = uniform(mesh[0]), integral = 0.0, sr = 0.0, mr = 0.0;
+    if (lane == 0) new_mesh[0] = t;
+    const int nk = __builtin_amdgcn_readfirstlane(n), Nu = __builtin_amdgcn_readfirstlane((int)Ns);
+    int i = 0;
+    bool ok = true;
+    for (int k = 0, kb = -WAVE; k < nk;) {
+        if (k == kb + WAVE) {
+            kb = k;
+            const int q = min(k + lane, nk - 1);
+            sr = shat[q];
+            mr = mesh[q + 1];
         }
-        new_mesh[Ns] = mesh[n];
-        sh.flag = ok;
+        const double s = read_lane(sr, k - kb), tk = read_lane(mr, k - kb);
+        const double next_piece = s * (tk - t);
+        const double int_next = integral + next_piece;
+        if (int_next > zeta) {
+            const double tn = (zeta - integral) / s + t;
+            if (i + 1 > Nu) { ok = false; break; }
+            if (lane == 0) new_mesh[i + 1] = tn;
+            t = tn;
+            ++i;
+            integral = 0.0;
+        } else {
+            integral = int_next;
+            t = tk;
+            ++k;
+        }
     }
+    if (lane == 0) new_mesh[Ns] = mesh[n];
     Sync()();
-    return sh.flag ? (int)Ns : -1;
+    return ok ? Nu : -1;
 }
 
 // Solution transfer from the old continuous extension to the new nodes
@@ -1892,17 +1908,39 @@ __device__ inline void transfer(const Inst<M> &I, const double *mesh, const doub
         }
     }
     __syncthreads();
-    if (mode == BVP_TRANSFER_REFERENCE && lane == 0) {
-        for (int j = 0; j <= Nn; ++j) {
-            const double iid = iiscr[j];
-            if (iid >= 0.0) {
-                const int ii = (int)iid;
+    if (mode == BVP_TRANSFER_REFERENCE) {
+        // 64 nodes at a time: bases before the block are final; a base within it is taken from
+        // its lane once that is final (each round finishes the first waiting node at least)
+        for (int j0 = 0; j0 <= Nn; j0 += WAVE) {
+            const int j = j0 + lane;
+            const double iid = j <= Nn ? iiscr[j] : -1.0;
+            const bool add = iid >= 0.0;
+            if (wave_any(add)) {
+                const int ii = add ? (int)iid : j0;
+                const int src = max(ii - j0, 0);
+                double v[M];
 #pragma unroll
-                for (int c = 0; c < M; ++c) ny[(size_t)j * M + c] += ny[(size_t)ii * M + c];
+                for (int c = 0; c < M; ++c) v[c] = j <= Nn ? ny[(size_t)j * M + c] : 0.0;
+                if (add && ii < j0)
+#pragma unroll
+                    for (int c = 0; c < M; ++c) v[c] += ny[(size_t)ii * M + c];
+                bool done = !add || ii < j0;
+                for (unsigned long long f = __ballot(done); ~f; f = __ballot(done)) {
+                    const bool go = !done && ((f >> src) & 1);
+#pragma unroll
+                    for (int c = 0; c < M; ++c) {
+                        const double b = __shfl(v[c], src);
+                        if (go) v[c] += b;
+                    }
+                    done |= go;
+                }
+                if (add)
+#pragma unroll
+                    for (int c = 0; c < M; ++c) ny[(size_t)j * M + c] = v[c];
             }
+            __syncthreads();
         }
     }
-    __syncthreads();
 }
 
 // ------------------------------------------------------------------ global error
@@ -2254,7 +2292,7 @@ __device__ __forceinline__ void solve_instance(const BatchDev &B, int b, Shared<
         if (info == BVP_RET_SUCCESS) {
             if (error_norm > B.abstol) {
                 if (cur == 1) bf.m0 = bf.mesh[0];  // buffer 0 receives the new mesh
-                const int Nn = mesh_select(mesh, N, shat, r1, r2, B.max_sub, mesh_o, lane, sh, rho);
+                const int Nn = mesh_select(mesh, N, shat, r1, r2, B.max_sub, mesh_o, lane, rho);
                 if (Nn < 0) {
                     info = BVP_RET_FAILURE;
                 } else {
@@ -2463,7 +2501,7 @@ __global__ __launch_bounds__(64) void k_component(BatchDev B, int op) {
             const double dn = defect_pass<M, METHOD>(I, mesh, y, N, lane, B.abstol, shat, nullptr, r1, r2);
             (void)dn;
             __syncthreads();
-            const int Nn = mesh_select(mesh, N, shat, r1, r2, B.max_sub, bf.mesh[1], lane, sh);
+            const int Nn = mesh_select(mesh, N, shat, r1, r2, B.max_sub, bf.mesh[1], lane);
             if (Nn < 0) {
                 if (lane == 0) { B.iout[(size_t)b * 2] = N; B.iout[(size_t)b * 2 + 1] = BVP_RET_FAILURE; }
             } else {
