@@ -1558,13 +1558,13 @@ int bvp_mlp_gradient(bvp_mlp *m, int32_t n, const float *x, const float *y, floa
     const int tiles = (n + mlp::T - 1) / mlp::T;
     int rc;
     if ((rc = dalloc(ctx, A, dx, (size_t)n * mlp::NIN)) || (rc = dalloc(ctx, A, dy, (size_t)n * mlp::NOUT)) ||
-        (rc = dalloc(ctx, A, dpart, (size_t)tiles * mlp::NSLOT)) || (rc = dalloc(ctx, A, dg, mlp::NSLOT)))
+        (rc = dalloc(ctx, A, dpart, mlp::work_floats(tiles))) || (rc = dalloc(ctx, A, dg, mlp::NPARAM + 1)))
         return rc;
     HIP_TRY(ctx, hipMemcpyAsync(dx, x, sizeof(float) * n * mlp::NIN, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(dy, y, sizeof(float) * n * mlp::NOUT, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, mlp::launch_grad(m->net(), dx, dy, n, dpart, dg, ctx->stream));
-    std::vector<float> h(mlp::NSLOT);
-    HIP_TRY(ctx, hipMemcpyAsync(h.data(), dg, sizeof(float) * mlp::NSLOT, hipMemcpyDeviceToHost, ctx->stream));
+    std::vector<float> h(mlp::NPARAM + 1);
+    HIP_TRY(ctx, hipMemcpyAsync(h.data(), dg, sizeof(float) * h.size(), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     std::memcpy(grad, h.data(), sizeof(float) * mlp::NPARAM);
     if (loss) *loss = h[mlp::NPARAM];
@@ -1627,7 +1627,7 @@ int bvp_mlp_train(bvp_mlp *m, int64_t n, const float *x, const float *y, const b
     const int tiles = o->batch / mlp::T;
     int rc;
     if ((rc = dalloc(ctx, A, dx, (size_t)n * mlp::NIN)) || (rc = dalloc(ctx, A, dy, (size_t)n * mlp::NOUT)) ||
-        (rc = dalloc(ctx, A, dpart, (size_t)tiles * mlp::NSLOT)) || (rc = dalloc(ctx, A, dloss, (size_t)total)) ||
+        (rc = dalloc(ctx, A, dpart, mlp::work_floats(tiles))) || (rc = dalloc(ctx, A, dloss, (size_t)total)) ||
         (rc = upload(ctx, A, dperm, perm)) || (rc = dalloc(ctx, A, dstep, 2)))
         return rc;
     HIP_TRY(ctx, hipMemcpyAsync(dx, x, sizeof(float) * n * mlp::NIN, hipMemcpyHostToDevice, ctx->stream));
@@ -1641,13 +1641,12 @@ int bvp_mlp_train(bvp_mlp *m, int64_t n, const float *x, const float *y, const b
     td.x = dx;
     td.y = dy;
     td.n = n;
-    td.batch_tiles = tiles;
     td.steps_per_epoch = spe;
     td.total_steps = (int)sched;
     td.step0 = (int)step0;
     td.perm = dperm;
     td.step = dstep;
-    td.partial = dpart;
+    td.work = mlp::work_of(dpart, tiles);
     td.loss = dloss;
     td.lr = o->lr;
     td.lr_min = o->lr_min;

@@ -27,9 +27,23 @@ constexpr int OB3 = OW3 + H * H;
 constexpr int OW4 = OB3 + H;
 constexpr int OB4 = OW4 + H * NOUT;
 constexpr int NPARAM = OB4 + NOUT;
-// per-tile partial: gradient, loss at [NPARAM], padded to a multiple of 4 floats
-// so that every slot (and its 16-byte gradient stores) stays 16-byte aligned
-constexpr int NSLOT = (NPARAM + 1 + 3) & ~3;
+// Per-tile slot of a training step: the gradients outside the hidden matrices and the loss.
+constexpr int SB2 = OW2, SB3 = SB2 + H, SW4 = SB3 + H, SB4 = SW4 + H * NOUT, SLOSS = SB4 + NOUT;
+constexpr int NSLOT = (SLOSS + 1 + 63) & ~63;
+// slot index of parameter j (j outside the hidden matrices; j = NPARAM: the loss)
+constexpr int slot_of(int j) { return j < OW2 ? j : j < OW3 ? j - OB2 + SB2 : j - OB3 + SB3; }
+
+// Work area of a gradient over `tiles` tiles: the slots, the hidden matrices' gradients over
+// `splits` ranges of points, and the BF16 operands of these (hidden activations 1 and 2,
+// dL/dz 2 and 3), each [tile][unit][64 points].
+struct Work {
+    float *slots;   // [tiles][NSLOT]
+    float *hidden;  // [splits][2][H * H], input-major
+    uint16_t *act;  // [4][tiles][H][T]
+    int tiles, splits;
+};
+size_t work_floats(int tiles);
+Work work_of(float *base, int tiles);
 
 // Device view of a network.
 struct Net {
@@ -55,12 +69,11 @@ struct TrainDev {
     const float *x;                 // samples [n][NIN] (raw features)
     const float *y;                 // targets [n][NOUT] (raw)
     long long n;
-    int batch_tiles;                // tiles per step
+    Work work;                      // of a step (its tiles are the batch)
     int steps_per_epoch;
     int total_steps;
     const unsigned long long *perm; // per epoch: (a, c) of the index permutation j -> (a j + c) mod n
     int *step;                      // device step counter; step[1]: the step k_adam works on
-    float *partial;                 // [batch_tiles][NSLOT]
     float *loss;                    // [steps of this call], indexed by step - step0
     int step0;                      // first step of this call
     float lr, lr_min, beta1, beta2, eps, weight_decay;
@@ -73,7 +86,7 @@ enum { FEAT_PARAM = 0, FEAT_LOG10_PARAM = 1 };
 hipError_t launch_quantize(const NetBufs &nb, hipStream_t s);
 hipError_t launch_train_step(const NetBufs &nb, const Net &net, const TrainDev &td, hipStream_t s);
 // one forward/backward over n points in order, FP32 gradient (sum over tiles) -> grad[NPARAM], loss -> grad[NPARAM]
-hipError_t launch_grad(const Net &net, const float *x, const float *y, int n, float *partial, float *grad,
+hipError_t launch_grad(const Net &net, const float *x, const float *y, int n, float *work, float *grad,
                        hipStream_t s);
 hipError_t launch_predict(const Net &net, const float *x, int n, float *out, int num_cus, hipStream_t s);
 // The learned guess of a batch (M = 2): the network at every node of the initial

@@ -5,9 +5,10 @@
 // layer live in LDS (about 137 KB), the hidden 256 x 256 products run on the
 // gfx950 matrix cores (v_mfma_f32_16x16x32_bf16, FP32 accumulation; each wave
 // owns 16 output columns of the 64-row tile), the 4-wide input layer and the
-// 2-wide output layer run on the vector ALUs.  Training keeps no activations in
-// HBM: the tile goes forward and backward in the same workgroup and writes its
-// FP32 parameter gradient to a per-tile slot; a second kernel sums the slots,
+// 2-wide output layer run on the vector ALUs.  The tile goes forward and
+// backward in the same workgroup; it writes the small FP32 gradients to a
+// per-tile slot and the BF16 operands of the hidden matrices' gradients, which a
+// second kernel forms over ranges of points; a third one sums slots and ranges,
 // applies Adam to the FP32 master parameters and re-rounds them to BF16 in the
 // two layouts the products read (output-major for the forward pass, input-major
 // for the backward pass).  The step counter lives in device memory so that a
@@ -48,7 +49,8 @@ struct __align__(16) Tile {
 
 // Training runs a tile with 16 waves (TW threads, four per SIMD): a tile is a chain of short
 // phases, each bound by the latency of its LDS and L2 reads, and a batch of 8,192 points has
-// only 128 tiles.  Tile kernel at that batch: 63 us with 4 waves, 48 us with 16.
+// only 128 tiles.  Tile kernel at that batch, the hidden gradients included: 63 us with 4
+// waves, 48 us with 16.
 constexpr int TW = 1024;
 
 // acc[rt] (rows 16rt.., columns 16*wave..) = A (LDS, T x H) times the matrix whose column
@@ -69,48 +71,87 @@ __device__ inline void gemm_tile(const uint16_t *A, const uint16_t *G, int wave,
                 *(const bf8 *)(A + (size_t)(16 * rt + i) * HP + 32 * ks + 8 * g), b[ks], acc[rt], 0, 0, 0);
 }
 
+typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-// eight BF16 values at p[0], p[stride], ..., p[7 stride], packed as one MFMA operand
-__device__ inline bf8 gather8(const uint16_t *p, int stride) {
-    u4 r;
-    r.x = (unsigned)p[0] | ((unsigned)p[stride] << 16);
-    r.y = (unsigned)p[2 * stride] | ((unsigned)p[3 * stride] << 16);
-    r.z = (unsigned)p[4 * stride] | ((unsigned)p[5 * stride] << 16);
-    r.w = (unsigned)p[6 * stride] | ((unsigned)p[7 * stride] << 16);
-    return __builtin_bit_cast(bf8, r);
+// The tile's rows of the operands of k_wgrad: act + array a of tile t, [H][T]
+__device__ inline uint16_t *act_tile(const Work &wk, int a, int t) {
+    return wk.act + ((size_t)a * wk.tiles + t) * (H * T);
+}
+// four consecutive points of a unit
+__device__ inline void store4(uint16_t *p, const uint16_t (&v)[4]) {
+    *(u2 *)p = u2{(unsigned)v[0] | ((unsigned)v[1] << 16), (unsigned)v[2] | ((unsigned)v[3] << 16)};
 }
 
-// dW[k][n] = sum_p Hin[p][k] dz[p][n] for this tile, written input-major (the parameters'
-// order) to part[k*H + n], four consecutive n per lane: one 16-byte store; a wave owns a
-// 64 x 64 block.
-__device__ inline void wgrad_tile(const uint16_t *Hin, const uint16_t *dz, float *part, int wave, int lane) {
-    const int i = lane & 15, g = lane >> 4, n0 = 64 * (wave >> 2), k0 = 64 * (wave & 3);
-    bf8 a[4][2];
+// Gradients of the hidden matrices, dW[k][n] = sum_p h[p][k] dz[p][n]: a workgroup forms
+// a 64 x 64 block of one matrix over one range of the points.  The tile kernel leaves both
+// operands with a unit's points contiguous, which is what an MFMA lane reads (16 bytes);
+// each of the eight waves takes an eighth of the range, four steps of 32 points loaded at
+// once (the loads' latency bounds it), and their sums meet in LDS.  At 8,192 points: tile
+// kernel 35.9 us and 12.2 us here, against 48 us with the products in the tile kernel,
+// which then wrote 0.5 MB of gradient per tile for k_adam to sum (15.3 us; now 6.7 us).
+constexpr int GW = 8;
+__global__ __launch_bounds__(64 * GW) void k_wgrad(Work wk) {
+    __shared__ f4 red[GW][16][64];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    // consecutive workgroups go to different XCDs: with eight ranges, each XCD's L2 holds one
+    const int z = blockIdx.x % wk.splits, x = blockIdx.x / wk.splits;
+    const int k0 = 64 * (x & 3), n0 = 64 * ((x >> 2) & 3), l = x >> 4;
+    const long long steps = 2LL * wk.tiles, parts = (long long)GW * wk.splits, part = (long long)GW * z + wave;
+    const int s0 = (int)(steps * part / parts), s1 = (int)(steps * (part + 1) / parts);
+    f4 acc[4][4];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) a[rt][ks] = gather8(dz + (size_t)(32 * ks + 8 * g) * HP + n0 + 16 * rt + i, HP);
-#pragma unroll 2
-    for (int ct = 0; ct < 4; ++ct) {
-        f4 acc[4];
+        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int s, bf8 (&a)[4], bf8 (&b)[4]) {
+        const int o = 32 * (s & 1) + 8 * g;
+        const uint16_t *hp = act_tile(wk, l, s >> 1) + (k0 + i) * T + o;
+        const uint16_t *dp = act_tile(wk, 2 + l, s >> 1) + (n0 + i) * T + o;
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) acc[rt] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const bf8 b = gather8(Hin + (size_t)(32 * ks + 8 * g) * HP + k0 + 16 * ct + i, HP);
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt)
-                acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt][ks], b, acc[rt], 0, 0, 0);
+        for (int q = 0; q < 4; ++q) {
+            a[q] = *(const bf8 *)(dp + 16 * q * T);
+            b[q] = *(const bf8 *)(hp + 16 * q * T);
         }
-        f4 *dst = (f4 *)(part + (size_t)(k0 + 16 * ct + i) * H + n0 + 4 * g);
+    };
+    auto mul = [&](const bf8 (&a)[4], const bf8 (&b)[4]) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) dst[4 * rt] = acc[rt];
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct)
+                acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], b[ct], acc[rt][ct], 0, 0, 0);
+    };
+    int s = s0;
+    for (; s + 4 <= s1; s += 4) {
+        bf8 a[4][4], b[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load(s + u, a[u], b[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) mul(a[u], b[u]);
+    }
+    for (; s < s1; ++s) {
+        bf8 a[4], b[4];
+        load(s, a, b);
+        mul(a, b);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) red[wave][4 * rt + ct][lane] = acc[rt][ct];
+    __syncthreads();
+    float *out = wk.hidden + ((size_t)z * 2 + l) * (H * H);
+#pragma unroll
+    for (int q = 0; q < 16 / GW; ++q) {
+        const int f = wave * (16 / GW) + q, rt = f / 4, ct = f % 4;
+        f4 v = red[0][f][lane];
+#pragma unroll
+        for (int w = 1; w < GW; ++w) v += red[w][f][lane];
+        *(f4 *)(out + (size_t)(k0 + 16 * ct + i) * H + n0 + 16 * rt + 4 * g) = v;
     }
 }
 
 // Forward pass of the tile (S.x filled): hidden activations into S.h, output into S.out.
-__device__ void forward_tile(Tile &S, const Net &net, int tid) {
+__device__ void forward_tile(Tile &S, const Net &net, int tid, const Work &wk) {
     const int wave = tid >> 6, lane = tid & 63;
     {  // layer 1 (4 -> 256): a thread owns column n and 16 points
         const int n = tid & (H - 1), p0 = (tid / H) * 16;
@@ -118,12 +159,21 @@ __device__ void forward_tile(Tile &S, const Net &net, int tid) {
 #pragma unroll
         for (int i = 0; i < NIN; ++i) w[i] = net.q[OW1 + i * H + n];
         const float b = net.q[OB1 + n];
-#pragma unroll 8
-        for (int p = p0; p < p0 + 16; ++p) {
-            float z = b;
+        uint16_t *act = act_tile(wk, 0, blockIdx.x) + n * T;
 #pragma unroll
-            for (int i = 0; i < NIN; ++i) z += S.x[p][i] * w[i];
-            S.h[0][p][n] = f2bf(tanh_f(z));
+        for (int p1 = 0; p1 < 16; p1 += 8) {
+            uint16_t v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int p = p0 + p1 + e;
+                float z = b;
+#pragma unroll
+                for (int i = 0; i < NIN; ++i) z += S.x[p][i] * w[i];
+                v[e] = f2bf(tanh_f(z));
+                S.h[0][p][n] = v[e];
+            }
+            *(u4 *)(act + p0 + p1) = u4{(unsigned)v[0] | ((unsigned)v[1] << 16), (unsigned)v[2] | ((unsigned)v[3] << 16),
+                                        (unsigned)v[4] | ((unsigned)v[5] << 16), (unsigned)v[6] | ((unsigned)v[7] << 16)};
         }
     }
     __syncthreads();
@@ -135,9 +185,15 @@ __device__ void forward_tile(Tile &S, const Net &net, int tid) {
         const float bn = net.q[(l == 0 ? OB2 : OB3) + n];
         gemm_tile(&S.h[l][0][0], l == 0 ? net.w2f : net.w3f, wave, lane, acc);
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int rt = 0; rt < 4; ++rt) {
+            uint16_t v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) S.h[l + 1][16 * rt + 4 * g + j][n] = f2bf(tanh_f(acc[rt][j] + bn));
+            for (int j = 0; j < 4; ++j) {
+                v[j] = f2bf(tanh_f(acc[rt][j] + bn));
+                S.h[l + 1][16 * rt + 4 * g + j][n] = v[j];
+            }
+            if (l == 0) store4(act_tile(wk, 1, blockIdx.x) + n * T + 16 * rt + 4 * g, v);
+        }
         __syncthreads();
     }
     {  // output layer (256 -> 2): sixteen threads per point, every sixteenth input each
@@ -164,9 +220,10 @@ __device__ void forward_tile(Tile &S, const Net &net, int tid) {
 }
 
 // Backward pass of the tile after forward_tile; inv_b = 1 / (points in the step).
-// Writes the tile's gradient and loss into part[NSLOT].  Sums over the tile's points: four
+// Writes the operands of k_wgrad, and the tile's other gradients and loss into its slot.  Sums over the tile's points: four
 // threads per unit, every fourth point each (pt = 4 it + sub), combined by shuffles.
-__device__ void backward_tile(Tile &S, const Net &net, int tid, float inv_b, float *part) {
+__device__ void backward_tile(Tile &S, const Net &net, int tid, float inv_b, const Work &wk) {
+    float *part = wk.slots + (size_t)blockIdx.x * NSLOT;
     const int wave = tid >> 6, lane = tid & 63;
     const int i = lane & 15, g = lane >> 4;
     const int unit = tid >> 2, sub = tid & 3;
@@ -193,50 +250,62 @@ __device__ void backward_tile(Tile &S, const Net &net, int tid, float inv_b, flo
             for (int o = 0; o < NOUT; ++o) d[o] += __shfl_xor(d[o], m);
         }
         if (p == 0) {
-            part[NPARAM] = l;
+            part[SLOSS] = l;
 #pragma unroll
-            for (int o = 0; o < NOUT; ++o) part[OB4 + o] = d[o];
+            for (int o = 0; o < NOUT; ++o) part[SB4 + o] = d[o];
         }
     }
     __syncthreads();
     {  // output layer: dW4, and dz3 = (dout W4^T) * (1 - h3^2)
         const float w0 = net.q[OW4 + 2 * unit], w1 = net.q[OW4 + 2 * unit + 1];
         float g0 = 0.f, g1 = 0.f;
-#pragma unroll 8
-        for (int it = 0; it < T / 4; ++it) {
-            const int p = 4 * it + sub;
-            const float hk = bf2f(S.h[2][p][unit]);
-            const float d0 = S.out[p][0], d1 = S.out[p][1];
-            g0 += hk * d0;
-            g1 += hk * d1;
-            S.dz[p][unit] = f2bf((d0 * w0 + d1 * w1) * (1.f - hk * hk));
+        // points in fours, so that their dz leave as one store
+        uint16_t *act = act_tile(wk, 3, blockIdx.x) + unit * T;
+#pragma unroll
+        for (int r = 0; r < T / 16; ++r) {
+            uint16_t v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int p = 16 * r + 4 * sub + e;
+                const float hk = bf2f(S.h[2][p][unit]);
+                const float d0 = S.out[p][0], d1 = S.out[p][1];
+                g0 += hk * d0;
+                g1 += hk * d1;
+                v[e] = f2bf((d0 * w0 + d1 * w1) * (1.f - hk * hk));
+                S.dz[p][unit] = v[e];
+            }
+            store4(act + 16 * r + 4 * sub, v);
         }
         g0 = sum4(g0);
         g1 = sum4(g1);
-        if (sub < NOUT) part[OW4 + 2 * unit + sub] = sub == 0 ? g0 : g1;
+        if (sub < NOUT) part[SW4 + 2 * unit + sub] = sub == 0 ? g0 : g1;
     }
     __syncthreads();
 #pragma unroll 1
     for (int l = 1; l >= 0; --l) {  // hidden layer l + 2 (weights W3 for l = 1, W2 for l = 0)
-        wgrad_tile(&S.h[l][0][0], &S.dz[0][0], part + (l == 1 ? OW3 : OW2), wave, lane);
         {
             float s = 0.f;
 #pragma unroll
             for (int it = 0; it < T / 4; ++it) s += bf2f(S.dz[4 * it + sub][unit]);
             s = sum4(s);
-            if (sub == 0) part[(l == 1 ? OB3 : OB2) + unit] = s;
+            if (sub == 0) part[(l == 1 ? SB3 : SB2) + unit] = s;
         }
         f4 acc[4];
         gemm_tile(&S.dz[0][0], l == 1 ? net.w3b : net.w2b, wave, lane, acc);
         __syncthreads();
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int rt = 0; rt < 4; ++rt) {
+            uint16_t v[4];
+            const int k = 16 * wave + i;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int p = 16 * rt + 4 * g + j, k = 16 * wave + i;
+                const int p = 16 * rt + 4 * g + j;
                 const float hk = bf2f(S.h[l][p][k]);
-                S.dz[p][k] = f2bf(acc[rt][j] * (1.f - hk * hk));
+                v[j] = f2bf(acc[rt][j] * (1.f - hk * hk));
+                S.dz[p][k] = v[j];
             }
+            if (l == 1) store4(act_tile(wk, 2, blockIdx.x) + k * T + 16 * rt + 4 * g, v);
+        }
         __syncthreads();
     }
     {  // input layer: dW1, db1
@@ -277,18 +346,18 @@ __global__ __launch_bounds__(TW) void k_train_tile(Net net, TrainDev td) {
     if (blockIdx.x == 0 && tid == 0) td.step[1] = step;  // for k_adam
     const int epoch = step / td.steps_per_epoch, sin = step % td.steps_per_epoch;
     const unsigned long long a = td.perm[2 * epoch], c = td.perm[2 * epoch + 1];
-    const long long bsz = (long long)td.batch_tiles * T;
+    const long long bsz = (long long)td.work.tiles * T;
     if (tid < T) {
         const unsigned long long gidx = (unsigned long long)sin * bsz + (unsigned long long)blockIdx.x * T + tid;
         const long long j = (long long)((a * gidx + c) % (unsigned long long)td.n);
         load_point(S, net, tid, true, td.x + j * NIN, td.y + j * NOUT);
     }
     __syncthreads();
-    forward_tile(S, net, tid);
-    backward_tile(S, net, tid, 1.0f / (float)bsz, td.partial + (size_t)blockIdx.x * NSLOT);
+    forward_tile(S, net, tid, td.work);
+    backward_tile(S, net, tid, 1.0f / (float)bsz, td.work);
 }
 
-__global__ __launch_bounds__(TW) void k_grad_tile(Net net, const float *x, const float *y, int n, float *partial) {
+__global__ __launch_bounds__(TW) void k_grad_tile(Net net, const float *x, const float *y, int n, Work wk) {
     __shared__ Tile S;
     const int tid = threadIdx.x;
     if (tid < T) {
@@ -297,37 +366,54 @@ __global__ __launch_bounds__(TW) void k_grad_tile(Net net, const float *x, const
         load_point(S, net, tid, v, x + (v ? j : 0) * NIN, y + (v ? j : 0) * NOUT);
     }
     __syncthreads();
-    forward_tile(S, net, tid);
-    backward_tile(S, net, tid, 1.0f / (float)n, partial + (size_t)blockIdx.x * NSLOT);
+    forward_tile(S, net, tid, wk);
+    backward_tile(S, net, tid, 1.0f / (float)n, wk);
 }
 
-// Sum over the per-tile gradient slots of value j = 256 blockIdx + threadIdx (gradient at
-// [0, NPARAM), the loss at NPARAM), in a fixed order (the same bits on every run).  Each of
-// the block's four waves sums a quarter of the slots for all 256 values, 16 bytes per lane
-// and eight loads in flight (with 4 bytes per lane the bytes in flight bounded the sum).
-// k_adam over 128 slots (68 MB): 21.7 us and a counter kernel of 4.1 us before, 15.3 us
-// (4.5 TB/s) with the slots in the parameters' order.
-__device__ inline float sum_slots(const float *partial, int tiles) {
+// Gradient of parameter j = 256 blockIdx + threadIdx (the loss for j = NPARAM): the sum over
+// the tiles' slots, or over the ranges for the hidden matrices, in a fixed order (the same
+// bits on every run).  Each of the block's four waves sums a quarter for all 256 values, 16
+// bytes per lane and sixteen loads in flight.
+__device__ inline float sum_grad(const Work &wk) {
+    static_assert(OW2 % 256 == 0 && OB2 % 256 == 0 && OW3 % 256 == 0 && OB3 % 256 == 0 && (H * H) % 256 == 0,
+                  "a block of 256 parameters lies within a hidden matrix or outside");
     __shared__ f4 red[4][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int j4 = blockIdx.x * 256 + 4 * lane;
-    const int per = (tiles + 3) / 4, t0 = min(tiles, wave * per), t1 = min(tiles, t0 + per);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j0 = blockIdx.x * 256;
+    const bool w2 = j0 >= OW2 && j0 < OB2, w3 = j0 >= OW3 && j0 < OB3;
+    const float *src;
+    int cnt, stride;
+    bool in = true;
+    if (w2 || w3) {
+        src = wk.hidden + (w2 ? j0 - OW2 : H * H + j0 - OW3) + 4 * lane;
+        cnt = wk.splits;
+        stride = 2 * H * H;
+    } else {
+        src = wk.slots + slot_of(j0) + 4 * lane;
+        in = slot_of(j0) + 4 * lane < NSLOT;
+        cnt = wk.tiles;
+        stride = NSLOT;
+    }
+    const int per = (cnt + 3) / 4, t0 = min(cnt, wave * per), t1 = min(cnt, t0 + per);
     f4 s = f4{0.f, 0.f, 0.f, 0.f};
-    if (j4 < NSLOT) {
-        const float *src = partial + j4;
-        f4 a[8];
+    if (in) {
+        constexpr int U = 16;
+        f4 a[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] = s;
-        int t = t0;
-        for (; t + 8 <= t1; t += 8) {
-            f4 v[8];
+        for (int u = 0; u < U; ++u) a[u] = s;
+        for (int t = t0; t < t1; t += U) {
+            f4 v[U];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = *(const f4 *)(src + (size_t)(t + u) * NSLOT);
+            for (int u = 0; u < U; ++u)
+                if (t + u < t1) v[u] = *(const f4 *)(src + (size_t)(t + u) * stride);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) a[u] += v[u];
+            for (int u = 0; u < U; ++u)
+                if (t + u < t1) a[u] += v[u];
         }
-        for (; t < t1; ++t) a[0] += *(const f4 *)(src + (size_t)t * NSLOT);
-        s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+#pragma unroll
+        for (int o = U / 2; o > 0; o /= 2)
+#pragma unroll
+            for (int u = 0; u < o; ++u) a[u] += a[u + o];
+        s = a[0];
     }
     red[wave][lane] = s;
     __syncthreads();
@@ -335,8 +421,8 @@ __device__ inline float sum_slots(const float *partial, int tiles) {
     return (r[0] + r[256]) + (r[512] + r[768]);
 }
 
-__global__ __launch_bounds__(256) void k_sum_slots(const float *partial, int tiles, float *grad) {
-    const float g = sum_slots(partial, tiles);
+__global__ __launch_bounds__(256) void k_sum_grad(Work wk, float *grad) {
+    const float g = sum_grad(wk);
     const int j = blockIdx.x * 256 + threadIdx.x;
     if (j <= NPARAM) grad[j] = g;
 }
@@ -366,8 +452,14 @@ __global__ void k_quantize(NetBufs nb) {
 // step[0], which nothing else reads meanwhile.
 __global__ __launch_bounds__(256) void k_adam(NetBufs nb, TrainDev td) {
     const int step = td.step[1];
-    const float g = sum_slots(td.partial, td.batch_tiles);
     const int j = blockIdx.x * 256 + threadIdx.x;
+    float m = 0.f, v = 0.f, w = 0.f;  // read before the sums, so that one wait covers both
+    if (j < NPARAM) {
+        m = nb.m[j];
+        v = nb.v[j];
+        w = nb.w[j];
+    }
+    const float g = sum_grad(td.work);
     if (j > NPARAM) return;
     if (j == NPARAM) {
         td.loss[step - td.step0] = g;
@@ -381,11 +473,10 @@ __global__ __launch_bounds__(256) void k_adam(NetBufs nb, TrainDev td) {
         lr = td.lr_min + 0.5f * (td.lr - td.lr_min) * (1.f + cosf(3.14159265358979f * fminf(f, 1.f)));
     }
     const float t = (float)(step + 1);
-    const float m = nb.m[j] = td.beta1 * nb.m[j] + (1.f - td.beta1) * g;
-    const float v = nb.v[j] = td.beta2 * nb.v[j] + (1.f - td.beta2) * g * g;
+    m = nb.m[j] = td.beta1 * m + (1.f - td.beta1) * g;
+    v = nb.v[j] = td.beta2 * v + (1.f - td.beta2) * g * g;
     const float mh = m / (1.f - powf(td.beta1, t)), vh = v / (1.f - powf(td.beta2, t));
     const bool matrix = (j < OB1) || (j >= OW2 && j < OB2) || (j >= OW3 && j < OB3) || (j >= OW4 && j < OB4);
-    float w = nb.w[j];
     if (matrix) w -= lr * td.weight_decay * w;
     w -= lr * mh / (sqrtf(vh) + td.eps);
     nb.w[j] = w;
@@ -634,17 +725,39 @@ hipError_t launch_quantize(const NetBufs &nb, hipStream_t s) {
     return hipGetLastError();
 }
 
+// ranges of points of the hidden matrices' gradients: sixteen tiles each at least, so that a
+// wave of k_wgrad has its four steps, and at most eight (8 x 32 blocks fill the chip)
+static int splits_of(int tiles) { return tiles < 16 ? 1 : tiles < 128 ? tiles / 16 : 8; }
+
+size_t work_floats(int tiles) {
+    return (size_t)tiles * NSLOT + (size_t)splits_of(tiles) * 2 * H * H + (size_t)tiles * (4 * H * T / 2);
+}
+
+Work work_of(float *base, int tiles) {
+    Work w;
+    w.tiles = tiles;
+    w.splits = splits_of(tiles);
+    w.slots = base;
+    w.hidden = base + (size_t)tiles * NSLOT;
+    w.act = (uint16_t *)(w.hidden + (size_t)w.splits * 2 * H * H);
+    return w;
+}
+
+constexpr int kGradBlocks = (NPARAM + 1 + 255) / 256;
+
 hipError_t launch_train_step(const NetBufs &nb, const Net &net, const TrainDev &td, hipStream_t s) {
-    k_train_tile<<<td.batch_tiles, TW, 0, s>>>(net, td);
-    k_adam<<<(NSLOT + 255) / 256, 256, 0, s>>>(nb, td);
+    k_train_tile<<<td.work.tiles, TW, 0, s>>>(net, td);
+    k_wgrad<<<32 * td.work.splits, 64 * GW, 0, s>>>(td.work);
+    k_adam<<<kGradBlocks, 256, 0, s>>>(nb, td);
     return hipGetLastError();
 }
 
-hipError_t launch_grad(const Net &net, const float *x, const float *y, int n, float *partial, float *grad,
+hipError_t launch_grad(const Net &net, const float *x, const float *y, int n, float *work, float *grad,
                        hipStream_t s) {
-    const int tiles = (n + T - 1) / T;
-    k_grad_tile<<<tiles, TW, 0, s>>>(net, x, y, n, partial);
-    k_sum_slots<<<(NSLOT + 255) / 256, 256, 0, s>>>(partial, tiles, grad);
+    const Work wk = work_of(work, (n + T - 1) / T);
+    k_grad_tile<<<wk.tiles, TW, 0, s>>>(net, x, y, n, wk);
+    k_wgrad<<<32 * wk.splits, 64 * GW, 0, s>>>(wk);
+    k_sum_grad<<<kGradBlocks, 256, 0, s>>>(wk, grad);
     return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 """The network kernels at the edges of their tiles: gradients over tile counts around the
 four quarters in which the per-tile slots are summed (fewer tiles than quarters, uneven
-quarters, more than eight slots per quarter), predictions of one point, around a tile of 64,
+quarters, more than sixteen slots per quarter) and around the ranges of points of the hidden
+matrices' gradients (fewer steps than waves, one, two and eight ranges, uneven), predictions of one point, around a tile of 64,
 and with more than eight tiles per workgroup (two rounds of features read ahead).
 
 Tolerances: as tests/test_gpu_mlp.py -- outputs 5e-3 and gradients 1e-2 relative (FP32
@@ -18,7 +19,7 @@ from test_gpu_mlp import _net
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 63, 65, 3 * 64, 5 * 64, 33 * 64 + 5, 35 * 64])
+@pytest.mark.parametrize("n", [1, 63, 65, 3 * 64, 5 * 64, 33 * 64 + 5, 35 * 64, 130 * 64 + 1])
 def test_gradient_slots(n):
     print("mlp gradient slots", n, flush=True)
     sys.stdout.flush()
