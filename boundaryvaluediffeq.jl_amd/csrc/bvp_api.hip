@@ -215,6 +215,7 @@ int fetch(bvp_ctx *ctx, const std::vector<Pieces> &ps, bool pinned) {
             if (hi > lo) k.p->scatter(k.a + lo, k.a + hi, src + lo);
         };
         std::vector<std::thread> th;
+        th.reserve(nt);
         int t = 1;
         if (len > PinnedStage::kSmall) {
             try {
