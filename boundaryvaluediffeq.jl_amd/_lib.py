@@ -3,6 +3,7 @@
 missing GPU raises."""
 import ctypes as C
 import pathlib
+import threading
 
 import numpy as np
 
@@ -109,15 +110,17 @@ class Context:
 
     def __init__(self, device=0):
         self._h = C.c_void_p()
+        self._lock = threading.RLock()  # re-entered where a finalizer runs between two calls
         rc = lib().bvp_ctx_create(device, C.byref(self._h))
         if rc != 0:
             raise BVPError(f"bvp_ctx_create(device={device}) failed with {rc} (no usable GPU?)")
         self.device = device
 
     def close(self):
-        if self._h:
-            lib().bvp_ctx_destroy(self._h)
-            self._h = C.c_void_p()
+        with self._lock:
+            if self._h:
+                lib().bvp_ctx_destroy(self._h)
+                self._h = C.c_void_p()
 
     def __del__(self):
         try:
@@ -129,6 +132,15 @@ class Context:
     def handle(self):
         return self._h
 
+    def call(self, name, *args):
+        """``lib().name(*args)``, one call of the context at a time: a C context serves one host
+        thread (a call in progress owns its stream's events, staging memory and error text), and
+        Python threads share the default contexts.  Raises on an error code."""
+        with self._lock:
+            rc = getattr(lib(), name)(*args)
+            if rc is not None:
+                self.check(rc, name.removeprefix("bvp_").removeprefix("mirk_"))
+
     def check(self, rc, what):
         if rc != 0:
             msg = lib().bvp_last_error(self._h)
@@ -136,12 +148,14 @@ class Context:
 
 
 _ctx = {}
+_ctx_lock = threading.Lock()
 
 
 def context(device=0):
-    if device not in _ctx:
-        _ctx[device] = Context(device)
-    return _ctx[device]
+    with _ctx_lock:
+        if device not in _ctx:
+            _ctx[device] = Context(device)
+        return _ctx[device]
 
 
 def _nodes(specs):
@@ -153,7 +167,7 @@ def residual(ctx, method, specs):
     M = specs[0].M
     tot = sum(_nodes(specs)) * M
     out = np.zeros(tot)
-    ctx.check(lib().bvp_mirk_residual(ctx.handle, method, len(specs), arr, out.ctypes.data_as(_dp)), "residual")
+    ctx.call("bvp_mirk_residual", ctx.handle, method, len(specs), arr, out.ctypes.data_as(_dp))
     res, o = [], 0
     for s in specs:
         k = M * (s.N + 1)
@@ -169,8 +183,8 @@ def jacobian_blocks(ctx, method, specs):
     S = np.zeros(nint * M * M)
     R = np.zeros(nint * M * M)
     node = np.zeros(len(specs) * M, dtype=np.int32)
-    ctx.check(lib().bvp_mirk_jacobian_blocks(ctx.handle, method, len(specs), arr, S.ctypes.data_as(_dp),
-                                             R.ctypes.data_as(_dp), node.ctypes.data_as(_ip)), "jacobian_blocks")
+    ctx.call("bvp_mirk_jacobian_blocks", ctx.handle, method, len(specs), arr, S.ctypes.data_as(_dp),
+             R.ctypes.data_as(_dp), node.ctypes.data_as(_ip))
     out, o = [], 0
     for i, s in enumerate(specs):
         k = s.N * M * M
@@ -184,8 +198,8 @@ def newton_step(ctx, method, specs, precision=_abi.PREC_FP64, refine_iters=0):
     arr = instance_array(specs)
     M = specs[0].M
     out = np.zeros(sum(_nodes(specs)) * M)
-    ctx.check(lib().bvp_mirk_newton_step(ctx.handle, method, precision, refine_iters, len(specs), arr,
-                                         out.ctypes.data_as(_dp)), "newton_step")
+    ctx.call("bvp_mirk_newton_step", ctx.handle, method, precision, refine_iters, len(specs), arr,
+             out.ctypes.data_as(_dp))
     res, o = [], 0
     for s in specs:
         k = M * (s.N + 1)
@@ -200,8 +214,8 @@ def defect(ctx, method, specs):
     nint = sum(s.N for s in specs)
     err = np.zeros(nint * M)
     dn = np.zeros(len(specs))
-    ctx.check(lib().bvp_mirk_defect(ctx.handle, method, len(specs), arr, err.ctypes.data_as(_dp),
-                                    dn.ctypes.data_as(_dp)), "defect")
+    ctx.call("bvp_mirk_defect", ctx.handle, method, len(specs), arr, err.ctypes.data_as(_dp),
+             dn.ctypes.data_as(_dp))
     out, o = [], 0
     for i, s in enumerate(specs):
         out.append((err[o:o + s.N * M].reshape(s.N, M).copy(), float(dn[i])))
@@ -216,8 +230,8 @@ def global_error(ctx, opts, specs):
     M = specs[0].M
     err = np.zeros(sum(s.N for s in specs) * M)
     nrm = np.zeros(len(specs))
-    ctx.check(lib().bvp_mirk_global_error(ctx.handle, C.byref(opts), len(specs), arr, err.ctypes.data_as(_dp),
-                                          nrm.ctypes.data_as(_dp)), "global_error")
+    ctx.call("bvp_mirk_global_error", ctx.handle, C.byref(opts), len(specs), arr, err.ctypes.data_as(_dp),
+             nrm.ctypes.data_as(_dp))
     out, o = [], 0
     for i, s in enumerate(specs):
         out.append((err[o:o + s.N * M].reshape(s.N, M).copy(), float(nrm[i])))
@@ -235,9 +249,9 @@ def interpolate(ctx, method, specs, tvals, derivative=True):
     tt = np.concatenate(ts) if len(ts) else np.zeros(0)
     u = np.zeros(max(1, len(tt)) * M)
     du = np.zeros(max(1, len(tt)) * M) if derivative else None
-    ctx.check(lib().bvp_mirk_interpolate(ctx.handle, method, len(specs), arr, nt.ctypes.data_as(_ip),
-                                         tt.ctypes.data_as(_dp), u.ctypes.data_as(_dp),
-                                         du.ctypes.data_as(_dp) if derivative else _dp()), "interpolate")
+    ctx.call("bvp_mirk_interpolate", ctx.handle, method, len(specs), arr, nt.ctypes.data_as(_ip),
+             tt.ctypes.data_as(_dp), u.ctypes.data_as(_dp),
+             du.ctypes.data_as(_dp) if derivative else _dp())
     out, o = [], 0
     for k in nt:
         out.append((u[o * M:(o + k) * M].reshape(k, M).copy(),
@@ -255,9 +269,9 @@ def mesh_select(ctx, opts, specs, capacity=None):
     info = np.zeros(n, dtype=np.int32)
     nm = np.zeros(n * cap)
     ny = np.zeros(n * cap * M)
-    ctx.check(lib().bvp_mirk_mesh_select(ctx.handle, C.byref(opts), n, arr, cap, nN.ctypes.data_as(_ip),
-                                         info.ctypes.data_as(_ip), nm.ctypes.data_as(_dp),
-                                         ny.ctypes.data_as(_dp)), "mesh_select")
+    ctx.call("bvp_mirk_mesh_select", ctx.handle, C.byref(opts), n, arr, cap, nN.ctypes.data_as(_ip),
+             info.ctypes.data_as(_ip), nm.ctypes.data_as(_dp),
+             ny.ctypes.data_as(_dp))
     out = []
     for i in range(n):
         k = int(nN[i])
@@ -286,9 +300,9 @@ def firk_residual(ctx, method, specs, stages=None):
     arr = instance_array(specs)
     st = _firk_stages_arg(method, specs, stages)
     out = np.zeros(sum(_nx(method, s) for s in specs))
-    ctx.check(lib().bvp_firk_residual(ctx.handle, method, len(specs), arr,
-                                      st.ctypes.data_as(_dp) if st is not None else _dp(),
-                                      out.ctypes.data_as(_dp)), "firk_residual")
+    ctx.call("bvp_firk_residual", ctx.handle, method, len(specs), arr,
+             st.ctypes.data_as(_dp) if st is not None else _dp(),
+             out.ctypes.data_as(_dp))
     res, o = [], 0
     for s in specs:
         k = _nx(method, s)
@@ -301,9 +315,9 @@ def firk_newton_step(ctx, method, specs, stages=None):
     arr = instance_array(specs)
     st = _firk_stages_arg(method, specs, stages)
     out = np.zeros(sum(_nx(method, s) for s in specs))
-    ctx.check(lib().bvp_firk_newton_step(ctx.handle, method, len(specs), arr,
-                                         st.ctypes.data_as(_dp) if st is not None else _dp(),
-                                         out.ctypes.data_as(_dp)), "firk_newton_step")
+    ctx.call("bvp_firk_newton_step", ctx.handle, method, len(specs), arr,
+             st.ctypes.data_as(_dp) if st is not None else _dp(),
+             out.ctypes.data_as(_dp))
     res, o = [], 0
     for s in specs:
         k = _nx(method, s)
@@ -318,9 +332,9 @@ def firk_defect(ctx, method, specs, stages=None):
     M = specs[0].M
     err = np.zeros(sum(s.N for s in specs) * M)
     dn = np.zeros(len(specs))
-    ctx.check(lib().bvp_firk_defect(ctx.handle, method, len(specs), arr,
-                                    st.ctypes.data_as(_dp) if st is not None else _dp(),
-                                    err.ctypes.data_as(_dp), dn.ctypes.data_as(_dp)), "firk_defect")
+    ctx.call("bvp_firk_defect", ctx.handle, method, len(specs), arr,
+             st.ctypes.data_as(_dp) if st is not None else _dp(),
+             err.ctypes.data_as(_dp), dn.ctypes.data_as(_dp))
     out, o = [], 0
     for i, s in enumerate(specs):
         out.append((err[o:o + s.N * M].reshape(s.N, M).copy(), float(dn[i])))
@@ -337,10 +351,10 @@ def firk_interpolate(ctx, method, specs, tvals, stages=None, derivative=True):
     tt = np.concatenate(ts) if len(ts) else np.zeros(0)
     u = np.zeros(max(1, len(tt)) * M)
     du = np.zeros(max(1, len(tt)) * M) if derivative else None
-    ctx.check(lib().bvp_firk_interpolate(ctx.handle, method, len(specs), arr,
-                                         st.ctypes.data_as(_dp) if st is not None else _dp(),
-                                         nt.ctypes.data_as(_ip), tt.ctypes.data_as(_dp), u.ctypes.data_as(_dp),
-                                         du.ctypes.data_as(_dp) if derivative else _dp()), "firk_interpolate")
+    ctx.call("bvp_firk_interpolate", ctx.handle, method, len(specs), arr,
+             st.ctypes.data_as(_dp) if st is not None else _dp(),
+             nt.ctypes.data_as(_ip), tt.ctypes.data_as(_dp), u.ctypes.data_as(_dp),
+             du.ctypes.data_as(_dp) if derivative else _dp())
     out, o = [], 0
     for k in nt:
         out.append((u[o * M:(o + k) * M].reshape(k, M).copy(),
@@ -351,7 +365,7 @@ def firk_interpolate(ctx, method, specs, tvals, stages=None, derivative=True):
 
 def copy_probe(ctx, nbytes, repeats=3):
     ms = C.c_float()
-    ctx.check(lib().bvp_copy_probe(ctx.handle, int(nbytes), int(repeats), C.byref(ms)), "copy_probe")
+    ctx.call("bvp_copy_probe", ctx.handle, int(nbytes), int(repeats), C.byref(ms))
     return float(ms.value)
 
 
@@ -410,7 +424,7 @@ def solve_batch(ctx, opts, specs):
     cap = max(opts.max_num_subintervals, max(s.N for s in specs)) + 1
     st = _abi.firk_stages(opts.method) if _abi.is_firk(opts.method) else 0
     res, bufs = _result_array(specs, cap, st)
-    ctx.check(lib().bvp_mirk_solve_batch(ctx.handle, C.byref(opts), len(specs), arr, res), "solve_batch")
+    ctx.call("bvp_mirk_solve_batch", ctx.handle, C.byref(opts), len(specs), arr, res)
     return _raws(res, specs, bufs, st)
 
 
@@ -421,8 +435,7 @@ def solve_batch_noalloc(ctx, opts, specs):
     cap = max(opts.max_num_subintervals, max(s.N for s in specs)) + 1
     st = _abi.firk_stages(opts.method) if _abi.is_firk(opts.method) else 0
     res, bufs = _result_array(specs, cap, st)
-    ctx.check(lib().bvp_mirk_solve_batch_noalloc(ctx.handle, C.byref(opts), len(specs), arr, res),
-              "solve_batch_noalloc")
+    ctx.call("bvp_mirk_solve_batch_noalloc", ctx.handle, C.byref(opts), len(specs), arr, res)
     return _raws(res, specs, bufs, st)
 
 
@@ -435,22 +448,21 @@ class Batch:
         self.opts = opts
         self._arr = instance_array(specs)
         self._h = C.c_void_p()
-        ctx.check(lib().bvp_batch_create(ctx.handle, C.byref(opts), len(specs), self._arr, C.byref(self._h)),
-                  "batch_create")
+        ctx.call("bvp_batch_create", ctx.handle, C.byref(opts), len(specs), self._arr, C.byref(self._h))
 
     def run(self):
-        self.ctx.check(lib().bvp_batch_run(self.ctx.handle, self._h), "batch_run")
+        self.ctx.call("bvp_batch_run", self.ctx.handle, self._h)
 
     def sync(self):
         ms = C.c_float()
-        self.ctx.check(lib().bvp_batch_sync(self.ctx.handle, self._h, C.byref(ms)), "batch_sync")
+        self.ctx.call("bvp_batch_sync", self.ctx.handle, self._h, C.byref(ms))
         return float(ms.value)
 
     def results(self):
         cap = max(self.opts.max_num_subintervals, max(s.N for s in self.specs)) + 1
         st = _abi.firk_stages(self.opts.method) if _abi.is_firk(self.opts.method) else 0
         res, bufs = _result_array(self.specs, cap, st)
-        self.ctx.check(lib().bvp_batch_results(self.ctx.handle, self._h, res), "batch_results")
+        self.ctx.call("bvp_batch_results", self.ctx.handle, self._h, res)
         return _raws(res, self.specs, bufs, st)
 
     def learned_guess(self):
@@ -458,8 +470,7 @@ class Batch:
         M = self.specs[0].M
         tot = sum(s.N + 1 for s in self.specs)
         y = np.zeros(tot * M)
-        self.ctx.check(lib().bvp_batch_learned_guess(self.ctx.handle, self._h, y.ctypes.data_as(_dp)),
-                       "batch_learned_guess")
+        self.ctx.call("bvp_batch_learned_guess", self.ctx.handle, self._h, y.ctypes.data_as(_dp))
         out, o = [], 0
         for s in self.specs:
             out.append(y[o * M:(o + s.N + 1) * M].reshape(s.N + 1, M).copy())
@@ -471,12 +482,12 @@ class Batch:
         device ms of every candidate and the chosen (variant, persistent waves)."""
         ms = np.zeros(16, np.float32)
         n = C.c_int32()
-        self.ctx.check(lib().bvp_batch_autotune(self.ctx.handle, self._h, repeats, ms.ctypes.data_as(_fp),
-                                                C.byref(n)), "batch_autotune")
+        self.ctx.call("bvp_batch_autotune", self.ctx.handle, self._h, repeats, ms.ctypes.data_as(_fp),
+                      C.byref(n))
         return [float(x) for x in ms[:n.value]], self.config()
 
     def set_config(self, variant, blocks):
-        self.ctx.check(lib().bvp_batch_set_config(self.ctx.handle, self._h, variant, blocks), "batch_set_config")
+        self.ctx.call("bvp_batch_set_config", self.ctx.handle, self._h, variant, blocks)
 
     def config(self):
         v, b = C.c_int32(), C.c_int32()
@@ -518,13 +529,11 @@ class Batch:
         points per instance and Hermite interpolation, or at every node for 0)."""
         self._net = net
         h = net.handle if net is not None else C.c_void_p()
-        rc = lib().bvp_batch_set_warm_start(self._h, h, feature_kind, anchors)
-        if rc != 0:
-            raise BVPError(f"batch_set_warm_start failed ({rc}): {lib().bvp_last_error(self.ctx.handle).decode()}")
+        self.ctx.call("bvp_batch_set_warm_start", self._h, h, feature_kind, anchors)
 
     def counters(self):
         c = (C.c_longlong * 4)()
-        self.ctx.check(lib().bvp_batch_counters(self.ctx.handle, self._h, c), "batch_counters")
+        self.ctx.call("bvp_batch_counters", self.ctx.handle, self._h, c)
         return [int(x) for x in c]
 
     def info(self):
@@ -534,7 +543,7 @@ class Batch:
 
     def close(self):
         if self._h:
-            lib().bvp_batch_destroy(self._h)
+            self.ctx.call("bvp_batch_destroy", self._h)
             self._h = C.c_void_p()
 
     def __del__(self):
@@ -560,7 +569,7 @@ class MLP:
     def __init__(self, ctx, seed=1):
         self.ctx = ctx
         self._h = C.c_void_p()
-        ctx.check(lib().bvp_mlp_create(ctx.handle, C.c_uint64(seed), C.byref(self._h)), "mlp_create")
+        ctx.call("bvp_mlp_create", ctx.handle, C.c_uint64(seed), C.byref(self._h))
         self.norm = (np.zeros(4, np.float32), np.ones(4, np.float32), np.zeros(2, np.float32),
                      np.ones(2, np.float32))
 
@@ -570,33 +579,31 @@ class MLP:
 
     def set_normalization(self, in_shift, in_scale, out_shift, out_scale):
         v = [_f32(in_shift, 4), _f32(in_scale, 4), _f32(out_shift, 2), _f32(out_scale, 2)]
-        self.ctx.check(lib().bvp_mlp_set_normalization(self._h, *[a.ctypes.data_as(_fp) for a in v]),
-                       "mlp_set_normalization")
+        self.ctx.call("bvp_mlp_set_normalization", self._h, *[a.ctypes.data_as(_fp) for a in v])
         self.norm = tuple(v)
 
     def params(self):
         w = np.zeros(self.NPARAM, np.float32)
-        self.ctx.check(lib().bvp_mlp_get_params(self._h, w.ctypes.data_as(_fp)), "mlp_get_params")
+        self.ctx.call("bvp_mlp_get_params", self._h, w.ctypes.data_as(_fp))
         return w
 
     def set_params(self, w):
         w = _f32(w, self.NPARAM)
-        self.ctx.check(lib().bvp_mlp_set_params(self._h, w.ctypes.data_as(_fp)), "mlp_set_params")
+        self.ctx.call("bvp_mlp_set_params", self._h, w.ctypes.data_as(_fp))
 
     def gradient(self, x, y):
         x = _f32(x).reshape(-1, 4)
         y = _f32(y).reshape(-1, 2)
         g = np.zeros(self.NPARAM, np.float32)
         loss = C.c_float()
-        self.ctx.check(lib().bvp_mlp_gradient(self._h, len(x), x.ctypes.data_as(_fp), y.ctypes.data_as(_fp),
-                                              g.ctypes.data_as(_fp), C.byref(loss)), "mlp_gradient")
+        self.ctx.call("bvp_mlp_gradient", self._h, len(x), x.ctypes.data_as(_fp), y.ctypes.data_as(_fp),
+                      g.ctypes.data_as(_fp), C.byref(loss))
         return float(loss.value), g
 
     def predict(self, x):
         x = _f32(x).reshape(-1, 4)
         y = np.zeros((len(x), 2), np.float32)
-        self.ctx.check(lib().bvp_mlp_predict(self._h, len(x), x.ctypes.data_as(_fp), y.ctypes.data_as(_fp)),
-                       "mlp_predict")
+        self.ctx.call("bvp_mlp_predict", self._h, len(x), x.ctypes.data_as(_fp), y.ctypes.data_as(_fp))
         return y
 
     def train(self, x, y, epochs=10, batch=8192, lr=2e-3, lr_min=2e-5, weight_decay=0.0, warmup=100, seed=7,
@@ -611,14 +618,13 @@ class MLP:
         loss = np.zeros(max(nsteps, 1), np.float32)
         steps = C.c_int32()
         ms = C.c_float()
-        self.ctx.check(lib().bvp_mlp_train(self._h, len(x), x.ctypes.data_as(_fp), y.ctypes.data_as(_fp),
-                                           C.byref(o), loss.ctypes.data_as(_fp), C.byref(steps), C.byref(ms)),
-                       "mlp_train")
+        self.ctx.call("bvp_mlp_train", self._h, len(x), x.ctypes.data_as(_fp), y.ctypes.data_as(_fp),
+                      C.byref(o), loss.ctypes.data_as(_fp), C.byref(steps), C.byref(ms))
         return loss[:steps.value], float(ms.value)
 
     def close(self):
         if self._h:
-            lib().bvp_mlp_destroy(self._h)
+            self.ctx.call("bvp_mlp_destroy", self._h)
             self._h = C.c_void_p()
 
     def __del__(self):
