@@ -74,13 +74,14 @@ void *arena_bytes(bvp_ctx *ctx, DevArena &arena, size_t count) {
         size_t got = 0;
         const bool own = bytes > kShared / 4;
         void *q = arena.pool->take(own ? bytes : kShared, got);
+        const bool shared = q && !own;
+        if (!q && !own) q = arena.pool->take(bytes, got);  // no room for a shared block
         if (!q) {
-            set_err(ctx, "hipMalloc(%zu bytes) failed: out of memory", own ? bytes : kShared);
-            (void)hipGetLastError();
+            set_err(ctx, "hipMalloc(%zu bytes) failed: out of memory", bytes);
             return nullptr;
         }
         arena.blocks.emplace_back(q, got);
-        if (own) return q;
+        if (!shared) return q;
         arena.cur = (char *)q;
         arena.cur_left = got;
     }
@@ -234,60 +235,6 @@ int fetch(bvp_ctx *ctx, const std::vector<Pieces> &ps, bool pinned) {
 
 DevArena::~DevArena() {
     for (auto &b : blocks) pool->give(b.first, b.second);
-}
-
-void *DevPool::take(size_t bytes, size_t &got) {
-    // sizes in steps of an eighth of their power of two, so that blocks of nearly the same
-    // calls fit each other
-    size_t step = 4096;
-    while (step * 16 < bytes) step *= 2;
-    got = (bytes + step - 1) / step * step;
-    {
-        std::lock_guard<std::mutex> g(mu_);
-        auto it = held_.lower_bound(got);
-        if (it != held_.end() && it->first <= got + got / 4) {
-            void *p = it->second;
-            got = it->first;
-            held_bytes_ -= got;
-            held_.erase(it);
-            return p;
-        }
-    }
-    void *q = nullptr;
-    if (hipMalloc(&q, got) == hipSuccess) return q;
-    release();  // the held blocks may be what is missing
-    (void)hipGetLastError();
-    return hipMalloc(&q, got) == hipSuccess ? q : nullptr;
-}
-
-void DevPool::give(void *p, size_t bytes) {
-    {
-        std::lock_guard<std::mutex> g(mu_);
-        if (!closed_ && bytes <= kMaxBlock && held_bytes_ + bytes <= kMaxHeld) {
-            held_.emplace(bytes, p);
-            held_bytes_ += bytes;
-            return;
-        }
-    }
-    (void)hipFree(p);
-}
-
-void DevPool::release() {
-    std::multimap<size_t, void *> out;
-    {
-        std::lock_guard<std::mutex> g(mu_);
-        out.swap(held_);
-        held_bytes_ = 0;
-    }
-    for (auto &b : out) (void)hipFree(b.second);
-}
-
-void DevPool::close() {
-    {
-        std::lock_guard<std::mutex> g(mu_);
-        closed_ = true;
-    }
-    release();
 }
 
 char *PinnedStage::take(size_t bytes) {
@@ -520,10 +467,10 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
     } else {
         // factor records of one instance live in its workgroup's slot: rec_cap intervals.
         // budget: 80% of the device memory free at this point (the problem data is
-        // already allocated)
+        // already allocated; what the pool holds is given back when it is missing)
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b == 0) free_b = (size_t)120 << 30;
-        const size_t budget = free_b / 10 * 8;
+        const size_t budget = (free_b + ctx->pool->held()) / 10 * 8;
         D.aux_per_slot = block_aux_doubles(M, o->method, cap);
         auto per_slot = [&](int rc) {
             return block_slot_bytes(M, o->precision, rc) + D.aux_per_slot * sizeof(double);

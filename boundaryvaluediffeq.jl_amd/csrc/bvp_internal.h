@@ -5,41 +5,27 @@
 
 #include <map>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <tuple>
 #include <utility>
 #include <vector>
 
 #include "../../include/bvp_mirk.h"
+#include "dev_pool.h"
 #include "mirk_wave.h"
 #include "mlp.h"
 
-// Device blocks of a context that freed arenas leave for later ones (hipMalloc and hipFree
-// cost tens of microseconds each, and a call needs a handful of blocks: a lone pendulum solve
-// takes 0.46 ms, 0.89 ms with some 35 allocations and 17 small uploads per call).  At most kMaxHeld
-// bytes are held, no block above kMaxBlock; the rest, and everything when the context is
-// destroyed, goes back to the device.  All work on pooled memory is enqueued on the
-// context's one stream, so a block handed on is rewritten only after its last reader.
-class DevPool {
-  public:
-    static constexpr size_t kMaxHeld = (size_t)1 << 30, kMaxBlock = (size_t)256 << 20;
-    DevPool() = default;
-    DevPool(const DevPool &) = delete;
-    DevPool &operator=(const DevPool &) = delete;
-    ~DevPool() { close(); }
-    // a block of at least `bytes` (its true size in got), or null
-    void *take(size_t bytes, size_t &got);
-    void give(void *p, size_t bytes);
-    void release();  // frees the held blocks
-    void close();    // release(), and hold nothing from now on
-
-  private:
-    std::mutex mu_;
-    std::multimap<size_t, void *> held_;
-    size_t held_bytes_ = 0;
-    bool closed_ = false;
-};
+// a context's pool on the current device
+inline std::shared_ptr<DevPool> make_dev_pool() {
+    return std::make_shared<DevPool>(
+        [](size_t bytes) -> void * {
+            void *p = nullptr;
+            if (hipMalloc(&p, bytes) == hipSuccess) return p;
+            (void)hipGetLastError();
+            return nullptr;
+        },
+        [](void *p) { (void)hipFree(p); });
+}
 
 // Pinned host memory of a context: a small area that uploads and small results are staged
 // in, and two chunks that large results stream through (allocated when first needed).
@@ -65,7 +51,7 @@ struct bvp_ctx {
     // device address of the no-allocation entry point's scratch array on this
     // context's device (hipGetSymbolAddress at creation)
     char *noalloc = nullptr;
-    std::shared_ptr<DevPool> pool = std::make_shared<DevPool>();
+    std::shared_ptr<DevPool> pool = make_dev_pool();
     PinnedStage pin;
     // autotuner choices, (M, method, precision, kernel kind (0 wave, 1 block, 2 wave
     // under a global-error controller), family or -1) -> (variant,
