@@ -335,6 +335,7 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
     for (int i = 0; i < n; ++i) maxN0 = std::max(maxN0, inst[i].N);
     int cap = std::max(cap_req, std::max(o->max_num_subintervals, maxN0) + 1);
     auto *B = new bvp_batch();
+    B->device = ctx->device;
     B->arena.bump = bump;
     B->arena.bump_cap = bump_cap;
     B->n = n;
@@ -823,13 +824,24 @@ int bvp_batch_create(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_insta
     (void)hipSetDevice(ctx->device);
     return batch_build(ctx, o, n, inst, 0, out, nullptr, 0);
 }
-int bvp_batch_run(bvp_ctx *ctx, bvp_batch *B) { return (ctx && B) ? batch_run(ctx, B) : BVP_EINVAL; }
-int bvp_batch_sync(bvp_ctx *ctx, bvp_batch *B, float *ms) { return (ctx && B) ? batch_sync(ctx, B, ms) : BVP_EINVAL; }
+int bvp_batch_run(bvp_ctx *ctx, bvp_batch *B) {
+    if (!ctx || !B) return BVP_EINVAL;
+    (void)hipSetDevice(ctx->device);
+    return batch_run(ctx, B);
+}
+int bvp_batch_sync(bvp_ctx *ctx, bvp_batch *B, float *ms) {
+    if (!ctx || !B) return BVP_EINVAL;
+    (void)hipSetDevice(ctx->device);
+    return batch_sync(ctx, B, ms);
+}
 int bvp_batch_results(bvp_ctx *ctx, bvp_batch *B, bvp_result *res) {
-    return (ctx && B && res) ? batch_results(ctx, B, res) : BVP_EINVAL;
+    if (!ctx || !B || !res) return BVP_EINVAL;
+    (void)hipSetDevice(ctx->device);
+    return batch_results(ctx, B, res);
 }
 int bvp_batch_counters(bvp_ctx *ctx, bvp_batch *B, long long *out4) {
     if (!ctx || !B || !out4) return BVP_EINVAL;
+    (void)hipSetDevice(ctx->device);
     std::vector<long long> c((size_t)B->n * 4);
     HIP_TRY(ctx, hipMemcpy(c.data(), B->dev.cnt, c.size() * sizeof(long long), hipMemcpyDeviceToHost));
     for (int k = 0; k < 4; ++k) out4[k] = 0;
@@ -845,7 +857,11 @@ int bvp_batch_info(bvp_batch *B, int32_t *out4) {
     out4[3] = (int32_t)B->dev.scratch_per_slot;
     return 0;
 }
-void bvp_batch_destroy(bvp_batch *B) { delete B; }
+void bvp_batch_destroy(bvp_batch *B) {
+    if (!B) return;
+    (void)hipSetDevice(B->device);
+    delete B;
+}
 
 // ---- component entry points
 static int run_component(bvp_ctx *ctx, int method, int op, int32_t n, const bvp_instance *inst, int cap_req,
@@ -1408,7 +1424,10 @@ static double unit01(uint64_t &s) { return (double)(mix64(s) >> 11) * (1.0 / 900
 
 void bvp_mlp_destroy(bvp_mlp *m) {
     if (!m) return;
-    if (m->ctx) (void)hipStreamSynchronize(m->ctx->stream);
+    if (m->ctx) {
+        (void)hipSetDevice(m->ctx->device);
+        (void)hipStreamSynchronize(m->ctx->stream);
+    }
     delete m;
 }
 
@@ -1647,6 +1666,7 @@ int bvp_batch_set_warm_start(bvp_batch *B, const bvp_mlp *m, int32_t kind, int32
         return 0;
     }
     bvp_ctx *ctx = m->ctx;
+    (void)hipSetDevice(B->device);
     if (B->block || B->M != 2) { set_err(ctx, "the learned warm start serves M = 2 plans"); return BVP_ENOTSUP; }
     if (!B->has_u0) { set_err(ctx, "warm start: every instance needs u0 (the fallback guess)"); return BVP_EINVAL; }
     if (kind != BVP_FEAT_PARAM && kind != BVP_FEAT_LOG10_PARAM) { set_err(ctx, "bad feature kind"); return BVP_EINVAL; }

@@ -92,6 +92,7 @@ struct bvp_mlp {
 };
 
 struct bvp_batch {
+    int device = 0;      // of the context it was built on
     int n = 0, M = 0, method = 4, cap = 0, blocks = 0;
     int variant = 0;     // solve-kernel variant (wave_variants)
     int family = -1;     // the batch's single family when all its BCs are two-point, else -1
