@@ -597,8 +597,20 @@ static int capture(bvp_ctx *ctx, bvp_batch *B, int (*fn)(bvp_ctx *, bvp_batch *)
     return 0;
 }
 
+// A plan's blocks come from the pool of the context it was built on, whose stream orders their
+// reuse; batch_build leaves that stream idle.  For a run on another context's stream, blocks
+// taken since then wait here for their earlier readers, and bvp_batch_destroy for the run.
+static int order_run(bvp_ctx *ctx, bvp_batch *B) {
+    if (!B->arena.pool || B->arena.pool == ctx->pool) return 0;
+    B->foreign = true;
+    if (B->grown) HIP_TRY(ctx, hipDeviceSynchronize());
+    B->grown = false;
+    return 0;
+}
+
 int batch_run(bvp_ctx *ctx, bvp_batch *B) {
     if (fp64_block32_blocked(ctx, B)) return BVP_ENOTSUP;
+    if (int rc = order_run(ctx, B)) return rc;
     if (B->use_graph) {
         if (B->graph_exec && B->mlp && B->mlp_gen != B->mlp->gen) B->drop_graph();  // normalisation changed
         if (!B->graph_exec) {
@@ -860,6 +872,7 @@ int bvp_batch_info(bvp_batch *B, int32_t *out4) {
 void bvp_batch_destroy(bvp_batch *B) {
     if (!B) return;
     (void)hipSetDevice(B->device);
+    if (B->foreign) (void)hipDeviceSynchronize();
     delete B;
 }
 
@@ -1257,6 +1270,7 @@ int bvp_batch_learned_guess(bvp_ctx *ctx, bvp_batch *B, double *y) {
     if (!ctx || !B || !y) return BVP_EINVAL;
     if (!B->mlp) { set_err(ctx, "no network attached to the plan"); return BVP_EINVAL; }
     (void)hipSetDevice(ctx->device);
+    if (int rc = order_run(ctx, B)) return rc;
     if (int rc = enqueue_guess(ctx, B)) return rc;
     if (B->anchors > 0) HIP_TRY(ctx, mlp::launch_anchor_fill(B->dev, B->anc, B->anchors, B->warm_y, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(y, B->warm_y, sizeof(double) * (size_t)B->total_nodes * B->M,
@@ -1454,6 +1468,10 @@ int bvp_mlp_create(bvp_ctx *ctx, uint64_t seed, bvp_mlp **out) {
     *out = nullptr;
     auto *m = new bvp_mlp();
     m->ctx = ctx;
+    // not pooled: plans of other contexts may read the network, and memory that goes straight
+    // back to the device waits for their streams too
+    m->arena.pool = make_dev_pool();
+    m->arena.pool->close();
     int rc;
     mlp::NetBufs &nb = m->nb;
     if ((rc = dalloc(ctx, m->arena, nb.w, mlp::NPARAM)) || (rc = dalloc(ctx, m->arena, nb.m, mlp::NPARAM)) ||
@@ -1677,10 +1695,12 @@ int bvp_batch_set_warm_start(bvp_batch *B, const bvp_mlp *m, int32_t kind, int32
     if (!B->warm_y) {
         const int rc = dalloc(ctx, B->arena, B->warm_y, (size_t)B->total_nodes * B->M);
         if (rc) return rc;
+        B->grown = true;
     }
     if (anchors > B->anc_cap) {  // grows only; the arena frees with the plan
         const int rc = dalloc(ctx, B->arena, B->anc, (size_t)B->n * anchors * 4);
         if (rc) return rc;
+        B->grown = true;
         B->anc_cap = anchors;
     }
     B->anchors = anchors;

@@ -92,7 +92,9 @@ struct bvp_mlp {
 };
 
 struct bvp_batch {
-    int device = 0;      // of the context it was built on
+    int device = 0;       // of the context it was built on
+    bool foreign = false; // has run on another context's stream
+    bool grown = false;   // has taken blocks since it was built
     int n = 0, M = 0, method = 4, cap = 0, blocks = 0;
     int variant = 0;     // solve-kernel variant (wave_variants)
     int family = -1;     // the batch's single family when all its BCs are two-point, else -1
