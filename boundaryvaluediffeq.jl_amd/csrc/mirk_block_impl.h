@@ -145,6 +145,35 @@ __device__ inline int wave_argmax_first(float v) {
     const unsigned long long b = __ballot(v == mx);
     return __builtin_amdgcn_readfirstlane(b ? __ffsll((long long)b) - 1 : 0);
 }
+// maximum of v over the wave, by the same moves
+__device__ inline int wave_max_int(int v) {
+#define BVP_DPP_MAX(ctrl, rmask) v = max(v, __builtin_amdgcn_update_dpp(v, v, ctrl, rmask, 0xf, false))
+    BVP_DPP_MAX(0x111, 0xf);
+    BVP_DPP_MAX(0x112, 0xf);
+    BVP_DPP_MAX(0x114, 0xf);
+    BVP_DPP_MAX(0x118, 0xf);
+    BVP_DPP_MAX(0x142, 0xa);
+    BVP_DPP_MAX(0x143, 0xc);
+#undef BVP_DPP_MAX
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Lane of the first maximum of |v| over the lanes that are not done, compared in the
+// precision of v.  FP64: by the high words (whose order as integers is that of the values),
+// and only where several lanes share the largest one by the low words too.
+__device__ inline int pivot_lane(float v, bool done) { return wave_argmax_first(done ? -1.f : fabsf(v)); }
+__device__ inline int pivot_lane(double v, bool done) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(fabs(v));
+    const int hi = done ? -1 : (int)(b >> 32);
+    const bool in = hi == wave_max_int(hi);
+    unsigned long long c = __ballot(in);
+    if (__builtin_expect((c & (c - 1)) != 0, 0)) {
+        const int lo = in ? (int)((unsigned)b ^ 0x80000000u) : (int)0x80000000;
+        const int ml = wave_max_int(lo);
+        c = __ballot(in && lo == ml);
+    }
+    return __builtin_amdgcn_readfirstlane(__ffsll((long long)c) - 1);
+}
 
 // ------------------------------------------------------------------ records
 // Per eliminated node k (and in the same slots the nodes between the chunks):
@@ -170,7 +199,7 @@ template <int M> struct BRoot {
 // left in row[0 .. NW_-NC).  Steps run in groups of G with compile-time column indexes
 // (the row stays in registers); between groups the row is shifted by G columns, which
 // keeps the code of one group for all.  The pivot of a step is the first maximum of
-// |row[j]| over rows not used yet (compared in FP32).  Pivot rows stay in their lanes,
+// |row[j]| over rows not used yet.  Pivot rows stay in their lanes,
 // unscaled; dinv receives 1 / pivot in those lanes, pstep the step (else -1).
 // put(j, m) stores lane's multiplier of step j; pivs: lane j's value is the pivot lane
 // of step j (j < 64).  The columns are updated 16 (FP64: 8) at a time: left to itself the
@@ -188,7 +217,7 @@ __device__ __forceinline__ void gauss_jordan(T (&row)[NW_], int lane, int &pstep
 #pragma unroll
         for (int jj = 0; jj < G; ++jj) {
             const T rj = row[jj];
-            const int p = wave_argmax_first(done ? -1.f : (float)fabs(rj));
+            const int p = pivot_lane(rj, done);
             const T inv = (T)1 / rdlane(rj, p);
             const bool mine = lane == p;
             const T m = mine ? (T)0 : rj * inv;
