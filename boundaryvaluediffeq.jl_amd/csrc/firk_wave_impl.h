@@ -17,7 +17,15 @@
 // those of the expanded system.
 //
 // One wave (64 lanes) per instance, lanes own contiguous chunks of intervals.
-// Template parameters: M state dimension (1..4), S stages (1, 2, 3, 4, 5, 7).
+// Template parameters: M state dimension (1..4, 6), S stages (1, 2, 3, 4, 5, 7).
+//
+// The solve (firk_solve_instance and what it calls once) is one inlined body per form: a function
+// that the compiler leaves out of line takes the instance and its parameters by reference, which
+// keeps them in private memory for the whole kernel, and serves both forms at run time.  What is
+// large and called from several places is out of line on purpose and takes its arguments by
+// value.  (Left to the compiler's choice: M = 3, s = 3 4.2 KB of scratch per lane and 0.83 ms for
+// 2,048 linear problems, this way 0.56 KB and 0.63 ms; M = 2, s = 5, general kernels, 4,096 Bratu
+// problems 2.7 -> 1.4 ms.)
 #pragma once
 
 #include "mirk_wave_impl.h"
@@ -28,7 +36,7 @@ namespace bvpdev {
 // is interleaved over the lanes that own the intervals: field q of interval k lies at
 // [step i][q][64 lanes] with k the i-th interval of its lane's chunk, so that the 64 lanes
 // walking their chunks read and write whole 512-byte lines.  (In [interval][field] order
-// every access of the wave touched 64 lines.)  An area holds kFirkPad<cap> intervals.
+// every access of the wave touched 64 lines.)  An area holds firk_pad(cap) intervals.
 __host__ __device__ inline size_t firk_pad(int cap) { return (size_t)cap + WAVE; }
 
 struct FirkAt {
@@ -67,10 +75,26 @@ __device__ inline const FirkTab &firk_tab_of(const BatchDev &B) {
     return *(const FirkTab *)(const __attribute__((address_space(4))) FirkTab *)B.firk_tab;
 }
 
+// Arguments of functions that are not inlined arrive as generic pointers in vector registers;
+// named by their memory they compile to plain accesses instead of flat ones, and uniform
+// ones to scalar loads.
+template <typename T> __device__ __forceinline__ T &as_private(T &x) {
+    return *(T *)(__attribute__((address_space(5))) T *)&x;
+}
+template <typename T> __device__ __forceinline__ T *as_private_ptr(T *p) {
+    return (T *)(__attribute__((address_space(5))) T *)p;
+}
+template <typename T> __device__ __forceinline__ T *as_lds(T *p) {
+    return (T *)(__attribute__((address_space(3))) T *)p;
+}
+__device__ __forceinline__ const FirkTab &firk_tab_uniform(const FirkTab &T) {
+    return *(const FirkTab *)(const __attribute__((address_space(4))) FirkTab *)uni(&T);
+}
+
 // ------------------------------------------------------------------ dense solve
 // W X = R in place (R becomes X), Gaussian elimination with partial pivoting (first
 // maximum).  Small systems stay in registers (unrolled, row swaps by selects); larger
-// ones (S M > 8) run as loops over private arrays.  Returns false on a zero pivot.
+// ones (S M > 12) run as loops over private arrays.  Returns false on a zero pivot.
 // (All unrolled loops have constant trip counts with a condition inside: triangular bounds
 // leave the arrays in private memory, with a store for every update.)
 template <int NN, int NR>
@@ -234,14 +258,17 @@ __device__ __forceinline__ bool lu_solve_diag(double (&W)[NN][NN], double (&R)[N
 // Stage points Y_r = h (sum_j a_rj K_j) + y_i, stage residuals G_r = f(t_i + c_r h, Y_r)
 // - K_r and the continuity residual Phi = (y_{i+1} - y_i) - h (sum_j b_j K_j), in the
 // order of operations of Phi! (FIRK/collocation.jl:59-93); with JAC the stage Jacobians
-// J_r.  Where the exchange area ([field][64 lanes], in the LDS that the tree uses between
-// the interval passes) holds f and J of all stages, the stages run as a loop (the families'
-// code once instead of S times) and pass them through the lane's column sl of it.  Without
-// it (LD false), and for systems of more than 12 unknowns, whose arrays lie in private
-// memory in any case, the pieces run out of line, so that a kernel holds their frames once.
+// J_r.  At M = 2, whose families branch most, the stages run as a loop (the families' code
+// once instead of S times) and pass f and J through the lane's column sl of an exchange area
+// ([field][64 lanes], in the LDS that the tree uses between the interval passes); elsewhere, and
+// in the rare evaluations (HOT false), they are unrolled.  (M = 3, s = 3, 2,048 linear problems:
+// 0.85 ms; with the exchange area and the pass without row exchanges 1.18 ms, with that pass alone
+// 0.96 ms.)  Systems of more than 12 unknowns, whose arrays lie in private memory in any case, run
+// rolled and out of line, so that a kernel holds their frames once.
 template <int M, int S> constexpr int kFirkSlot = S * (M + M * M);  // fields of the exchange area
 template <int M, int S> constexpr bool kFirkBig = S * M > 12;
-template <int M, int S> constexpr bool kFirkSlotLds = !kFirkBig<M, S> && kFirkSlot<M, S> * WAVE <= kStageNodes<M> * M;
+template <int M, int S> constexpr bool kFirkLoop =
+    M == 2 && !kFirkBig<M, S> && kFirkSlot<M, S> * WAVE <= kStageNodes<M> * M;
 
 template <int M, int S, bool JAC>
 __device__ __forceinline__ void firk_stage(const Inst<M> &I, const FirkTab &T, int r, double ti, double h,
@@ -271,9 +298,9 @@ __device__ __forceinline__ void firk_phi(const FirkTab &T, double h, const doubl
     }
 }
 template <int M, int S, bool JAC>
-__device__ __noinline__ void firk_interval_big(const Inst<M> &I, const FirkTab &T, double ti, double h,
-                                               const double *yi, const double *yj, const double (&K)[S][M],
-                                               double (&G)[S][M], double (&Phi)[M], double (&J)[S][M][M]) {
+__device__ __forceinline__ void firk_interval_rolled(const Inst<M> &I, const FirkTab &T, double ti, double h,
+                                                     const double *yi, const double *yj, const double (&K)[S][M],
+                                                     double (&G)[S][M], double (&Phi)[M], double (&J)[S][M][M]) {
 #pragma unroll 1
     for (int r = 0; r < S; ++r) {
         double F[M], Jr[M][M];
@@ -288,12 +315,29 @@ __device__ __noinline__ void firk_interval_big(const Inst<M> &I, const FirkTab &
     }
     firk_phi<M, S>(T, h, yi, yj, K, Phi);
 }
-template <int M, int S, bool JAC, bool LD = kFirkSlotLds<M, S>>
+template <int M, int S, bool JAC>
+__device__ __noinline__ void firk_interval_big(const Inst<M> &I, const FirkTab &T, double ti, double h,
+                                               const double *yi, const double *yj, const double (&K)[S][M],
+                                               double (&G)[S][M], double (&Phi)[M], double (&J)[S][M][M]) {
+    firk_interval_rolled<M, S, JAC>(as_private(I), firk_tab_uniform(T), ti, h, as_private_ptr(yi), as_private_ptr(yj),
+                                    as_private(K), as_private(G), as_private(Phi), as_private(J));
+}
+template <int M, int S, bool JAC, bool HOT = true>
 __device__ __forceinline__ void firk_interval(const Inst<M> &I, const FirkTab &T, double *sl, double ti, double h,
                                               const double *yi, const double *yj, const double (&K)[S][M],
                                               double (&G)[S][M], double (&Phi)[M], double (&J)[S][M][M]) {
-    if constexpr (!LD) {
-        firk_interval_big<M, S, JAC>(I, T, ti, h, yi, yj, K, G, Phi, J);
+    if constexpr (kFirkBig<M, S>) {
+        if constexpr (HOT) firk_interval_big<M, S, JAC>(I, T, ti, h, yi, yj, K, G, Phi, J);
+        else firk_interval_rolled<M, S, JAC>(I, T, ti, h, yi, yj, K, G, Phi, J);
+    } else if constexpr (!HOT || !kFirkLoop<M, S>) {
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            double F[M];
+            firk_stage<M, S, JAC>(I, T, r, ti, h, yi, K, F, J[r]);
+#pragma unroll
+            for (int a = 0; a < M; ++a) G[r][a] = F[a] - K[r][a];
+        }
+        firk_phi<M, S>(T, h, yi, yj, K, Phi);
     } else {
         constexpr int NS = M + M * M;
 #pragma unroll 1
@@ -328,8 +372,8 @@ __device__ __forceinline__ void firk_interval(const Inst<M> &I, const FirkTab &T
 // PIV false: without row exchanges; piv is set when a lane needs one (X is then undefined),
 // and the caller repeats its pass with PIV true.
 template <int M, int S, int NR>
-__device__ __noinline__ bool firk_local_big(const FirkTab &T, double h, const double (&G)[S][M],
-                                            const double (&J)[S][M][M], double (&X)[S * M][NR]) {
+__device__ __forceinline__ bool firk_local_rolled(const FirkTab &T, double h, const double (&G)[S][M],
+                                                  const double (&J)[S][M][M], double (&X)[S * M][NR]) {
     constexpr int NN = S * M;
     double W[NN][NN];
 #pragma unroll 1
@@ -348,12 +392,18 @@ __device__ __noinline__ bool firk_local_big(const FirkTab &T, double h, const do
         }
     return lu_solve<NN, NR>(W, X);
 }
-template <int M, int S, int NR, bool PIV>
+template <int M, int S, int NR>
+__device__ __noinline__ bool firk_local_big(const FirkTab &T, double h, const double (&G)[S][M],
+                                            const double (&J)[S][M][M], double (&X)[S * M][NR]) {
+    return firk_local_rolled<M, S, NR>(firk_tab_uniform(T), h, as_private(G), as_private(J), as_private(X));
+}
+template <int M, int S, int NR, bool PIV, bool HOT = true>
 __device__ __forceinline__ bool firk_local(const FirkTab &T, double h, const double (&G)[S][M],
                                            const double (&J)[S][M][M], double (&X)[S * M][NR], bool &piv) {
     if constexpr (kFirkBig<M, S>) {
         static_assert(PIV, "systems above 12 unknowns are solved with row exchanges");
-        return firk_local_big<M, S, NR>(T, h, G, J, X);
+        if constexpr (HOT) return firk_local_big<M, S, NR>(T, h, G, J, X);
+        else return firk_local_rolled<M, S, NR>(T, h, G, J, X);
     } else {
         constexpr int NN = S * M;
         double W[NN][NN];
@@ -433,27 +483,31 @@ __device__ __forceinline__ void load_stages(const double *K, size_t off, double 
 // until max|G| <= tol, checked before every step, NaN stops, at most 1000 steps) and
 // the residual is Phi_i.  Its Jacobian enters the outer one by the implicit function
 // theorem, dK/dy_i = W^-1 [J_1; ...; J_s] -- the KJ of the condensation.
-template <int M> struct FirkNest {
-    bool on;
-    bool irows;  // boundary rows inside the span may occur (EvalSol rows)
+// ON: 1 the nested form, 0 the expanded one, -1 either (the component kernels).  ROWS: boundary
+// rows inside the span may occur (EvalSol rows).  Both are part of the type, so that a kernel of
+// one form carries no code of the other, inlined or not.
+template <int M, int ON, bool ROWS> struct FirkNest {
+    static constexpr int form = ON;
+    static constexpr bool irows = ROWS;
+    bool is;
     double tol;
     double k0[M];
+    __device__ __forceinline__ bool on() const { return ON < 0 ? is : ON != 0; }
 };
 
-template <int M>
-__device__ inline FirkNest<M> firk_nest_of(const BatchDev &B, int b) {
-    FirkNest<M> n;
-    n.on = B.firk_nested != 0;
+template <int M, int ON, bool ROWS>
+__device__ inline FirkNest<M, ON, ROWS> firk_nest_of(const BatchDev &B, int b) {
+    FirkNest<M, ON, ROWS> n;
+    n.is = B.firk_nested != 0;
     n.tol = B.nest_tol;
-    n.irows = true;
 #pragma unroll
-    for (int c = 0; c < M; ++c) n.k0[c] = n.on ? B.u0c[(size_t)b * M + c] : 0.0;
+    for (int c = 0; c < M; ++c) n.k0[c] = n.on() ? B.u0c[(size_t)b * M + c] : 0.0;
     return n;
 }
 
 // PIV false: stops with piv set where a lane's system needs row exchanges (K undefined).
-template <int M, int S, bool LD, bool PIV>
-__device__ __forceinline__ void firk_inner_body(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double *sl,
+template <int M, int S, bool HOT, bool PIV, class NT>
+__device__ __forceinline__ void firk_inner_body(const Inst<M> &I, const FirkTab &T, const NT &nest, double *sl,
                                            double ti, double h, const double *yi, double (&K)[S][M], bool &piv) {
 #pragma unroll
     for (int r = 0; r < S; ++r)
@@ -461,7 +515,7 @@ __device__ __forceinline__ void firk_inner_body(const Inst<M> &I, const FirkTab 
         for (int c = 0; c < M; ++c) K[r][c] = nest.k0[c];
     for (int it = 0; it < 1000; ++it) {
         double G[S][M], Phi[M], J[S][M][M];
-        firk_interval<M, S, true, LD>(I, T, sl, ti, h, yi, yi, K, G, Phi, J);
+        firk_interval<M, S, true, HOT>(I, T, sl, ti, h, yi, yi, K, G, Phi, J);
         double mx = 0.0;
         bool bad = false;
 #pragma unroll
@@ -473,7 +527,7 @@ __device__ __forceinline__ void firk_inner_body(const Inst<M> &I, const FirkTab 
             }
         if (bad || !(mx > nest.tol)) break;
         double X[S * M][1];
-        if (!firk_local<M, S, 1, PIV>(T, h, G, J, X, piv)) break;
+        if (!firk_local<M, S, 1, PIV, HOT>(T, h, G, J, X, piv)) break;
         if (!PIV && piv) break;
 #pragma unroll
         for (int r = 0; r < S; ++r)
@@ -482,17 +536,57 @@ __device__ __forceinline__ void firk_inner_body(const Inst<M> &I, const FirkTab 
     }
 }
 
-template <int M, int S>
-__device__ __noinline__ void firk_inner_big(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double ti,
-                                            double h, const double *yi, double (&K)[S][M]) {
-    bool piv = false;
-    firk_inner_body<M, S, false, true>(I, T, nest, nullptr, ti, h, yi, K, piv);
+// Inner solves out of line, with everything they need inside: of large systems, and the rare
+// ones of boundary rows inside the span and of the dense output (HOT false).  Arguments and
+// result by value: a reference would keep the caller's parameters in private memory.
+template <int M> struct FirkInnerArgs {
+    const FirkTab *T;
+    const double *params;
+    int pcnt, fam;
+    double ti, h, yi[M];
+    FirkNest<M, 1, false> nest;
+};
+template <int M, int S> struct FirkStages {
+    double k[S][M];
+};
+// UNIFORM: one instance for the whole wave (the dense output has one per thread)
+template <int M, bool UNIFORM>
+__device__ __forceinline__ void firk_inst(const double *params, int pcnt, int fam, Inst<M> &I) {
+    params = UNIFORM ? uni(params) : as_global(params);
+    I.fam = UNIFORM ? uni(fam) : fam;
+    I.minc = 1;
+    if (UNIFORM) pcnt = uni(pcnt);
+#pragma unroll
+    for (int k = 0; k < Params<M>::MAXP; ++k) I.P.p[k] = k < pcnt ? params[k] : 0.0;
 }
-template <int M, int S, bool LD, bool PIV>
-__device__ __forceinline__ void firk_inner(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double *sl,
+template <int M, int S, bool UNIFORM>
+__device__ __noinline__ FirkStages<M, S> firk_inner_out(FirkInnerArgs<M> a) {
+    Inst<M> I;
+    firk_inst<M, UNIFORM>(a.params, a.pcnt, a.fam, I);
+    FirkStages<M, S> K;
+    bool piv = false;
+    firk_inner_body<M, S, false, true>(I, firk_tab_uniform(*a.T), a.nest, nullptr, a.ti, a.h, a.yi, K.k, piv);
+    return K;
+}
+template <int M, int S, bool HOT, bool PIV, class NT>
+__device__ __forceinline__ void firk_inner(const Inst<M> &I, const FirkTab &T, const NT &nest, double *sl,
                                            double ti, double h, const double *yi, double (&K)[S][M], bool &piv) {
-    if constexpr (kFirkBig<M, S>) firk_inner_big<M, S>(I, T, nest, ti, h, yi, K);
-    else firk_inner_body<M, S, LD, PIV>(I, T, nest, sl, ti, h, yi, K, piv);
+    if constexpr (NT::form == 0) {  // no inner solves in the expanded form
+    } else if constexpr (kFirkBig<M, S> || !HOT) {
+        FirkInnerArgs<M> a{&T, I.params, I.pcnt, I.fam, ti, h, {}, {true, nest.tol, {}}};
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            a.yi[c] = yi[c];
+            a.nest.k0[c] = nest.k0[c];
+        }
+        const FirkStages<M, S> r = firk_inner_out<M, S, HOT>(a);
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+#pragma unroll
+            for (int c = 0; c < M; ++c) K[q][c] = r.k[q][c];
+    } else {
+        firk_inner_body<M, S, true, PIV>(I, T, nest, sl, ti, h, yi, K, piv);
+    }
 }
 
 template <int M, int S>
@@ -538,7 +632,7 @@ template <int M> struct FirkShared : Shared<M> {
 };
 // this lane's column of the exchange area
 template <int M, int S> __device__ __forceinline__ double *firk_slot(Shared<M> &sh, int lane) {
-    return kFirkSlotLds<M, S> ? sh.stage + lane : nullptr;
+    return kFirkLoop<M, S> ? sh.stage + lane : nullptr;
 }
 
 // ------------------------------------------------------------------ interior boundary rows
@@ -660,8 +754,8 @@ __device__ inline double firk_evalsol(const Inst<M> &I, const FirkTab &T, bool e
 // its linearisation for the root solve into ir: [M] coefficients of dy_j, [M] of dy_{j+1},
 // the constant, with the stage corrections eliminated through the interval's record in loc
 // (dK = kg + KJ dy_j).  N: the mesh the lane-interleaved areas belong to.
-template <int M, int S, bool WANTG>
-__device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest,
+template <int M, int S, bool WANTG, class NT>
+__device__ __noinline__ double firk_bc_interior(Inst<M> I, const FirkTab &T, NT nest,
                                           const double *mesh, const double *y, const double *K, const double *dy,
                                           const double *dK, double alpha, int k, int j, const double *loc,
                                           double *ir, int N, const double *dy2 = nullptr,
@@ -681,8 +775,8 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
             yj[c] += beta * dy2[(size_t)(j + 1) * M + c];
         }
     }
-    if (nest.on) {
-        FirkNest<M> z = nest;
+    if (nest.on()) {
+        NT z = nest;
 #pragma unroll
         for (int c = 0; c < M; ++c) z.k0[c] = 0.0;
         bool piv = false;
@@ -699,7 +793,7 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
     }
     double g[(S + 2) * M];
     const double v =
-        firk_evalsol<M, S, WANTG>(I, T, !nest.on, mesh[j], mesh[j + 1], sel<M>(I.bct, k), comp, yi, yj, Kk, g);
+        firk_evalsol<M, S, WANTG>(I, T, !nest.on(), mesh[j], mesh[j + 1], sel<M>(I.bct, k), comp, yi, yj, Kk, g);
     if constexpr (WANTG) {
         if (graw)
 #pragma unroll
@@ -710,7 +804,7 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
         double cst = 0.0, ca[M];
 #pragma unroll
         for (int c = 0; c < M; ++c) ca[c] = g[c];
-        if (!nest.on) {
+        if (!nest.on()) {
             const double *lk = loc + firk_off<kFirkLoc<M, S>>(N, j, true);
 #pragma unroll
             for (int q = 0; q < NN; ++q) {
@@ -728,12 +822,12 @@ __device__ inline double firk_bc_interior(const Inst<M> &I, const FirkTab &T, co
 }
 
 // Residual of boundary row k (L: where it sits) at (y + alpha dy, K + alpha dK).
-template <int M, int S>
-__device__ inline double firk_bc_row(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, const double *mesh,
+template <int M, int S, class NT>
+__device__ __forceinline__ double firk_bc_row(const Inst<M> &I, const FirkTab &T, const NT &nest, const double *mesh,
                                      const double *y, const double *K, const double *dy, const double *dK,
                                      double alpha, int k, const BcLoc &L, int N, const double *dy2 = nullptr,
                                      const double *dK2 = nullptr, double beta = 0.0) {
-    if (L.iv < 0 || !nest.irows) {
+    if (!NT::irows || L.iv < 0) {
         const size_t q = (size_t)L.node * M + sel<M>(I.bcc, k);
         return (dy ? y[q] + alpha * dy[q] : y[q]) + (dy2 ? beta * dy2[q] : 0.0) - sel<M>(I.bcv, k);
     }
@@ -742,8 +836,8 @@ __device__ inline double firk_bc_row(const Inst<M> &I, const FirkTab &T, const F
 }
 
 // Boundary rows of the FIRK path at (y, K): residuals and nodes in sh.
-template <int M, int S>
-__device__ inline void firk_bc_rows(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+template <int M, int S, class NT>
+__device__ __forceinline__ void firk_bc_rows(const Inst<M> &I, const FirkTab &T, const NT &nest, Shared<M> &sh,
                                     const double *mesh, const double *y, const double *K, int N, int lane) {
     if (lane < M) {
         const BcLoc L = bc_locate<M>(I, lane, mesh, N);
@@ -786,8 +880,8 @@ template <int M> struct FirkPass {
     double mx;
     bool bad, sg, piv;
 };
-template <int M, int S, bool PIV>
-__device__ __forceinline__ void firk_chunk(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, double *sl,
+template <int M, int S, bool PIV, class NT>
+__device__ __forceinline__ void firk_chunk(const Inst<M> &I, const FirkTab &T, const NT &nest, double *sl,
                                            const double *mesh, const double *y, double *K, int N, int lane,
                                            double *scr, double *loc, Rel<M> &rel, FirkPass<M> &ps) {
     int P, start, len;
@@ -808,18 +902,18 @@ __device__ __forceinline__ void firk_chunk(const Inst<M> &I, const FirkTab &T, c
 #pragma unroll
         for (int c = 0; c < M; ++c) yj[c] = y[(size_t)(k + 1) * M + c];
         const size_t ko = firk_off<S * M>(lane, i);
-        if (nest.on) {
-            firk_inner<M, S, kFirkSlotLds<M, S>, PIV>(I, T, nest, sl, ti, h, yi, Kk, ps.piv);
+        if (nest.on()) {
+            firk_inner<M, S, true, PIV>(I, T, nest, sl, ti, h, yi, Kk, ps.piv);
             store_stages<M, S>(K, ko, Kk);
         } else {
             load_stages<M, S>(K, ko, Kk);
         }
         firk_interval<M, S, true>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
-        firk_fold<M, S>(Phi, G, nest.on, ps.mx, ps.bad);
+        firk_fold<M, S>(Phi, G, nest.on(), ps.mx, ps.bad);
         double Sb[M][M], rhs[M], Rb[M][M];
-        ps.sg |= !firk_condense<M, S, PIV>(T, h, G, Phi, J, loc + firk_off<kFirkLoc<M, S>>(lane, i), Sb, rhs, nest.on,
+        ps.sg |= !firk_condense<M, S, PIV>(T, h, G, Phi, J, loc + firk_off<kFirkLoc<M, S>>(lane, i), Sb, rhs, nest.on(),
                                            ps.piv);
-        if (!PIV && ps.piv) break;
+        if (!PIV && __any(ps.piv)) break;  // one lane's need ends the pass of all
 #pragma unroll
         for (int a = 0; a < M; ++a)
 #pragma unroll
@@ -845,30 +939,27 @@ __device__ __forceinline__ void firk_chunk(const Inst<M> &I, const FirkTab &T, c
 }
 
 // The chunk pass with row exchanges, out of line (in line, the exchanges cost the plain
-// pass hundreds of spill stores per interval); its relation comes back through LDS.  NEST:
-// the form, -1 for both.
-template <int M> struct FirkPivArgs {
+// pass hundreds of spill stores per interval); its relation comes back through LDS.
+template <int M, class NT> struct FirkPivArgs {
     const FirkTab *T;
     const double *params, *mesh, *y;
     double *sl, *K, *scr, *loc, *rel;
     int pcnt, fam, N, lane;
-    FirkNest<M> nest;
+    NT nest;
 };
-template <int M, int S, int NEST>
-__device__ __noinline__ FirkPass<M> firk_chunk_pivoted(FirkPivArgs<M> a) {
+template <int M, int S, class NT>
+__device__ __noinline__ FirkPass<M> firk_chunk_pivoted(FirkPivArgs<M, NT> a) {
     Inst<M> I;
-    I.fam = a.fam;
-    I.minc = 1;
-#pragma unroll
-    for (int k = 0; k < Params<M>::MAXP; ++k) I.P.p[k] = k < a.pcnt ? a.params[k] : 0.0;
-    FirkNest<M> nest = a.nest;
-    if constexpr (NEST >= 0) nest.on = NEST != 0;
+    firk_inst<M, true>(a.params, a.pcnt, a.fam, I);
+    I.params = a.params;
+    I.pcnt = a.pcnt;
     Rel<M> rel;
     FirkPass<M> ps;
-    firk_chunk<M, S, true>(I, *a.T, nest, a.sl, a.mesh, a.y, a.K, a.N, a.lane, a.scr, a.loc, rel, ps);
+    firk_chunk<M, S, true>(I, firk_tab_uniform(*a.T), a.nest, as_lds(a.sl), uni(a.mesh), uni(a.y), uni(a.K), uni(a.N),
+                           a.lane, uni(a.scr), uni(a.loc), rel, ps);
     __syncthreads();  // the exchange area shares its LDS with the relations
     int f = 0;
-    double *o = a.rel + (size_t)a.lane * kRelFields<M>;
+    double *o = as_lds(a.rel) + (size_t)a.lane * kRelFields<M>;
 #pragma unroll
     for (int i = 0; i < M; ++i)
 #pragma unroll
@@ -882,36 +973,69 @@ __device__ __noinline__ FirkPass<M> firk_chunk_pivoted(FirkPivArgs<M> a) {
     return ps;
 }
 
-// Where the local systems run without row exchanges first (DIAG): from 6 unknowns (below, the
-// exchanges cost little) to 12 (above, the solve runs rolled over private arrays), in the
-// solve kernels of one wave per SIMD (the pivoted pass takes more registers than two leave).
-// Solve kernel at M = 2, one wave per SIMD: s = 5, 2,048 Bratu problems 12.6 ms before, 3.6 ms
-// (7.9 ms with the layout and the stage loop alone); nested s = 3, 4,096 problems 3.18 -> 2.50 ms.
-template <int M, int S> constexpr bool kFirkDiag = S * M >= 6 && S * M <= 12;
+// Where the local systems run without row exchanges first (DIAG): at M = 2 (at M = 3 it cost
+// more than the exchanges, see firk_interval) from 6 unknowns (below, the exchanges cost little)
+// to 12 (above, the solve runs rolled over private arrays), in the solve kernels of one wave per
+// SIMD (the pivoted pass takes more registers than two leave).
+// Solve kernel, s = 5, 2,048 Bratu problems: 12.6 ms before, 3.6 ms (7.9 ms with the layout and
+// the stage loop alone); nested s = 3, 4,096 problems 3.18 -> 2.50 ms.  Problems that need the
+// exchanges in every interval (u'' = k^2 u, 2,048 of 64..255 intervals): s = 3 0.191 ms before and
+// now, 0.209 ms without the look below; s = 5 1.38 -> 0.42 ms; nested s = 3 0.222 -> 0.218 ms.
+template <int M, int S> constexpr bool kFirkDiag = M == 2 && S * M >= 6 && S * M <= 12;
 
-// sticky: an earlier pass of this instance needed row exchanges (kept by the caller)
-template <int M, int S, bool DIAG>
-__device__ __forceinline__ double firk_forward(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest,
+// Whether the first columns of the local system at the left node of this lane's first interval
+// already call for a row exchange: an instance that needs them is not sent through a pass
+// without first (where the look misses one, that pass finds it).
+template <int M, int S>
+__device__ __forceinline__ bool firk_look(const Inst<M> &I, const FirkTab &T, const double *mesh, const double *y, int N,
+                                          int lane) {
+    int P, start, len;
+    chunk_of(N, lane, P, start, len);
+    bool need = false;
+    if (len > 0) {
+        const double t = mesh[start], h = mesh[start + 1] - t;
+        double yi[M], F[M], J[M][M];
+#pragma unroll
+        for (int c = 0; c < M; ++c) yi[c] = y[(size_t)start * M + c];
+        f_jac<M>(I.fam, I.P, t, yi, F, J);
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            const double best = fabs(1.0 - h * T.A[0][0] * J[c][c]);
+#pragma unroll
+            for (int r = 0; r < S; ++r)
+#pragma unroll
+                for (int a = 0; a < M; ++a)
+                    if (r > 0 || a > c) need |= fabs(h * T.A[r][0] * J[a][c]) > best;
+        }
+    }
+    return need;
+}
+
+// sticky: an earlier pass of this instance needed row exchanges (kept by the caller); -1: no
+// pass yet
+template <int M, int S, bool DIAG, class NT>
+__device__ __forceinline__ double firk_forward(const Inst<M> &I, const FirkTab &T, const NT &nest,
                                                Shared<M> &sh, const double *mesh, const double *y, double *K, int N,
                                                int lane, double *scr, double *loc, Rel<M> &rel, bool &sing,
-                                               bool &sticky) {
+                                               int &sticky) {
     double *sl = firk_slot<M, S>(sh, lane);
     FirkPass<M> ps;
     if constexpr (kFirkBig<M, S>) {
-        FirkPivArgs<M> a{&T, I.params, mesh, y, sl, K, scr, loc, &sh.rel[0][0], I.pcnt, I.fam, N, lane, nest};
-        ps = firk_chunk_pivoted<M, S, -1>(a);
+        FirkPivArgs<M, NT> a{&T, I.params, mesh, y, sl, K, scr, loc, &sh.rel[0][0], I.pcnt, I.fam, N, lane, nest};
+        ps = firk_chunk_pivoted<M, S>(a);
         __syncthreads();
         rel_from_lds<M>(sh, lane, rel);
         __syncthreads();
     } else if constexpr (DIAG) {
+        if (sticky < 0) sticky = wave_any(firk_look<M, S>(I, T, mesh, y, N, lane));
         if (!sticky) {
             firk_chunk<M, S, false>(I, T, nest, sl, mesh, y, K, N, lane, scr, loc, rel, ps);
             sticky = wave_any(ps.piv);
             __syncthreads();  // the exchange area's LDS is the tree's next
         }
         if (sticky) {
-            FirkPivArgs<M> a{&T, I.params, mesh, y, sl, K, scr, loc, &sh.rel[0][0], I.pcnt, I.fam, N, lane, nest};
-            ps = nest.on ? firk_chunk_pivoted<M, S, 1>(a) : firk_chunk_pivoted<M, S, 0>(a);
+            FirkPivArgs<M, NT> a{&T, I.params, mesh, y, sl, K, scr, loc, &sh.rel[0][0], I.pcnt, I.fam, N, lane, nest};
+            ps = firk_chunk_pivoted<M, S>(a);
             __syncthreads();
             rel_from_lds<M>(sh, lane, rel);
             __syncthreads();
@@ -944,8 +1068,8 @@ enum { FIRK_STORE = 0, FIRK_APPLY = 1, FIRK_CHECK = 2 };
 
 // Tree solve of the condensed system: the corrections at the chunk ends in sh.lo, sh.hi.
 // Returns false when the root system is singular.
-template <int M, int S, bool IR>
-__device__ __forceinline__ bool firk_tree(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+template <int M, int S, bool IR, class NT>
+__device__ __forceinline__ bool firk_tree(const Inst<M> &I, const FirkTab &T, const NT &nest, Shared<M> &sh,
                                           const double *mesh, const double *y, const double *K, int N, int lane,
                                           double *scr, const double *loc, Rel<M> &rel) {
     int P, start, len;
@@ -969,18 +1093,18 @@ __device__ __forceinline__ bool firk_tree(const Inst<M> &I, const FirkTab &T, co
 
 // Back-substitution after firk_tree; fn receives max|F| at the new state (FIRK_CHECK; NaN if
 // not finite).
-template <int M, int S, bool DIAG, int MODE>
-__device__ __forceinline__ void firk_back(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+template <int M, int S, int MODE, class NT>
+__device__ __forceinline__ void firk_back(const Inst<M> &I, const FirkTab &T, const NT &nest, Shared<M> &sh,
                                           const double *mesh, double *y, double *K, int N, int lane,
                                           const double *scr, const double *loc, double *dy, double *dK,
                                           double *fn = nullptr) {
     constexpr int NN = S * M;
-    const bool nested = nest.on;
+    const bool nested = nest.on();
     double *sl = firk_slot<M, S>(sh, lane);
     int P, start, len;
     chunk_of(N, lane, P, start, len);
     double mx = 0.0;
-    bool bad = false, piv = false;
+    bool bad = false;
     // tree_solve ends on a barrier; its lo and hi lie outside the exchange area's LDS
     if (len > 0) {
         double ya[M], yn[M], yr[M], tr = 0.0;
@@ -992,6 +1116,8 @@ __device__ __forceinline__ void firk_back(const Inst<M> &I, const FirkTab &T, co
 #pragma unroll
             for (int c = 0; c < M; ++c) yr[c] = y[(size_t)(start + len) * M + c] + yn[c];
         }
+        // (a compiler fence: the node is the next lane's left end, written below)
+        if constexpr (MODE == FIRK_CHECK) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (lane == P - 1)
 #pragma unroll
             for (int c = 0; c < M; ++c) {
@@ -1040,13 +1166,9 @@ __device__ __forceinline__ void firk_back(const Inst<M> &I, const FirkTab &T, co
             }
             if constexpr (MODE == FIRK_CHECK) {
                 const double tl = mesh[k], h = tr - tl;
-                if (nested) {
-                    firk_inner<M, S, kFirkSlotLds<M, S>, !DIAG>(I, T, nest, sl, tl, h, yl, Kk, piv);
-                    store_stages<M, S>(K, ko, Kk);
-                }
                 double G[S][M], Phi[M], J[S][M][M];
                 firk_interval<M, S, false>(I, T, sl, tl, h, yl, yr, Kk, G, Phi, J);
-                firk_fold<M, S>(Phi, G, nested, mx, bad);
+                firk_fold<M, S>(Phi, G, false, mx, bad);
                 tr = tl;
 #pragma unroll
                 for (int c = 0; c < M; ++c) yr[c] = yl[c];
@@ -1064,63 +1186,105 @@ __device__ __forceinline__ void firk_back(const Inst<M> &I, const FirkTab &T, co
         }
         const bool anybad = wave_any(bad);
         mx = wave_max(mx);
-        // an inner solve that needs row exchanges: not known to have converged, the next
-        // forward pass decides
-        *fn = wave_any(piv) ? 1.7976931348623157e308 : uniform(anybad ? NAN : mx);
+        *fn = uniform(anybad ? NAN : mx);
         __syncthreads();
     }
 }
 
 
-// Sum of squares of the residual at (y + alpha dy, K + alpha dK) (the line search's
-// merit, times 2) in all lanes; NaN if not finite.
-template <int M, int S>
-__device__ inline double firk_trial_sumsq(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
-                                          const double *mesh, const double *y, const double *K, const double *dy,
-                                          const double *dK, double alpha, int N, int lane) {
+// Sum of squares and largest entry of this lane's intervals' residual at
+// (y + alpha dy + beta gy, K + alpha dK + beta gK) (TWO: with the second direction).  Out of line
+// (a line search calls it from several places) but for the smallest systems, its arguments by
+// value as above.
+struct FirkTrial {
+    double ss, mx;
+};
+template <int M, class NT> struct FirkTrialArgs {
+    const FirkTab *T;
+    const double *params, *mesh, *y, *K, *dy, *dK, *gy, *gK;
+    double *sl;
+    double alpha, beta;
+    int pcnt, fam, N, lane;
+    NT nest;
+};
+template <int M, int S, bool TWO, class NT>
+__device__ __forceinline__ FirkTrial firk_trial_body(const FirkTrialArgs<M, NT> &a) {
+    Inst<M> I;
+    firk_inst<M, true>(a.params, a.pcnt, a.fam, I);
+    I.params = a.params;
+    I.pcnt = a.pcnt;
+    const FirkTab &T = firk_tab_uniform(*a.T);
+    const double *mesh = uni(a.mesh), *y = uni(a.y), *K = uni(a.K), *dy = uni(a.dy), *dK = uni(a.dK);
+    const double *gy = TWO ? uni(a.gy) : nullptr, *gK = TWO ? uni(a.gK) : nullptr;
+    double *sl = as_lds(a.sl);
+    const double alpha = uniform(a.alpha), beta = uniform(a.beta);
+    const int N = uni(a.N), lane = a.lane;
     int P, start, len;
     chunk_of(N, lane, P, start, len);
-    double *sl = firk_slot<M, S>(sh, lane);
-    double ss = 0.0;
-    bool bad = false, piv = false;
+    FirkTrial r{0.0, 0.0};
+    bool piv = false;
     for (int i = 0; i < len; ++i) {
         const int k = start + i;
         const double ti = mesh[k], h = mesh[k + 1] - ti;
         double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
         for (int c = 0; c < M; ++c) {
-            yi[c] = y[(size_t)k * M + c] + alpha * dy[(size_t)k * M + c];
-            yj[c] = y[(size_t)(k + 1) * M + c] + alpha * dy[(size_t)(k + 1) * M + c];
+            const size_t p = (size_t)k * M + c, q = p + M;
+            yi[c] = y[p] + alpha * dy[p];
+            yj[c] = y[q] + alpha * dy[q];
+            if constexpr (TWO) {
+                yi[c] += beta * gy[p];
+                yj[c] += beta * gy[q];
+            }
         }
-        if (nest.on) {
-            firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
+        if (a.nest.on()) {
+            firk_inner<M, S, true, true>(I, T, a.nest, sl, ti, h, yi, Kk, piv);
         } else {
             const size_t ko = firk_off<S * M>(lane, i);
 #pragma unroll
-            for (int r = 0; r < S; ++r)
-#pragma unroll
-                for (int c = 0; c < M; ++c) {
-                    const size_t q = ko + (size_t)(r * M + c) * WAVE;
-                    Kk[r][c] = K[q] + alpha * dK[q];
-                }
+            for (int q = 0; q < S * M; ++q) {
+                const size_t o = ko + (size_t)q * WAVE;
+                Kk[q / M][q % M] = K[o] + alpha * dK[o];
+                if constexpr (TWO) Kk[q / M][q % M] += beta * gK[o];
+            }
         }
         firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
 #pragma unroll
-        for (int c = 0; c < M; ++c) ss += Phi[c] * Phi[c];
-        if (!nest.on) {
+        for (int c = 0; c < M; ++c) { r.ss += Phi[c] * Phi[c]; r.mx = fmax(r.mx, fabs(Phi[c])); }
+        if (!a.nest.on()) {
 #pragma unroll
-            for (int r = 0; r < S; ++r)
+            for (int q = 0; q < S; ++q)
 #pragma unroll
-                for (int c = 0; c < M; ++c) ss += G[r][c] * G[r][c];
+                for (int c = 0; c < M; ++c) { r.ss += G[q][c] * G[q][c]; r.mx = fmax(r.mx, fabs(G[q][c])); }
         }
     }
+    return r;
+}
+template <int M, int S, bool TWO, class NT>
+__device__ __noinline__ FirkTrial firk_trial_out(FirkTrialArgs<M, NT> a) {
+    return firk_trial_body<M, S, TWO>(a);
+}
+template <int M, int S, bool TWO, class NT>
+__device__ __forceinline__ FirkTrial firk_trial_part(const FirkTrialArgs<M, NT> &a) {
+    if constexpr (S * M <= 4) return firk_trial_body<M, S, TWO>(a);
+    else return firk_trial_out<M, S, TWO>(a);
+}
+
+// Sum of squares of the residual at (y + alpha dy, K + alpha dK) (the line search's
+// merit, times 2) in all lanes; NaN if not finite.
+template <int M, int S, class NT>
+__device__ __forceinline__ double firk_trial_sumsq(const Inst<M> &I, const FirkTab &T, const NT &nest, Shared<M> &sh,
+                                                   const double *mesh, const double *y, const double *K,
+                                                   const double *dy, const double *dK, double alpha, int N, int lane) {
+    FirkTrialArgs<M, NT> a{&T, I.params, mesh, y, K, dy, dK, nullptr, nullptr, firk_slot<M, S>(sh, lane),
+                           alpha, 0.0, I.pcnt, I.fam, N, lane, nest};
+    double ss = firk_trial_part<M, S, false>(a).ss;
     if (lane < M) {
         const BcLoc L = bc_locate<M>(I, lane, mesh, N);
         const double v = firk_bc_row<M, S>(I, T, nest, mesh, y, K, dy, dK, alpha, lane, L, N);
         ss += v * v;
     }
-    bad = !(fabs(ss) <= 1.7976931348623157e308);
-    const bool anybad = wave_any(bad);
+    const bool anybad = wave_any(!(fabs(ss) <= 1.7976931348623157e308));
     ss = wave_sum(ss);
     return uniform(anybad ? NAN : ss);
 }
@@ -1164,12 +1328,7 @@ struct FirkNewtonOut {
 
 // ------------------------------------------------------------------ trust region (expanded form)
 // the expanded form with boundary rows anywhere in the span
-template <int M> __device__ inline FirkNest<M> firk_expanded_rows() {
-    FirkNest<M> n{};
-    n.on = false;
-    n.irows = true;
-    return n;
-}
+template <int M> __device__ inline FirkNest<M, 0, true> firk_expanded_rows() { return {}; }
 
 // Products with the expanded Jacobian for the TrustRegion stage, rows
 //   Phi_i = y_{i+1} - y_i - h sum_j b_j K_ij,  G_ir = f(t_i + c_r h, Y_ir) - K_ir,
@@ -1177,7 +1336,7 @@ template <int M> __device__ inline FirkNest<M> firk_expanded_rows() {
 // (the Jacobian of FIRK/collocation.jl:59-93 that the oracle assembles), stage
 // Jacobians J_r evaluated at (y, K).  firk_jt_f: g = J'F into (gy [N+1][M], gK [N][S][M]).
 template <int M, int S>
-__device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
+__device__ __forceinline__ void firk_jt_f(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
                                  const double *y, const double *K, int N, int lane, double *gy, double *gK) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
@@ -1258,7 +1417,7 @@ __device__ inline void firk_jt_f(const Inst<M> &I, const FirkTab &T, Shared<M> &
 
 // |J g|^2 for g = (gy, gK), in all lanes
 template <int M, int S>
-__device__ inline double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
+__device__ __forceinline__ double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
                                         const double *y, const double *K, const double *gy, const double *gK, int N,
                                         int lane) {
     int P, start, len;
@@ -1322,50 +1481,23 @@ __device__ inline double firk_jac_norm2(const Inst<M> &I, const FirkTab &T, Shar
 
 // |F|^2 and max|F| at (y + a dy + b gy, K + a dK + b gK), in all lanes (NaN if not finite)
 template <int M, int S>
-__device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
-                                     const double *y, const double *K, const double *dy, const double *dK, double a, const double *gy,
-                                     const double *gK, double b, int N, int lane, double &mx) {
-    int P, start, len;
-    chunk_of(N, lane, P, start, len);
-    double *sl = firk_slot<M, S>(sh, lane);
-    double ss = 0.0, m = 0.0;
-    for (int i = 0; i < len; ++i) {
-        const int k = start + i;
-        const size_t ko = firk_off<S * M>(lane, i);
-        const double ti = mesh[k], h = mesh[k + 1] - ti;
-        double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
-#pragma unroll
-        for (int c = 0; c < M; ++c) {
-            const size_t p = (size_t)k * M + c, q = (size_t)(k + 1) * M + c;
-            yi[c] = y[p] + a * dy[p] + b * gy[p];
-            yj[c] = y[q] + a * dy[q] + b * gy[q];
-        }
-#pragma unroll
-        for (int r = 0; r < S; ++r)
-#pragma unroll
-            for (int c = 0; c < M; ++c) {
-                const size_t q = ko + (size_t)(r * M + c) * WAVE;
-                Kk[r][c] = K[q] + a * dK[q] + b * gK[q];
-            }
-        firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
-#pragma unroll
-        for (int c = 0; c < M; ++c) { ss += Phi[c] * Phi[c]; m = fmax(m, fabs(Phi[c])); }
-#pragma unroll
-        for (int r = 0; r < S; ++r)
-#pragma unroll
-            for (int c = 0; c < M; ++c) { ss += G[r][c] * G[r][c]; m = fmax(m, fabs(G[r][c])); }
-    }
+__device__ __forceinline__ double firk_trial2(const Inst<M> &I, const FirkTab &T, Shared<M> &sh, const double *mesh,
+                                              const double *y, const double *K, const double *dy, const double *dK,
+                                              double a, const double *gy, const double *gK, double b, int N, int lane,
+                                              double &mx) {
+    const auto nest = firk_expanded_rows<M>();
+    FirkTrialArgs<M, FirkNest<M, 0, true>> t{&T, I.params, mesh, y, K, dy, dK, gy, gK, firk_slot<M, S>(sh, lane),
+                                             a, b, I.pcnt, I.fam, N, lane, nest};
+    FirkTrial r = firk_trial_part<M, S, true>(t);
     if (lane < M) {
         const BcLoc L = bc_locate<M>(I, lane, mesh, N);
-        const double v =
-            firk_bc_row<M, S>(I, T, firk_expanded_rows<M>(), mesh, y, K, dy, dK, a, lane, L, N, gy, gK, b);
-        ss += v * v;
-        m = fmax(m, fabs(v));
+        const double v = firk_bc_row<M, S>(I, T, nest, mesh, y, K, dy, dK, a, lane, L, N, gy, gK, b);
+        r.ss += v * v;
+        r.mx = fmax(r.mx, fabs(v));
     }
-    const bool bad = !(fabs(ss) <= 1.7976931348623157e308);
-    const bool anybad = wave_any(bad);
-    ss = uniform(wave_sum(ss));
-    mx = anybad ? NAN : uniform(wave_max(m));
+    const bool anybad = wave_any(!(fabs(r.ss) <= 1.7976931348623157e308));
+    const double ss = uniform(wave_sum(r.ss));
+    mx = anybad ? NAN : uniform(wave_max(r.mx));
     __syncthreads();
     return anybad ? NAN : ss;
 }
@@ -1375,9 +1507,9 @@ __device__ inline double firk_trial2(const Inst<M> &I, const FirkTab &T, Shared<
 // radius update; the restatement the oracle follows, Core/default_internal_solve.jl:
 // 37-43).  Boundary rows anywhere in the span.
 // gy, gK: work areas for J'F.
-template <int M, int S, bool DIAG>
-__device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, const FirkTab &T,
-                                        const FirkNest<M> &nest, Shared<M> &sh, const double *mesh, double *y,
+template <int M, int S, bool DIAG, class NT>
+__device__ __forceinline__ int firk_trust_region(const BatchDev &B, const Inst<M> &I, const FirkTab &T,
+                                        const NT &nest, Shared<M> &sh, const double *mesh, double *y,
                                         double *K, int N, int lane, double *scr, double *loc, double *dy, double *dK,
                                         double *gy, double *gK, FirkNewtonOut &out) {
     double mx;
@@ -1395,7 +1527,8 @@ __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, con
     __syncthreads();
     double radius = fmax(sqrt(ss), xmax - xmin) / 11.0;
     int shrinks = 0;
-    bool fresh = true, sticky = false;
+    bool fresh = true;
+    int sticky = -1;
     double dn2 = 0.0, l2 = 0.0, gdn = 0.0, jg2 = 0.0;
     for (int it = 0;; ++it) {
         out.fn = mx;
@@ -1407,7 +1540,7 @@ __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, con
             bool sing = false;
             firk_forward<M, S, DIAG>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing, sticky);
             if (sing || !firk_tree<M, S, false>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel)) return BVP_RET_FAILURE;
-            firk_back<M, S, DIAG, FIRK_STORE>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
+            firk_back<M, S, FIRK_STORE>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
             firk_jt_f<M, S>(I, T, sh, mesh, y, K, N, lane, gy, gK);
             double a = 0.0, b = 0.0, c = 0.0;
             for (int q = lane; q < (N + 1) * M; q += WAVE) {
@@ -1479,23 +1612,24 @@ __device__ inline int firk_trust_region(const BatchDev &B, const Inst<M> &I, con
 // plain, then with the BackTracking line search, each from the same start, stopping
 // when max|F| <= tol (checked before every step).  Work areas: dy [cap][M], dK, the
 // start copy y0 [cap][M], K0, loc.
-template <int M, int S, bool IR, bool DIAG>
-__device__ inline FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I, const FirkTab &T,
-                                            const FirkNest<M> &nest, Shared<M> &sh, const double *mesh, double *y,
+template <int M, int S, bool IR, bool DIAG, class NT>
+__device__ __forceinline__ FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I, const FirkTab &T,
+                                            const NT &nest, Shared<M> &sh, const double *mesh, double *y,
                                             double *K, int N, int lane, double *scr, double *loc, double *dy,
                                             double *dK, double *y0, double *K0) {
     FirkNewtonOut out{BVP_RET_MAXITERS, 0, -1, NAN};
     // the TrustRegion stage: compiled into the general kernels (IR) only
     const int stages = B.stages & (IR ? 7 : 3);
-    bool first = true, sticky = false;
+    bool first = true;
+    int sticky = -1;
     if (__popc(stages) > 1) firk_copy_state<M, S>(y0, K0, y, K, N, lane);
     for (int st = 0; st < 3; ++st) {
         if (!(stages & (1 << st))) continue;
         if (!first) firk_copy_state<M, S>(y, K, y0, K0, N, lane);
         first = false;
         out.stage = st;
-        if constexpr (IR) {
-            if (st == 2 && !nest.on) {
+        if constexpr (IR && NT::form == 0) {
+            if (st == 2) {
                 // the last stage: the start copy is free for J'F
                 out.ret = firk_trust_region<M, S, DIAG>(B, I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, y0, K0,
                                                   out);
@@ -1515,29 +1649,32 @@ __device__ inline FirkNewtonOut firk_newton(const BatchDev &B, const Inst<M> &I,
                 break;
             }
             out.iters++;
-            if (st == 0 && fn <= 100.0 * sqrt(B.newton_tol)) {
+            if (st == 0 && !nest.on() && fn <= 100.0 * sqrt(B.newton_tol)) {
                 // a step predicted to converge (as in the MIRK path: quadratic convergence with
                 // a constant of 1e-4): the residual at the new state is evaluated with the
                 // update, which spares the forward pass that would only find it converged
+                // (2,048 linear problems, s = 5: M = 3 12.1 -> 9.9 ms, M = 4 34.6 -> 28.3 ms; not in
+                // the nested form, where the inner solves are the cost of either: M = 2, s = 5,
+                // 4,096 Bratu problems 2.66 -> 1.52 ms without)
                 double fn2 = NAN;
-                firk_back<M, S, DIAG, FIRK_CHECK>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, &fn2);
+                firk_back<M, S, FIRK_CHECK>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK, &fn2);
                 out.fn = fn2;
                 if (!(fabs(fn2) <= 1.7976931348623157e308)) { out.ret = BVP_RET_UNSTABLE; break; }
                 if (fn2 <= B.newton_tol) { out.ret = BVP_RET_SUCCESS; break; }
                 continue;
             }
             if (st == 0) {
-                firk_back<M, S, DIAG, FIRK_APPLY>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
+                firk_back<M, S, FIRK_APPLY>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
                 continue;
             }
-            firk_back<M, S, DIAG, FIRK_STORE>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
+            firk_back<M, S, FIRK_STORE>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, dy, dK);
             double alpha = 1.0;
             const double ss = firk_trial_sumsq<M, S>(I, T, nest, sh, mesh, y, K, dy, dK, 0.0, N, lane);
             auto phi = [&](double a) {
                 return 0.5 * firk_trial_sumsq<M, S>(I, T, nest, sh, mesh, y, K, dy, dK, a, N, lane);
             };
             if (!backtracking(phi, 0.5 * ss, -ss, alpha)) { out.ret = BVP_RET_FAILURE; break; }
-            firk_apply<M, S>(y, K, dy, dK, alpha, N, lane, nest.on);
+            firk_apply<M, S>(y, K, dy, dK, alpha, N, lane, nest.on());
         }
         if (out.ret == BVP_RET_SUCCESS) break;
     }
@@ -1576,7 +1713,7 @@ __device__ inline void firk_eval_q(const FirkTab &T, const double *yi, double ta
 // FIRK/adaptivity.jl:247-300) and, when errs is set, the vectors; r1, r2 the max and
 // sum of shat.  Returns the defect norm (NaN-aware) in all lanes.
 template <int M, int S>
-__device__ inline double firk_defect_pass(const Inst<M> &I, const FirkTab &T, const double *mesh, const double *y,
+__device__ __forceinline__ double firk_defect_pass(const Inst<M> &I, const FirkTab &T, const double *mesh, const double *y,
                                           const double *K, int N, int lane, double abstol, double *shat,
                                           double *errs, double &r1, double &r2) {
     int P, start, len;
@@ -1631,12 +1768,12 @@ __device__ inline double firk_defect_pass(const Inst<M> &I, const FirkTab &T, co
 // (FIRK/adaptivity.jl:8-135): the quintic of interval(mesh, t) through y_i, y_{i+1},
 // f(y_i), f(y_{i+1}) and the stage polynomial at the midpoint.  hscale multiplies the
 // interval's step in the stage polynomial and the quintic (the nested form's transfer
-// passes the reference's growth factor, FIRK/adaptivity.jl:98-104); with nest.on the
+// passes the reference's growth factor, FIRK/adaptivity.jl:98-104); with nest.on() the
 // stages come from the inner solve (at the unscaled step), else from K.
 // K: the stages in [interval][S][M] order (PLAIN: the dense output's packed input), or the
 // lane-interleaved state.
-template <int M, int S, bool PLAIN>
-__device__ inline void firk_interp_at(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, const double *mesh,
+template <int M, int S, bool PLAIN, class NT>
+__device__ __forceinline__ void firk_interp_at(const Inst<M> &I, const FirkTab &T, const NT &nest, const double *mesh,
                                       const double *y, const double *K, int N, double t, double *u, double *du,
                                       double hscale = 1.0) {
     const int j = interval_of(mesh, N, t);
@@ -1644,14 +1781,16 @@ __device__ inline void firk_interp_at(const Inst<M> &I, const FirkTab &T, const 
     double yi[M], yj[M], fi[M], fj[M], z[M], zp[M], Kk[S][M];
 #pragma unroll
     for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)j * M + c]; yj[c] = y[(size_t)(j + 1) * M + c]; }
-    if (nest.on && !K) {
-        bool piv = false;
-        firk_inner<M, S, false, true>(I, T, nest, nullptr, tj, h0, yi, Kk, piv);
-    } else if constexpr (PLAIN) {
+    if constexpr (PLAIN) {
+        if (nest.on()) {
+            bool piv = false;
+            firk_inner<M, S, false, true>(I, T, nest, nullptr, tj, h0, yi, Kk, piv);
+        } else {
 #pragma unroll
-        for (int r = 0; r < S; ++r)
+            for (int r = 0; r < S; ++r)
 #pragma unroll
-            for (int c = 0; c < M; ++c) Kk[r][c] = K[((size_t)j * S + r) * M + c];
+                for (int c = 0; c < M; ++c) Kk[r][c] = K[((size_t)j * S + r) * M + c];
+        }
     } else {
         load_stages<M, S>(K, firk_off<S * M>(N, j, true), Kk);
     }
@@ -1694,8 +1833,8 @@ __device__ inline void firk_extend(const double *y, double *K, int N, int lane) 
 }
 
 // max|F| at (y, K) (NaN if not finite); the nested form's stages are solved into K
-template <int M, int S>
-__device__ inline double firk_residual_max(const Inst<M> &I, const FirkTab &T, const FirkNest<M> &nest, Shared<M> &sh,
+template <int M, int S, class NT>
+__device__ __forceinline__ double firk_residual_max(const Inst<M> &I, const FirkTab &T, const NT &nest, Shared<M> &sh,
                                            const double *mesh, const double *y, double *K, int N, int lane) {
     int P, start, len;
     chunk_of(N, lane, P, start, len);
@@ -1709,14 +1848,14 @@ __device__ inline double firk_residual_max(const Inst<M> &I, const FirkTab &T, c
         double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
         for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
-        if (nest.on) {
-            firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
+        if (nest.on()) {
+            firk_inner<M, S, true, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
             store_stages<M, S>(K, ko, Kk);
         } else {
             load_stages<M, S>(K, ko, Kk);
         }
         firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
-        firk_fold<M, S>(Phi, G, nest.on, mx, bad);
+        firk_fold<M, S>(Phi, G, nest.on(), mx, bad);
     }
     __syncthreads();
     firk_bc_rows<M, S>(I, T, nest, sh, mesh, y, K, N, lane);
@@ -1737,16 +1876,14 @@ __device__ inline double firk_residual_max(const Inst<M> &I, const FirkTab &T, c
 // extend_y sets them for a new problem), or halving with a zero restart when Newton or
 // the defect threshold failed.
 template <int M, int S, bool NEST, bool IR, bool DIAG>
-__device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, int b, Shared<M> &sh, int lane,
+__device__ __forceinline__ void firk_solve_instance(const BatchDev &B, const FirkTab &T, int b, Shared<M> &sh, int lane,
                                            double *scr, double *aux) {
     Inst<M> I;
     load_inst<M>(B, b, I);
     I.minc = 1;
     Bufs<M> bf = bufs_of<M>(B, b);
     double *K = firk_stages_of<M, S>(B, b);
-    FirkNest<M> nest = firk_nest_of<M>(B, b);
-    nest.on = NEST;  // compile-time forms: the expanded kernels carry no inner-solve code,
-    nest.irows = IR;  // and kernels for batches without interior rows no EvalSol code
+    const auto nest = firk_nest_of<M, NEST ? 1 : 0, IR>(B, b);
     // node areas [cap][M]; interval areas lane-interleaved
     const size_t cap = (size_t)B.cap, icap = firk_pad(B.cap);
     double *dy = aux;
@@ -1765,7 +1902,7 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
             for (int c = 0; c < M; ++c) bf.y[0][(size_t)k * M + c] = B.init_y[(off + k) * M + c];
         }
         __syncthreads();
-        if (!nest.on) firk_extend<M, S>(bf.y[0], K, N, lane);
+        if (!nest.on()) firk_extend<M, S>(bf.y[0], K, N, lane);
     }
     int info = BVP_RET_SUCCESS, nl_ret = BVP_RET_SUCCESS;
     int outer = 0, iters = 0, fb = 0;
@@ -1805,11 +1942,11 @@ __device__ inline void firk_solve_instance(const BatchDev &B, const FirkTab &T, 
                     // the nested form restates interp_eval! with its step scaled by the growth
                     // of the node count (FIRK/adaptivity.jl:98-104); the expanded form's
                     // restart is the interpolated nodes with extend_y's stages
-                    const double hs = (nest.on && Nn > N) ? (double)Nn / (double)N : 1.0;
+                    const double hs = (nest.on() && Nn > N) ? (double)Nn / (double)N : 1.0;
                     for (int j = lane; j <= Nn; j += WAVE)
                         firk_interp_at<M, S, false>(I, T, nest, mesh, y, K, N, mesh_o[j], y_o + (size_t)j * M, nullptr, hs);
                     __syncthreads();
-                    if (!nest.on) firk_extend<M, S>(y_o, K, Nn, lane);
+                    if (!nest.on()) firk_extend<M, S>(y_o, K, Nn, lane);
                     cnt_tr += N + Nn;
                     N = Nn;
                     cur = 1 - cur;
@@ -1915,11 +2052,11 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
         const double *y = as_global(B.init_y + off * M);
         const size_t icap = firk_pad(B.cap);
         double *dy = aux, *dK = dy + 2 * cap * M, *K = dK + icap * S * M, *loc = K + icap * S * M;
-        const FirkNest<M> nest = firk_nest_of<M>(B, b);
+        const auto nest = firk_nest_of<M, -1, true>(B, b);
         double *sl = firk_slot<M, S>(sh, lane);
         // the stage state in the slot: the packed input lane-interleaved, or (nested) the
         // inner solves' stages
-        if (!nest.on) {
+        if (!nest.on()) {
             const double *Ki = as_global(B.init_K + ioff * S * M);
             int P, start, len;
             chunk_of(N, lane, P, start, len);
@@ -1928,8 +2065,8 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
                     K[firk_off<S * M>(lane, i) + (size_t)q * WAVE] = Ki[(size_t)(start + i) * S * M + q];
             __syncthreads();
         }
-        const size_t xo = nest.on ? (size_t)M * off : (size_t)M * ((size_t)(S + 1) * ioff + b);  // slot offset
-        const int rowlen = nest.on ? M : (S + 1) * M;  // residual entries per interval
+        const size_t xo = nest.on() ? (size_t)M * off : (size_t)M * ((size_t)(S + 1) * ioff + b);  // slot offset
+        const int rowlen = nest.on() ? M : (S + 1) * M;  // residual entries per interval
         if (op == OP_RESIDUAL) {
             double *out = B.out0 + xo;
             int nbca = 0;
@@ -1946,13 +2083,13 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
                 double yi[M], yj[M], Kk[S][M], G[S][M], Phi[M], J[S][M][M];
 #pragma unroll
                 for (int c = 0; c < M; ++c) { yi[c] = y[(size_t)k * M + c]; yj[c] = y[(size_t)(k + 1) * M + c]; }
-                if (nest.on) firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
+                if (nest.on()) firk_inner<M, S, true, true>(I, T, nest, sl, ti, h, yi, Kk, piv);
                 else load_stages<M, S>(K, firk_off<S * M>(lane, i), Kk);
                 firk_interval<M, S, false>(I, T, sl, ti, h, yi, yj, Kk, G, Phi, J);
                 double *o = out + nbca + (size_t)k * rowlen;
 #pragma unroll
                 for (int c = 0; c < M; ++c) o[c] = Phi[c];
-                if (!nest.on) {
+                if (!nest.on()) {
 #pragma unroll
                     for (int r = 0; r < S; ++r)
 #pragma unroll
@@ -1973,24 +2110,25 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
             }
         } else if (op == OP_NEWTON_STEP) {
             Rel<M> rel;
-            bool sing = false, sticky = false;
+            bool sing = false;
+            int sticky = -1;
             firk_forward<M, S, false>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel, sing, sticky);
             const bool ok = !sing && firk_tree<M, S, true>(I, T, nest, sh, mesh, y, K, N, lane, scr, loc, rel);
             if (ok)
-                firk_back<M, S, false, FIRK_STORE>(I, T, nest, sh, mesh, const_cast<double *>(y), K, N, lane, scr, loc, dy,
+                firk_back<M, S, FIRK_STORE>(I, T, nest, sh, mesh, const_cast<double *>(y), K, N, lane, scr, loc, dy,
                                                    dK);
             double *out = B.out0 + xo;
             for (int q = lane; q < (N + 1) * M; q += WAVE) {
                 const int i = q / M, c = q % M;
                 out[(size_t)i * rowlen + c] = ok ? dy[q] : NAN;
             }
-            for (int q = lane; q < (nest.on ? 0 : N * S * M); q += WAVE) {
+            for (int q = lane; q < (nest.on() ? 0 : N * S * M); q += WAVE) {
                 const int i = q / (S * M), rc = q % (S * M);
                 out[(size_t)i * (S + 1) * M + M + rc] =
                     ok ? dK[firk_off<S * M>(N, i, true) + (size_t)rc * WAVE] : NAN;
             }
         } else if (op == OP_DEFECT) {
-            if (nest.on) {
+            if (nest.on()) {
                 // the stages from the inner solves, as defect_estimate! solves them
                 // (FIRK/adaptivity.jl:465-517)
                 int P, start, len;
@@ -2001,7 +2139,7 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
                     double yi[M], Kk[S][M];
 #pragma unroll
                     for (int c = 0; c < M; ++c) yi[c] = y[(size_t)k * M + c];
-                    firk_inner<M, S, kFirkSlotLds<M, S>, true>(I, T, nest, sl, mesh[k], mesh[k + 1] - mesh[k], yi, Kk, piv);
+                    firk_inner<M, S, true, true>(I, T, nest, sl, mesh[k], mesh[k + 1] - mesh[k], yi, Kk, piv);
                     store_stages<M, S>(K, firk_off<S * M>(lane, i), Kk);
                 }
                 __syncthreads();
@@ -2031,8 +2169,8 @@ __global__ __launch_bounds__(256) void k_firk_interp(BatchDev B, const int *qins
     const double *y = as_global(B.init_y + off * M);
     const int N = B.N0[b];
     const double t = tq[q];
-    const FirkNest<M> nest = firk_nest_of<M>(B, b);
-    const double *K = nest.on ? nullptr : as_global(B.init_K + ioff * S * M);
+    const auto nest = firk_nest_of<M, -1, true>(B, b);
+    const double *K = nest.on() ? nullptr : as_global(B.init_K + ioff * S * M);
     double u[M], du[M];
     firk_interp_at<M, S, true>(I, T, nest, mesh, y, K, N, t, u, du);
 #pragma unroll

@@ -83,16 +83,6 @@ template <int M, int METHOD, typename LT> __device__ __forceinline__ BShared<M, 
     return sh;
 }
 
-// values and pointers (into global memory) that are the same in every lane, in scalar
-// registers: arguments of functions that are not inlined arrive in vector registers
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-template <typename T> __device__ __forceinline__ T *uni(T *p) {
-    const unsigned long long b = (unsigned long long)p;
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
-    return (T *)(__attribute__((address_space(1))) T *)(((unsigned long long)hi << 32) | lo);
-}
-
 // order LDS (and register) traffic between the lanes of one wave
 __device__ __forceinline__ void wsync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

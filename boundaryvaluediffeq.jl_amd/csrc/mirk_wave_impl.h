@@ -81,6 +81,16 @@ __device__ __forceinline__ T *as_global(T *p) {
     return (T *)(__attribute__((address_space(1))) T *)p;
 }
 
+// values and pointers (into global memory) that are the same in every lane, in scalar
+// registers: arguments of functions that are not inlined arrive in vector registers
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <typename T> __device__ __forceinline__ T *uni(T *p) {
+    const unsigned long long b = (unsigned long long)p;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    return (T *)(__attribute__((address_space(1))) T *)(((unsigned long long)hi << 32) | lo);
+}
+
 // a[k] for a runtime k without dynamic register indexing (which would move the
 // array to scratch memory)
 template <int N, typename T>
