@@ -20,6 +20,7 @@
 #include "../../include/bvp_mirk.h"
 #include "bvp_host.h"
 #include "bvp_internal.h"
+#include "firk_layout.h"
 #include "mirk_wave.h"
 
 namespace {
@@ -279,8 +280,9 @@ void PinnedStage::free_all() {
 // array, which each device holds from module load until the process ends.  Host
 // code reaches it only through the address hipGetSymbolAddress returns for the
 // context's device (bvp_ctx::noalloc); calls on one device share it.
-constexpr size_t kNoAllocBytes = (size_t)64 << 20;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+// (a FIRK batch has kFirkMargin more, for the lines its areas round up to)
+constexpr size_t kNoAllocBytes = (size_t)64 << 20, kFirkMargin = (size_t)512 << 10;
+static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kFirkMargin];
 
 // The per-instance scalars of a batch's results, back to back (on the device and in the
 // host copy alike).
@@ -299,6 +301,20 @@ struct ResultHead {
         fb = outer + n;
     }
 };
+
+// Waves of a FIRK batch in the no-allocation scratch.  The areas hold whole lines of 64
+// intervals (firk_layout.h); where they do not fit it with room for the results, fewer waves
+// take the instances: as many as do, and as many at least as packed areas of that many waves
+// would leave memory for, so that no batch is refused for the lines.
+static int firk_bump_slots(const DevArena &A, int n, int cap, int M, int S, size_t scratch, int slots) {
+    const size_t room = (A.bump_cap - A.bump_used) / sizeof(double), stage = bvpdev::firk_stage_values(n, cap, S * M);
+    const size_t gather = (size_t)n * cap * (1 + M + S * M) + 2 * ((size_t)n + 1) + 8 * 32;
+    const size_t packed = (size_t)cap * (2 * M + 2 * S * M + S * M * (M + 1)), per = scratch + bvpdev::firk_aux_values(cap, M, S);
+    const size_t fit = room > stage + gather ? (room - stage - gather) / per : 0;
+    const size_t all = (size_t)slots * (scratch + packed) + (size_t)n * cap * S * M;
+    const size_t least = all > stage ? (all - stage) / per : 0;
+    return (int)std::min<size_t>(slots, std::max<size_t>(1, std::max(fit, least)));
+}
 
 // ------------------------------------------------------------------ batch build
 int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *inst, int cap_req, bvp_batch **out,
@@ -327,6 +343,7 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
         }
     }
     const bool firk = bvphost::is_firk(o->method);
+    if (firk && bump) bump_cap += kFirkMargin;
     bvphost::FirkTableau ftab;
     if (firk) bvphost::firk_tableau(o->method, ftab);  // validate_opts accepted the code
     bool has_u0 = true;
@@ -462,7 +479,8 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
         const size_t lmax = std::max((rcap + 63) / 64, (size_t)(2 * kMaxMinChunk)) + 1;
         D.tree_base = lmax * NF * 64;
         D.scratch_per_slot = D.tree_base + (size_t)64 * NF;
-        D.aux_per_slot = firk ? firk_aux_doubles(cap, M, ftab.s) : (size_t)cap * (3 * M + 1);
+        D.aux_per_slot = firk ? bvpdev::firk_aux_values(cap, M, ftab.s) : (size_t)cap * (3 * M + 1);
+        if (firk && bump) slots = firk_bump_slots(A, n, cap, M, ftab.s, D.scratch_per_slot, slots);
         scratch_doubles = D.scratch_per_slot * slots;
         D.rec_cap = cap;
     } else {
@@ -498,17 +516,14 @@ int batch_build(bvp_ctx *ctx, const bvp_opts *o, int32_t n, const bvp_instance *
     D.hybrid_ge = o->hybrid_ge;
     D.ge_per_slot = ge ? wave_ge_doubles(cap, M) : 0;
     D.min_chunk = blk ? 1 : std::max(1, std::min(kMaxMinChunk, tuned_minc));
-    if ((rc = dalloc(ctx, A, D.scratch, scratch_doubles)) ||
+    if ((firk && (rc = dalloc(ctx, A, D.stK, bvpdev::firk_stage_values(n, cap, ftab.s * M)))) ||
+        (rc = dalloc(ctx, A, D.scratch, scratch_doubles)) ||
         (rc = dalloc(ctx, A, D.aux, D.aux_per_slot * slots)) ||
         (ge && (rc = dalloc(ctx, A, D.ge, D.ge_per_slot * slots)))) {
         delete B;
         return rc;
     }
     if (firk) {
-        if ((rc = dalloc(ctx, A, D.stK, (size_t)n * ((size_t)cap + 64) * ftab.s * M))) {
-            delete B;
-            return rc;
-        }
         D.firk_tab = dtab;
         D.firk_nested = nested;
         D.firk_irows = (o->nlsolve_stages & BVP_STAGE_TRUST_REGION) != 0;  // the stage lives in those kernels

@@ -28,16 +28,10 @@
 // problems 2.7 -> 1.4 ms.)
 #pragma once
 
+#include "firk_layout.h"
 #include "mirk_wave_impl.h"
 
 namespace bvpdev {
-
-// Per-interval data of a wave (stage values, their corrections, the condensation records)
-// is interleaved over the lanes that own the intervals: field q of interval k lies at
-// [step i][q][64 lanes] with k the i-th interval of its lane's chunk, so that the 64 lanes
-// walking their chunks read and write whole 512-byte lines.  (In [interval][field] order
-// every access of the wave touched 64 lines.)  An area holds firk_pad(cap) intervals.
-__host__ __device__ inline size_t firk_pad(int cap) { return (size_t)cap + WAVE; }
 
 struct FirkAt {
     int lane, i;
@@ -50,7 +44,7 @@ __device__ inline FirkAt firk_at(int N, int k) {
     return a;
 }
 // offset of field 0 of step i in an area of NF fields (field q: + q * WAVE)
-template <int NF> __device__ __forceinline__ size_t firk_off(int lane, int i) { return (size_t)i * (NF * WAVE) + lane; }
+template <int NF> __device__ __forceinline__ size_t firk_off(int lane, int i) { return firk_cell(lane, i, NF); }
 template <int NF> __device__ __forceinline__ size_t firk_off(int N, int k, bool) {
     const FirkAt a = firk_at(N, k);
     return firk_off<NF>(a.lane, a.i);
@@ -63,10 +57,10 @@ template <int NF, typename Fn> __device__ __forceinline__ void firk_each(int N, 
     for (int i = 0; i < len; ++i) fn(firk_off<NF>(lane, i));
 }
 
-// stage values of instance b (lane-interleaved, S M fields per interval)
+// stage values of instance b (S M fields per interval)
 template <int M, int S>
 __device__ inline double *firk_stages_of(const BatchDev &B, int b) {
-    return as_global(B.stK + (size_t)b * firk_pad(B.cap) * S * M);
+    return as_global(B.stK + firk_stage_base(b, B.cap, S * M));
 }
 
 // the batch's tableau, in constant memory for the compiler (no kernel writes it): uniform
@@ -1885,7 +1879,7 @@ __device__ __forceinline__ void firk_solve_instance(const BatchDev &B, const Fir
     double *K = firk_stages_of<M, S>(B, b);
     const auto nest = firk_nest_of<M, NEST ? 1 : 0, IR>(B, b);
     // node areas [cap][M]; interval areas lane-interleaved
-    const size_t cap = (size_t)B.cap, icap = firk_pad(B.cap);
+    const size_t cap = (size_t)B.cap, icap = firk_lines(firk_intervals(B.cap));
     double *dy = aux;
     double *y0 = dy + cap * M;
     double *dK = y0 + cap * M;
@@ -2050,7 +2044,7 @@ __global__ __launch_bounds__(64, 1) void k_firk_component(BatchDev B, int op) {
         const long long ioff = off - b;  // interval offset
         const double *mesh = as_global(B.init_mesh + off);
         const double *y = as_global(B.init_y + off * M);
-        const size_t icap = firk_pad(B.cap);
+        const size_t icap = firk_lines(firk_intervals(B.cap));
         double *dy = aux, *dK = dy + 2 * cap * M, *K = dK + icap * S * M, *loc = K + icap * S * M;
         const auto nest = firk_nest_of<M, -1, true>(B, b);
         double *sl = firk_slot<M, S>(sh, lane);

@@ -57,7 +57,7 @@ struct BatchDev {
     size_t scratch_per_slot;  // doubles (block kernels: bytes)
     size_t tree_base;         // offset of the tree records inside a slot
     double *aux;              // [slot][cap*(3M+1)]: delta, trial state, transfer indices, J'F
-                              //   (block kernels: their own layout)
+                              //   (block kernels: block_aux_doubles, FIRK kernels: firk_aux_values)
     size_t aux_per_slot;
     unsigned *counter;        // work-queue head
 
@@ -87,7 +87,7 @@ struct BatchDev {
     size_t ge_per_slot;
 
     // FIRK methods (expanded form): the tableau (a FirkTab in device memory), the stage
-    // values of every instance (cap + 64 intervals each, lane-interleaved), and for the component kernels the packed
+    // values of every instance (firk_layout.h), and for the component kernels the packed
     // input stages [sum N][s][M] (interval offset = init_off[b] - b)
     const void *firk_tab;
     double *stK;
@@ -142,12 +142,6 @@ hipError_t firk_launch_interp(const BatchDev &B, int S, const int *qinst, const 
                               long long nq, hipStream_t s);
 hipError_t firk_launch_gather(const BatchDev &B, int S, const long long *out_off, double *out, hipStream_t s);
 int firk_blocks_per_cu(int M, int S, int variant, int nested);  // resident solve waves per CU
-// doubles per slot of the FIRK work area for node capacity cap
-inline size_t firk_aux_doubles(int cap, int M, int S) {
-    // node areas of cap nodes, lane-interleaved interval areas of cap + 64 intervals
-    return (size_t)cap * (2 * M) + ((size_t)cap + 64) * (2 * S * M + S * M * (M + 1));
-}
-
 hipError_t launch_copy_probe(const double *src, double *dst, size_t n, hipStream_t s);
 
 // block kernels (M = 8, 16, 32; LINEAR_TANH): precision 0 = FP64 factors, 1 = FP32 factors + FP64 refinement
