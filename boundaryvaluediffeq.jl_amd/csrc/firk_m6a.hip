@@ -1,5 +1,5 @@
 // firk_m6a.hip -- the FIRK collocation kernels (expanded and nested forms) for state dimension
-// M = 6, stage counts 1-3 (firk_m6b.hip: 4, 5, 7; two files so that they compile in parallel).
+// M = 6, stage counts 1 and 2 (firk_m6b.hip: 3, 4; firk_m6c.hip: 5, 7; they compile in parallel).
 #include "firk_wave_impl.h"
 
 namespace bvpdev {
@@ -14,6 +14,5 @@ namespace bvpdev {
     template int firk_occupancy_t<6, S, 2>(int);
 FIRK_INST(1)
 FIRK_INST(2)
-FIRK_INST(3)
 #undef FIRK_INST
 }  // namespace bvpdev

@@ -1,5 +1,5 @@
 // firk_m6b.hip -- the FIRK collocation kernels (expanded and nested forms) for state dimension
-// M = 6, stage counts 4, 5 and 7 (firk_m6a.hip: 1-3).
+// M = 6, stage counts 3 and 4.
 #include "firk_wave_impl.h"
 
 namespace bvpdev {
@@ -12,8 +12,7 @@ namespace bvpdev {
     template hipError_t firk_launch_gather_t<6, S>(const BatchDev &, const long long *, double *, hipStream_t); \
     template int firk_occupancy_t<6, S, 1>(int);                                                              \
     template int firk_occupancy_t<6, S, 2>(int);
+FIRK_INST(3)
 FIRK_INST(4)
-FIRK_INST(5)
-FIRK_INST(7)
 #undef FIRK_INST
 }  // namespace bvpdev

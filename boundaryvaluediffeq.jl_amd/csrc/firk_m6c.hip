@@ -1,0 +1,18 @@
+// firk_m6c.hip -- the FIRK collocation kernels (expanded and nested forms) for state dimension
+// M = 6, stage counts 5 and 7.
+#include "firk_wave_impl.h"
+
+namespace bvpdev {
+#define FIRK_INST(S)                                                                                         \
+    template hipError_t firk_launch_solve_t<6, S, 1>(const BatchDev &, int, hipStream_t);                   \
+    template hipError_t firk_launch_solve_t<6, S, 2>(const BatchDev &, int, hipStream_t);                   \
+    template hipError_t firk_launch_component_t<6, S>(const BatchDev &, int, int, hipStream_t);             \
+    template hipError_t firk_launch_interp_t<6, S>(const BatchDev &, const int *, const double *, double *,  \
+                                                     double *, long long, hipStream_t);                       \
+    template hipError_t firk_launch_gather_t<6, S>(const BatchDev &, const long long *, double *, hipStream_t); \
+    template int firk_occupancy_t<6, S, 1>(int);                                                              \
+    template int firk_occupancy_t<6, S, 2>(int);
+FIRK_INST(5)
+FIRK_INST(7)
+#undef FIRK_INST
+}  // namespace bvpdev
