@@ -43,7 +43,6 @@ struct __align__(16) Tile {
     float x[T][NIN];        // normalised inputs
     float out[T][NOUT];     // network output (normalised units), then dL/dout
     float tgt[T][NOUT];
-    float lossv[T];
     int valid[T];
 };
 
@@ -496,7 +495,7 @@ __device__ inline int instance_of_node(const BatchDev &B, long long gidx) {
 
 // ------------------------------------------------------------------ inference
 // Persistent inference: each workgroup keeps its waves' column slices of both
-// hidden weight matrices in registers (2 x 4 x 8 operands of 8 BF16 per lane)
+// hidden weight matrices in registers (2 x CT x 8 operands of 8 BF16 per lane)
 // and streams 64-point tiles through two LDS activation buffers, so that the
 // weights are read from memory once per workgroup instead of once per tile.
 // what a source keeps of a point between reading its features and storing its
