@@ -30,7 +30,7 @@
 // (flat accesses) and the rows staged through LDS per interval, measured at
 // M = 32, MIRK6, FP32 factors + 2 refinement steps: 1 instance of 301 intervals 120 ms,
 // 64 instances of 272..720 intervals 300 ms; M = 16, MIRK4, FP64, 200 instances of
-// 200..600 intervals 65 ms.  This split: 7.3 ms, 17.1 ms, 5.1 ms.
+// 200..600 intervals 65 ms.  This split: 7.3 ms, 17.1 ms, 5.2 ms (5.1 ms with pivots compared in FP32).
 // Reference counterparts as in mirk_wave_impl.h (MIRK/collocation.jl:44-102,
 // MIRK/mirk.jl:697-862 and 927-1002, MIRK/adaptivity.jl:23-75, 250-304, 370-461).
 #pragma once
