@@ -12,8 +12,9 @@
 // cost tens of microseconds each, and a call needs a handful of blocks: a lone pendulum solve
 // takes 0.46 ms, 0.89 ms with some 35 allocations and 17 small uploads per call).  At most kMaxHeld
 // bytes are held, no block above kMaxBlock; the rest, and everything when the context is
-// destroyed, goes back to the device.  All work on pooled memory is enqueued on the
-// context's one stream, so a block handed on is rewritten only after its last reader.
+// destroyed, goes back to the device.  Work on pooled memory is enqueued on the context's one
+// stream, so a block handed on is rewritten only after its last reader; what other streams may
+// read is not pooled (networks) or waits for them first (bvp_batch::foreign).
 class DevPool {
   public:
     static constexpr size_t kMaxHeld = (size_t)1 << 30, kMaxBlock = (size_t)256 << 20;
